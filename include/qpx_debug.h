@@ -17,15 +17,17 @@ extern "C" {
 #endif
 
 /* Force the sigma path of later qpx_sigma / qpx_sigma_device / qpx_davidson
- * calls: 0 automatic, 1 dense-map kernels (full-CI-like spaces), 2 scanning
- * kernel, 3 sub-string bucket kernel.  *last_path (may be NULL) receives the
+ * calls: 0 automatic, 1 string-driven kernels (product spaces) or else the
+ * dense-map kernels (full-CI-like spaces), 2 scanning kernel, 3 sub-string
+ * bucket kernel, 4 dense-map kernels.  *last_path reads 1 for both kinds of 1.  *last_path (may be NULL) receives the
  * path the previous sigma call took.  A forced path that does not apply to
  * the wavefunction makes the sigma call fail. */
 int qpx_debug_force_sigma_path(qpx_ctx *ctx, int path, int *last_path);
 
 /* One qpx_sigma_device call per repetition on `stream`; ms (2) receives the
- * average duration of its two kernel phases (dense path: column kernel, row
- * kernel; sparse path: the bucket kernel, 0), measured with HIP events on
+ * average duration of its two kernel phases (string-driven path: same-spin
+ * kernels, alpha/beta kernel; dense path: column kernel, row kernel; sparse
+ * path: the bucket kernel, 0), measured with HIP events on
  * that stream. */
 int qpx_debug_sigma_kernel_times(qpx_ctx *ctx, int prec, int n_st, const void *u_t, void *v_t, void *s_t,
                                  void *stream, float *ms, int reps);

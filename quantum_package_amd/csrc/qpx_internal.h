@@ -118,6 +118,40 @@ struct SparseIdx {
   }
 };
 
+// Tables of the string-driven sigma of product spaces (sigma_fci.hip), built
+// on first use: partners of 16 strings at a time, their matrix elements and
+// the placement tables, per precision.
+struct SpinTiles {
+  int ntile = 0, nchunk = 0;
+  DBuf<int> ptr, idx;
+};
+template <typename T>
+struct FciTables {
+  bool valid = false;
+  DBuf<T> coef_a, coef_b, gb, vo;
+  DBuf<uint4> tgt;
+  void clear() {
+    valid = false;
+    coef_a.release(); coef_b.release(); gb.release(); vo.release(); tgt.release();
+  }
+};
+struct FciPlan {
+  bool valid = false;
+  int lda = 0, ldb = 0, ldt = 0;
+  DBuf<int> vrow;
+  DBuf<uint32_t> map_a, map_b;
+  SpinTiles a, b;
+  FciTables<double> t64;
+  FciTables<float> t32;
+  void clear() {
+    valid = false;
+    vrow.release(); map_a.release(); map_b.release();
+    for (SpinTiles *t : {&a, &b}) { t->ptr.release(); t->idx.release(); t->ntile = t->nchunk = 0; }
+    t64.clear();
+    t32.clear();
+  }
+};
+
 struct Wfn {
   int64_t n_det = 0;
   int nint = 0;
@@ -138,6 +172,7 @@ struct Wfn {
   std::vector<int> col_len_h, row_len_h;
   int max_col = 0, max_row = 0;
   SparseIdx sp;                           // built on first use of the sparse path
+  FciPlan fci;                            // built on first use of the product-space path
 };
 
 struct Workspace {
@@ -145,6 +180,35 @@ struct Workspace {
   char *get(size_t bytes) {
     if (buf.n < bytes) buf.alloc(bytes + (bytes >> 3));
     return buf.p;
+  }
+};
+
+// Scratch of calls that are enqueued on a caller's stream and return before
+// they have run: a call on another stream first waits for the last user.
+struct StreamWorkspace {
+  DBuf<char> buf;
+  hipStream_t last = nullptr;
+  hipEvent_t done = nullptr;
+  bool pending = false;
+  ~StreamWorkspace() {
+    if (done) (void)hipEventDestroy(done);
+  }
+  static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+  }
+  char *get(size_t bytes, hipStream_t s) {
+    if (pending && last != s && !capturing(s)) QPX_HIP(hipStreamWaitEvent(s, done, 0));
+    // hipFree waits for the device, so the old buffer is not in use any more
+    if (buf.n < bytes) buf.alloc(bytes);
+    return buf.p;
+  }
+  void used(hipStream_t s) {
+    if (capturing(s)) return;
+    if (!done) QPX_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
+    QPX_HIP(hipEventRecord(done, s));
+    last = s;
+    pending = true;
   }
 };
 
@@ -162,6 +226,7 @@ struct qpx_ctx {
   qpx::Workspace ws_sigma_io;   // host-order u/v/s staging for qpx_sigma
   qpx::Workspace ws_sigma_t;    // transposed u_t/v_t/s_t
   qpx::Workspace ws_misc;
+  qpx::StreamWorkspace ws_fci;  // planes of u and the same-spin part (sigma_fci.hip)
   int64_t sel_stats[4] = {0, 0, 0, 0};
   std::vector<int64_t> sel_ticks;   // per-block durations of the last selection (benchmark hook)
   int sigma_path = 0;           // last sigma path: 1 = dense-map, 2 = generic scan, 3 = sparse buckets
@@ -181,6 +246,9 @@ void build_wavefunction(qpx_ctx *c, int n_int, int64_t n_det, const uint64_t *ps
 void ensure_conn(qpx_ctx *c);
 // implemented in sigma.hip
 void sigma_device(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, void *s_t, hipStream_t s);
+// implemented in sigma_fci.hip
+bool fci_ok(qpx_ctx *c, int n_st, size_t tsize);
+bool sigma_fci(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, void *s_t, hipStream_t s);
 // implemented in sigma_sparse.hip
 bool sparse_ok(qpx_ctx *c, int n_st);
 void sigma_sparse(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, void *s_t, hipStream_t s);

@@ -5,9 +5,10 @@
 // beta-singles b' of b and inside each column b' the alpha-singles of a,
 // and (B) the alpha singles/doubles inside column b and the beta
 // singles/doubles inside row a, plus the diagonal; rows are owned by one
-// thread (no write conflicts).  The same ownership is kept here, with two
-// device strategies:
+// thread (no write conflicts).  The same ownership is kept here, with several
+// device strategies (a fourth, for selected wavefunctions, is sigma_sparse.hip):
 //
+//  * string-driven path (product spaces, i.e. full CI): sigma_fci.hip.
 //  * dense-map path (unique alpha/beta sets small enough that one column of
 //    u fits in LDS): one workgroup owns a beta column b.  For every
 //    beta-single b' of b it stages column b' of u into LDS as a dense
@@ -684,12 +685,14 @@ static bool dense_ok(qpx_ctx *c, int nst, size_t tsize) {
   const Ham &H = c->H;
   if (W.nint > 2 || nst > 4) return false;
   if (W.n_a > 65534 || H.M > 128) return false;
-  ensure_conn(c);   // at most 65534 alpha strings here: cheap
-  if (W.ca.max_singles > 96) return false;
   size_t need_c = ((size_t)(W.n_a + 1) * nst + (size_t)H.M * H.M + (size_t)1024 * nst) * tsize;
   size_t need_r = ((size_t)W.n_b * nst + (size_t)H.M * H.M) * tsize;
   size_t lim = (size_t)c->lds_per_block;
-  return need_c <= lim && need_r <= lim;
+  // the sizes first: the all-pairs connectivity of a selected wavefunction's
+  // strings costs tens of milliseconds, and is not needed where they fail
+  if (need_c > lim || need_r > lim) return false;
+  ensure_conn(c);
+  return W.ca.max_singles <= 96;
 }
 
 void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, hipStream_t st) {
@@ -697,9 +700,16 @@ void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s
   QPX_REQUIRE(nst >= 1 && nst <= GMAXST, "n_st must be in 1..8");
   QPX_REQUIRE(prec == QPX_FP64 || prec == QPX_FP32, "prec must be QPX_FP64 or QPX_FP32");
   size_t ts = prec == QPX_FP64 ? sizeof(double) : sizeof(float);
+  // a product space takes the string-driven path (12.2 against 32.8 ms for
+  // 9.0M determinants, FP64, 4 states; 35 against 86 us for 4900)
+  if ((c->force_path == 0 || c->force_path == 1) && fci_ok(c, nst, ts) &&
+      sigma_fci(c, prec, nst, u, v, s, st)) {
+    c->sigma_path = 1;
+    return;
+  }
   bool dense = dense_ok(c, nst, ts);
-  if (c->force_path >= 2) dense = false;
-  if (c->force_path == 1) QPX_REQUIRE(dense, "dense-map sigma path not applicable to this wavefunction");
+  if (c->force_path == 2 || c->force_path == 3) dense = false;
+  if (c->force_path == 1 || c->force_path == 4) QPX_REQUIRE(dense, "dense-map sigma path not applicable to this wavefunction");
   if (!dense && c->force_path != 2 && sparse_ok(c, nst)) {
     c->sigma_path = 3;
     sigma_sparse(c, prec, nst, u, v, s, st);
@@ -841,10 +851,11 @@ extern "C" int qpx_debug_lds_bandwidth(qpx_ctx *c, double *bytes_per_s) {
   });
 }
 
-// test hook: 0 = automatic, 1 = dense-map only, 2 = generic only
+// test hook: the sigma path of later calls (include/qpx_debug.h)
 extern "C" int qpx_debug_force_sigma_path(qpx_ctx *c, int path, int *last_path) {
   return qpx_guard(c, [&] {
-    QPX_REQUIRE(path >= 0 && path <= 3, "path must be 0 (automatic), 1 (dense map), 2 (generic scan) or 3 (sparse buckets)");
+    QPX_REQUIRE(path >= 0 && path <= 4, "path must be 0 (automatic), 1 (string-driven or dense map), 2 (generic scan), "
+                                        "3 (sparse buckets) or 4 (dense map)");
     c->force_path = path;
     if (last_path) *last_path = c->sigma_path;
   });

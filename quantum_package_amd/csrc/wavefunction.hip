@@ -349,6 +349,7 @@ void build_wavefunction(qpx_ctx *c, int nint, int64_t n_det, const uint64_t *psi
   Wfn &W = c->W;
   W.valid = false;
   W.sp.clear();
+  W.fci.clear();
   W.perm.clear();
   W.n_det = n_det;
   W.nint = nint;

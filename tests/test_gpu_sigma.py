@@ -225,3 +225,51 @@ def test_bad_inputs_raise(ctx):
     dup = np.concatenate([fci_space(8, 4, 4)[:5]] * 2)
     with pytest.raises(QpxError):
         ctx.set_wavefunction(dup)
+
+
+def _product_space(M, na, nb, drop, seed):
+    """Every kept alpha string with every kept beta string; drop: share of the
+    full CI's strings left out of each set."""
+    rng = np.random.default_rng(seed)
+    full = fci_space(M, na, nb)
+    a, b = np.unique(full[:, 0, 0]), np.unique(full[:, 1, 0])
+    a = a[np.sort(rng.permutation(a.size)[: max(1, round(a.size * (1 - drop)))])]
+    b = b[np.sort(rng.permutation(b.size)[: max(1, round(b.size * (1 - drop)))])]
+    d = np.empty((a.size * b.size, 2, 1), dtype=np.uint64)
+    d[:, 0, 0], d[:, 1, 0] = np.repeat(a, b.size), np.tile(b, a.size)
+    return d[rng.permutation(d.shape[0])]
+
+
+# product spaces (the string-driven kernels): one string of a spin, string
+# sets below, at and just past 16 and 64, pair tiles with and without room for
+# the diagonal pairs, 2..24 steps of beta singles, incomplete string sets
+PRODUCT = [
+    (2, 1, 1, 0.0), (4, 4, 2, 0.0), (4, 4, 1, 0.0), (5, 2, 1, 0.0), (6, 3, 2, 0.0), (6, 5, 1, 0.0), (7, 3, 3, 0.0),
+    (8, 5, 2, 0.0), (9, 5, 4, 0.0), (10, 2, 2, 0.0), (11, 3, 2, 0.0), (12, 4, 3, 0.0), (13, 3, 2, 0.0),
+    (16, 2, 2, 0.0), (20, 2, 1, 0.0), (26, 4, 1, 0.9), (8, 4, 4, 0.3), (10, 4, 3, 0.55), (12, 6, 5, 0.8),
+]
+
+
+@pytest.mark.parametrize("M,na,nb,drop", PRODUCT)
+@pytest.mark.parametrize("nst", [1, 2, 3, 4])
+def test_sigma_product_space(ctx, M, na, nb, drop, nst):
+    """FP64 to 1e-11 of the largest entry, as the other paths; FP32 (same u,
+    rounded) to 2e-5 of the norm, the bound of the FP32 paths above."""
+    H = synthetic_hamiltonian(M, na, nb, seed=M + na)
+    dets = _product_space(M, na, nb, drop, 7)
+    _say(f"[sigma product] M={M} {na}a{nb}b drop={drop} nst={nst} n_det={dets.shape[0]}")
+    ctx.set_hamiltonian(H)
+    ctx.set_wavefunction(dets)
+    u = np.random.default_rng(nst).standard_normal((dets.shape[0], nst))
+    vo, so = O.sigma(O.Ham(H), O.Bilinear(dets), u)
+    ctx._force_sigma_path(1)
+    v, s = ctx.H_S2_u_0_nstates(u)
+    assert ctx._force_sigma_path(1) == 1
+    assert np.max(np.abs(v - vo)) < 1e-11 * max(1.0, np.max(np.abs(vo)))
+    assert np.max(np.abs(s - so)) < 1e-11 * max(1.0, np.max(np.abs(so)))
+    w, t = ctx.H_S2_u_0_nstates(u)
+    assert np.array_equal(v, w) and np.array_equal(s, t)     # every sum has a fixed order
+    v, s = ctx.H_S2_u_0_nstates(u, prec=1)
+    ctx._force_sigma_path(0)
+    assert np.linalg.norm(v - vo) < 2e-5 * np.linalg.norm(vo)
+    assert np.linalg.norm(s - so) < 2e-5 * max(1.0, np.linalg.norm(so))
