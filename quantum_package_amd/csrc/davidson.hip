@@ -37,11 +37,32 @@ namespace {
 constexpr int RB = 256;        // threads per reduction block
 constexpr int RBLOCKS = 1024;  // reduction blocks
 
-__global__ void permute_in_kernel(const double *__restrict__ src, int64_t ld_src, const int64_t *__restrict__ perm,
-                                  int64_t n, int ncol, double *__restrict__ dst, int64_t ld_dst) {
+__device__ inline uint64_t splitmix64_mix(uint64_t z) {
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
+  return z ^ (z >> 31);
+}
+
+// Guess vectors in bilinear order: column j < n_guess is src(:, j), the later
+// ones are Gaussian noise (reference: random_number + Box-Muller, one normal
+// per pair of uniforms).  SplitMix64's t-th output is a function of
+// seed + t * increment, so every element draws its own pair: element i (psi
+// order) of column n_guess + k takes outputs 2 (k n + i) + 1 and + 2.  On the
+// host the 732k x 1 normals of a 12-orbital space took 20 ms.
+__global__ void guess_kernel(const double *__restrict__ src, int64_t ld_src, int n_guess, uint64_t seed,
+                             const int64_t *__restrict__ perm, int64_t n, int ncol, double *__restrict__ dst) {
   for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < n * ncol; x += (int64_t)gridDim.x * blockDim.x) {
-    int64_t j = x / n, k = x - j * n;
-    dst[k + ld_dst * j] = src[perm[k] + ld_src * j];
+    const int64_t j = x / n, k = x - j * n, i = perm[k];
+    double v;
+    if (j < n_guess) {
+      v = src[i + ld_src * j];
+    } else {
+      const uint64_t t = 2 * (uint64_t)((j - n_guess) * n + i);
+      const double r1 = 1.0 - (double)(splitmix64_mix(seed + (t + 1) * 0x9E3779B97F4A7C15ULL) >> 11) * (1.0 / 9007199254740992.0);
+      const double r2 = (double)(splitmix64_mix(seed + (t + 2) * 0x9E3779B97F4A7C15ULL) >> 11) * (1.0 / 9007199254740992.0);
+      v = sqrt(-2.0 * log(r1)) * cos(6.283185307179586 * r2);
+    }
+    dst[x] = v;
   }
 }
 
@@ -319,13 +340,6 @@ void jacobi_eigh(int n, const std::vector<double> &Ain, int lda, std::vector<dou
   }
 }
 
-uint64_t splitmix64(uint64_t &s) {
-  uint64_t z = (s += 0x9E3779B97F4A7C15ULL);
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
-  return z ^ (z >> 31);
-}
-
 struct Dav {
   qpx_ctx *c;
   hipStream_t st;
@@ -468,31 +482,25 @@ extern "C" int qpx_davidson(qpx_ctx *c, int N_st, int N_st_diag, double threshol
     hipStream_t st = c->stream;
     Dav D(c);
     const int64_t n = sze;
-    // random extra guess vectors (reference: random_number + Box-Muller)
-    uint64_t rs = seed;
-    for (int k = N_st; k < N_st_diag; ++k)
-      for (int64_t i = 0; i < sze; ++i) {
-        double r1 = 1.0 - (double)(splitmix64(rs) >> 11) * (1.0 / 9007199254740992.0);
-        double r2 = (double)(splitmix64(rs) >> 11) * (1.0 / 9007199254740992.0);
-        u_in[i + dim_in * k] = std::sqrt(-2.0 * std::log(r1)) * std::cos(6.283185307179586 * r2);
-      }
-    for (int k = 0; k < N_st_diag; ++k) {
-      double nr = 0.0;
-      for (int64_t i = 0; i < sze; ++i) nr += u_in[i + dim_in * k] * u_in[i + dim_in * k];
-      QPX_REQUIRE(nr > 0.0, "Davidson guess vector is zero");
-      nr = 1.0 / std::sqrt(nr);
-      for (int64_t i = 0; i < sze; ++i) u_in[i + dim_in * k] *= nr;
-    }
     DBuf<double> U, W, S, uin_d, host_io;
     U.alloc((size_t)n * nc);
     W.alloc((size_t)n * nc);
     S.alloc((size_t)n * nc);
     uin_d.alloc((size_t)n * N_st_diag);
-    host_io.alloc((size_t)dim_in * N_st_diag);
-    QPX_HIP(hipMemcpyAsync(host_io.p, u_in, sizeof(double) * dim_in * N_st_diag, hipMemcpyHostToDevice, st));
+    host_io.alloc((size_t)n * N_st_diag);
+    // the caller's N_st guess vectors and random ones behind them, normalised
+    QPX_HIP(hipMemcpy2DAsync(host_io.p, sizeof(double) * n, u_in, sizeof(double) * dim_in, sizeof(double) * n, N_st,
+                             hipMemcpyHostToDevice, st));
     int gridp = (int)std::min<int64_t>((n * N_st_diag + 255) / 256, 65536);
-    hipLaunchKernelGGL(permute_in_kernel, dim3(gridp), dim3(256), 0, st, host_io.p, dim_in, Wf.perm_d.p, n,
-                       N_st_diag, uin_d.p, n);
+    hipLaunchKernelGGL(guess_kernel, dim3(gridp), dim3(256), 0, st, host_io.p, n, N_st, seed, Wf.perm_d.p, n,
+                       N_st_diag, uin_d.p);
+    QPX_HIP(hipGetLastError());
+    for (int k = 0; k < N_st_diag; ++k) {
+      double *x = uin_d.p + n * k;
+      const double nr = D.dot(x, x);
+      QPX_REQUIRE(nr > 0.0, "Davidson guess vector is zero");
+      hipLaunchKernelGGL(scale_col_kernel, dim3(D.grid_rows), dim3(256), 0, st, x, 1.0 / std::sqrt(nr), n);
+    }
     QPX_HIP(hipGetLastError());
     // sigma staging (state-fastest)
     DBuf<char> tbuf;
@@ -662,9 +670,10 @@ extern "C" int qpx_davidson(qpx_ctx *c, int N_st, int N_st_diag, double threshol
       (void)switched;
     }
     hipLaunchKernelGGL(permute_out_kernel, dim3(gridp), dim3(256), 0, st, uin_d.p, n, Wf.perm_d.p, n, N_st_diag,
-                       host_io.p, dim_in);
+                       host_io.p, n);
     QPX_HIP(hipGetLastError());
-    QPX_HIP(hipMemcpyAsync(u_in, host_io.p, sizeof(double) * dim_in * N_st_diag, hipMemcpyDeviceToHost, st));
+    QPX_HIP(hipMemcpy2DAsync(u_in, sizeof(double) * dim_in, host_io.p, sizeof(double) * n, sizeof(double) * n, N_st_diag,
+                             hipMemcpyDeviceToHost, st));
     QPX_HIP(hipStreamSynchronize(st));
     for (int k = 0; k < N_st_diag; ++k) {
       energies[k] = lambda[k];
