@@ -12,6 +12,15 @@
 // class (aa, bb, ab), one-hot excitation degree of the generator from HF
 // (0..4), zero padding to D_IN = 80.
 //
+// A row's way through the network, forward and backward, needs no other row:
+// mlp_rows_kernel takes 16 RT rows from their descriptors to the prediction
+// (and, in training, on to the bias, head and embedding gradients) with the
+// activations in LDS and the weights streamed from L2 in operand order.  A
+// training step is that kernel, one launch for the sums over the batch (the
+// three weight gradients, cut along it, and the column sums) and one that sums
+// their slices and makes the Adam step.  It was 28 launches, with every activation and its
+// gradient written and read in FP32 and bf16: 235 us a step at batch 4096.
+//
 // GEMM: C(MxN) = A(MxK) B(KxN), A and B bf16 with arbitrary row/column
 // strides (so A^T, B^T need no copies), C fp32; workgroup tile 64x64, four
 // wavefronts each owning 32x32 = 2x2 tiles of v_mfma_f32_16x16x32_bf16
@@ -26,6 +35,7 @@
 #include <cstring>
 #include <cstdio>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 #include <hip/hip_bf16.h>
 #include "qpx_internal.h"
@@ -62,6 +72,7 @@ struct GemmArgs {
   int ksplit;         // K is cut into ksplit chunks (blockIdx.z); 1 = no split
   int a_run, b_run;   // staging: 1 = runs along k, 2 = along i (A) / j (B), 0 = element by element
   const float *mask;  // optional: C(i,j) = 0 where mask(i,j) <= 0 (same layout as C; a ReLU's backward)
+  int to_part;        // write slices to part whatever their number
 };
 
 // LDK pads a tile row to 80 bytes: rows stay 16-byte aligned for the staging
@@ -107,11 +118,12 @@ __device__ inline void stage_tile(uint16_t (*T)[LDK], const uint16_t *__restrict
   }
 }
 
-__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
+// the 64 x 64 tile (by, bx) of slice bz
+__device__ inline void gemm_tile(const GemmArgs &g, int bx, int by, int bz) {
   __shared__ __align__(16) uint16_t As[TM][LDK];   // As[i][k]
   __shared__ __align__(16) uint16_t Bs[TN][LDK];   // Bs[j][k]
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int i0 = blockIdx.y * TM, j0 = blockIdx.x * TN;
+  const int i0 = by * TM, j0 = bx * TN;
   const int wi = (wv >> 1) * 32, wj = (wv & 1) * 32;
   floatx4 acc[2][2];
 #pragma unroll
@@ -121,7 +133,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
   // this workgroup's slice of K (all of it without a split); slices are
   // whole multiples of TK
   const int kc = ((g.K + g.ksplit - 1) / g.ksplit + TK - 1) / TK * TK;
-  const int k_lo = (int)blockIdx.z * kc, k_hi = min(g.K, k_lo + kc);
+  const int k_lo = bz * kc, k_hi = min(g.K, k_lo + kc);
   // A and B operands of v_mfma_f32_16x16x32_bf16: lane (r, g = lane / 16)
   // supplies row r of the tile at k = 8 g .. 8 g + 7; the result rows are
   // 4 g .. 4 g + 3 of column r
@@ -154,8 +166,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         int gi = i0 + wi + 16 * a + q + t, gj = j0 + wj + 16 * b + r;
-        if (gi < g.M && gj < g.N && g.ksplit > 1) {
-          g.part[((int64_t)blockIdx.z * g.M + gi) * g.N + gj] = acc[a][b][t];
+        if (gi < g.M && gj < g.N && (g.ksplit > 1 || g.to_part)) {
+          g.part[((int64_t)bz * g.M + gi) * g.N + gj] = acc[a][b][t];
         } else if (gi < g.M && gj < g.N) {
           float v = acc[a][b][t];
           float *c = g.C + gi * g.c_rs + gj;
@@ -167,6 +179,10 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
           if (g.Cb) g.Cb[gi * g.c_rs + gj] = f2bf(v);
         }
       }
+}
+
+__global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
+  gemm_tile(g, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
 
 // split-K: C = sum of the partial products in slice order, then the epilogue
@@ -193,210 +209,456 @@ __global__ void to_bf16_kernel(const float *__restrict__ x, uint16_t *__restrict
     y[i] = f2bf(x[i]);
 }
 
-// features of the blocks: desc = (h1, h2 (0-based), spin class 0..2,
-// degree 0..4) int32 x4; fdesc = (eps1, eps2, log|c|) float x3
-__global__ void features_kernel(const int *__restrict__ desc, const float *__restrict__ fdesc,
-                                const float *__restrict__ emb, int n, int din, float *__restrict__ X,
-                                uint16_t *__restrict__ Xb) {
-  for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < (int64_t)n * din;
-       x += (int64_t)gridDim.x * blockDim.x) {
-    int i = (int)(x / din), f = (int)(x - (int64_t)i * din);
-    const int *d = desc + 4 * i;
-    float v = 0.f;
-    if (f < 32) v = emb[d[0] * 32 + f];
-    else if (f < 64) v = emb[d[1] * 32 + (f - 32)];
-    else if (f < 67) v = fdesc[3 * i + (f - 64)];
-    else if (f < 70) v = (d[2] == f - 67) ? 1.f : 0.f;
-    else if (f < 75) v = (d[3] == f - 70) ? 1.f : 0.f;
-    X[x] = v;
-    Xb[x] = f2bf(v);
-  }
+constexpr int kDin = 80, kHid = 256;
+
+// Weights in operand order: an MFMA step of 32 k and a block of 16 columns is
+// 64 lanes x 8 elements, so a lane's operand is one 16-byte read and a
+// wavefront's is 1 KiB in a row.  Position of element (k, n) of a K x 16 nb
+// right factor.
+__host__ __device__ inline int packed_at(int k, int n, int nb) {
+  return ((((k >> 5) * nb + (n >> 4)) * 64 + ((k >> 3) & 3) * 16 + (n & 15)) << 3) + (k & 7);
+}
+constexpr int kPack1 = 3 * 16 * 512, kPack = 8 * 16 * 512, kPack1t = 8 * 5 * 512;
+
+__device__ inline void store_packed(uint16_t *f, uint16_t *t, int rows, int i, float w) {
+  const int k = i / kHid, n = i - k * kHid;
+  const uint16_t b = f2bf(w);
+  f[packed_at(k, n, kHid / 16)] = b;
+  t[packed_at(n, k, rows / 16)] = b;   // the transpose, for the gradient of the layer's input
+}
+__global__ void pack_kernel(const float *__restrict__ W, int rows, uint16_t *__restrict__ f, uint16_t *__restrict__ t) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows * kHid; i += gridDim.x * blockDim.x)
+    store_packed(f, t, rows, i, W[i]);
 }
 
-// y = H3 w4 + b4 (one output), loss partials and dy = 2 (y - t) / n
-// y = H w4 + b4 per row, one wavefront per row (the row read coalesced,
-// reduced by shuffles in a fixed order); with targets, dy = 2 (y - t) / n and
-// one partial sum of (y - t)^2 per workgroup
-__global__ __launch_bounds__(256) void head_kernel(const float *__restrict__ H, const float *__restrict__ w4,
-                                                   const float *__restrict__ b4p,
-                                                   int n, int hdim, const float *__restrict__ t,
-                                                   float *__restrict__ y, float *__restrict__ dy,
-                                                   float *__restrict__ loss_part) {
-  __shared__ float red[4];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  float l = 0.f;
-  for (int i = blockIdx.x * 4 + wv; i < n; i += gridDim.x * 4) {
-    float s = 0.f;
-    for (int k = lane; k < hdim; k += 64) s += H[(int64_t)i * hdim + k] * w4[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    s += *b4p;
-    if (lane == 0) {
-      y[i] = s;
-      if (t) {
-        const float e = s - t[i];
-        l += e * e;
-        if (dy) dy[i] = 2.f * e / n;
-      }
-    }
-  }
-  if (lane == 0) red[wv] = l;
-  __syncthreads();
-  if (threadIdx.x == 0 && loss_part) loss_part[blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-static inline int head_blocks(int n) { return std::max(1, std::min(1024, (n + 3) / 4)); }
-
-// out[0] = (sum of the nb loss partials, in a fixed order) / n
-__global__ __launch_bounds__(256) void loss_reduce_kernel(const float *__restrict__ part, int nb, int n,
-                                                          float *__restrict__ out) {
-  __shared__ float red[256];
-  float s = 0.f;
-  for (int i = threadIdx.x; i < nb; i += 256) s += part[i];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) out[0] = red[0] / (float)n;
-}
-
-// dZ = (dy w4^T) masked by H > 0; bf16 copy; dw4 = H^T dy partial sums
-__global__ void head_back_kernel(const float *__restrict__ H, const float *__restrict__ w4,
-                                 const float *__restrict__ dy, int n, int hdim, float *__restrict__ dZ,
-                                 uint16_t *__restrict__ dZb) {
-  for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < (int64_t)n * hdim;
-       x += (int64_t)gridDim.x * blockDim.x) {
-    int i = (int)(x / hdim), k = (int)(x - (int64_t)i * hdim);
-    float v = H[x] > 0.f ? dy[i] * w4[k] : 0.f;
-    dZ[x] = v;
-    dZb[x] = f2bf(v);
-  }
-}
-
-// column sums of a (n x m) row-major fp32 matrix (bias gradients), and the
-// head weight gradient dw4[k] = sum_i H[i,k] dy[i]
-// out[k] = sum_i A[i][k] (w[i]): a workgroup of 256 threads per CB columns
-// (CB = 32, or m when m < 32); CB consecutive threads read one row's
-// columns (coalesced), 256 / CB row groups stride the rows, and the groups
-// are summed in order (deterministic).  Launch with ceil(m / CB) groups.
-__global__ __launch_bounds__(256) void colsum_kernel(const float *__restrict__ A, const float *__restrict__ w, int n,
-                                                     int m, float *__restrict__ out) {
-  __shared__ float red[256];
-  const int cb = m < 32 ? m : 32, groups = 256 / cb;
-  const int t = threadIdx.x, c = t % cb, g = t / cb;
-  const int k = blockIdx.x * cb + c;
-  float s = 0.f;
-  if (g < groups && k < m)
-    for (int i = g; i < n; i += groups) s += A[(int64_t)i * m + k] * (w ? w[i] : 1.f);
-  red[t] = s;
-  __syncthreads();
-  if (t < cb && k < m) {
-    float acc = 0.f;
-    for (int q = 0; q < groups; ++q) acc += red[q * cb + t];
-    out[k] = acc;
-  }
-}
-
-static inline int colsum_grid(int m) { return m < 32 ? 1 : (m + 31) / 32; }
-
-// Column sums of a wide matrix in two passes, each in a fixed order:
-// workgroup (column block b, row chunk p) sums 64 columns over the rows of
-// its chunk (4 row phases per column, combined in phase order) into
-// part[p][k]; the second pass adds the chunks in chunk order.  Spreading the
-// rows over many workgroups is what fills the GPU: one workgroup per 32
-// columns left all but 8 CUs idle for m = 256.
-__global__ __launch_bounds__(256) void colsum_part_kernel(const float *__restrict__ A, const float *__restrict__ w,
-                                                          int n, int m, int chunk, float *__restrict__ part) {
-  __shared__ float red[4][64];
-  const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
-  const int k = blockIdx.x * 64 + c, p = blockIdx.y;
-  const int r0 = p * chunk, r1 = min(n, r0 + chunk);
-  float s = 0.f;
-  if (k < m)
-    for (int i = r0 + g; i < r1; i += 4) s += A[(int64_t)i * m + k] * (w ? w[i] : 1.f);
-  red[g][c] = s;
-  __syncthreads();
-  if (g == 0 && k < m) part[(int64_t)p * m + k] = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
-}
-
-// one wavefront per column: lane l adds chunks l, l + 64, ...; the lanes
-// are then combined by a fixed shuffle tree
-__global__ __launch_bounds__(256) void colsum_final_kernel(const float *__restrict__ part, int np, int m,
-                                                           float *__restrict__ out) {
-  const int lane = threadIdx.x & 63;
-  const int k = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (k >= m) return;   // whole wavefront
-  float s = 0.f;
-  for (int p = lane; p < np; p += 64) s += part[(int64_t)p * m + k];
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-  if (lane == 0) out[k] = s;
-}
-
-__global__ void emb_grad_kernel(const int *__restrict__ desc, const float *__restrict__ dX, int n, int din,
-                                float *__restrict__ demb) {
-  for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < (int64_t)n * 64;
-       x += (int64_t)gridDim.x * blockDim.x) {
-    int i = (int)(x / 64), f = (int)(x - (int64_t)i * 64);
-    int h = f < 32 ? desc[4 * i] : desc[4 * i + 1];
-    atomicAdd(&demb[h * 32 + (f & 31)], dX[(int64_t)i * din + f]);
-  }
-}
-
-// Adam over all parameter tensors in one launch: tensor q covers elements
-// [start[q], start[q+1]) of the concatenation.  Per element:
-// m = b1 m + (1 - b1) g, v = b2 v + (1 - b2) g^2,
-// p -= lr (m / c1) / (sqrt(v / c2) + eps), with c1, c2 the bias corrections
-// 1 - b1^t, 1 - b2^t; the bf16 copy of p is refreshed where there is one.
-constexpr int kAdamTensors = 9;
-struct AdamSet {
-  float *p[kAdamTensors];
-  const float *g[kAdamTensors];
-  float *m[kAdamTensors];
-  float *v[kAdamTensors];
-  uint16_t *pb[kAdamTensors];
-  int64_t start[kAdamTensors + 1];
+struct RowArgs {
+  const int *perm;      // rows of the training set (null: rows 0, 1, ...)
+  const int *desc;      // (h1, h2 (0-based), spin class 0..2, degree 0..4) per row
+  const float *fdesc;   // (eps1, eps2, log|c|) per row
+  const float *tgt;
+  const float *emb;
+  const uint16_t *p1, *p2, *p3, *p3t, *p2t, *p1t;
+  const float *b1, *b2, *b3, *w4, *b4;
+  int n;
+  float *y;
+  // training: operands of the weight gradients, what the column sums need in
+  // FP32, the output's errors and gradient per row, the gradient of the
+  // embedding features
+  uint16_t *Xb, *H1b, *H2b, *dZ3b, *dZ2b, *dZ1b;
+  float *Z3, *dZ2, *dZ1, *err, *dy, *dX;
 };
 
-__global__ void adam_multi_kernel(AdamSet S, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int64_t total = S.start[kAdamTensors];
-  for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < total; x += (int64_t)gridDim.x * blockDim.x) {
-    int q = 0;
+constexpr int LDA = kHid + 8;   // LDS row stride: the 16 rows of an operand read fall on different banks
+
+// 16 RT rows per workgroup; wavefront w computes the column blocks w, w + 4,
+// w + 8, w + 12 of every layer, which is the order the output sum wants
+// (column c belongs to lane c % 64 of a row's 64-lane sum).
+// Bound: in training a workgroup reads 600 KB of weights from L2, 4 us at 64
+// bytes a cycle, against 1 us of products per 16 rows at half the matrix peak.
+template <int RT, bool TRAIN>
+__global__ __launch_bounds__(256, 2) void mlp_rows_kernel(RowArgs A) {
+  constexpr int R = 16 * RT;
+  __shared__ __align__(16) uint16_t act[R][LDA];
+  __shared__ float sred[R][65];
+  __shared__ float dys[R];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, j = lane & 15, q = lane >> 4;
+  const int r0 = (int)blockIdx.x * R;
+  // features, eight at a time: the embeddings of h1 and h2, then the numbers
+  // and the one-hot spin class and degree, then padding
+  for (int x = tid; x < R * 12; x += 256) {
+    const int r = x / 12, f = x - r * 12, row = r0 + r;
+    float v[8];
 #pragma unroll
-    for (int t = 1; t < kAdamTensors; ++t) q += (x >= S.start[t]);
-    const int64_t i = x - S.start[q];
-    const float gi = S.g[q][i];
-    const float mi = b1 * S.m[q][i] + (1.f - b1) * gi;
-    const float vi = b2 * S.v[q][i] + (1.f - b2) * gi * gi;
-    S.m[q][i] = mi;
-    S.v[q][i] = vi;
-    const float upd = lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-    const float pi = S.p[q][i] - upd;
-    S.p[q][i] = pi;
-    if (S.pb[q]) S.pb[q][i] = f2bf(pi);
+    for (int e = 0; e < 8; ++e) v[e] = 0.f;
+    if (row < A.n && f < 10) {
+      const int64_t i = A.perm ? A.perm[row] : row;
+      const int4 d = reinterpret_cast<const int4 *>(A.desc)[i];
+      if (f < 8) {
+        const int h = f < 4 ? d.x : d.y;
+        const float4 *e = reinterpret_cast<const float4 *>(A.emb + h * 32 + (f & 3) * 8);
+        const float4 e0 = e[0], e1 = e[1];
+        v[0] = e0.x; v[1] = e0.y; v[2] = e0.z; v[3] = e0.w;
+        v[4] = e1.x; v[5] = e1.y; v[6] = e1.z; v[7] = e1.w;
+      } else if (f == 8) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) v[e] = A.fdesc[3 * i + e];
+#pragma unroll
+        for (int e = 3; e < 6; ++e) v[e] = d.z == e - 3 ? 1.f : 0.f;
+        v[6] = d.w == 0 ? 1.f : 0.f;
+        v[7] = d.w == 1 ? 1.f : 0.f;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 3; ++e) v[e] = d.w == e + 2 ? 1.f : 0.f;
+      }
+    }
+    u32x4 p;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) p[e] = (uint32_t)f2bf(v[2 * e]) | ((uint32_t)f2bf(v[2 * e + 1]) << 16);
+    *reinterpret_cast<u32x4 *>(&act[r][8 * f]) = p;
+    if (TRAIN && row < A.n && f < 10) *reinterpret_cast<u32x4 *>(A.Xb + (int64_t)row * kDin + 8 * f) = p;
   }
+  __syncthreads();
+
+  floatx4 acc[RT][4];
+  // The operands of a whole layer are requested at once, as soon as the
+  // previous layer's products have read theirs: they arrive during its
+  // epilogue.  Column blocks w, w + 4, ... (nc of them) of `steps` steps.
+  bf16x8 bv[8][4];
+  auto fetch = [&](const uint16_t *P, auto steps, auto nb, auto nc) {
+    constexpr int S = decltype(steps)::value, NB = decltype(nb)::value, NC = decltype(nc)::value;
+    const bf16x8 *p = reinterpret_cast<const bf16x8 *>(P) + w * 64 + lane;
+#pragma unroll
+    for (int ks = 0; ks < S; ++ks)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) bv[ks][c] = p[(ks * NB + 4 * c) * 64];
+  };
+  // acc = act times the fetched operands
+  auto product = [&](auto steps, auto nc) {
+    constexpr int S = decltype(steps)::value, NC = decltype(nc)::value;
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) acc[a][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int ks = 0; ks < S; ++ks)
+#pragma unroll
+      for (int a = 0; a < RT; ++a) {
+        const bf16x8 av = *reinterpret_cast<const bf16x8 *>(&act[16 * a + j][32 * ks + 8 * q]);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc[a][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av, bv[ks][c], acc[a][c], 0, 0, 0);
+      }
+  };
+  using I3 = std::integral_constant<int, 3>;
+  using I5 = std::integral_constant<int, 5>;
+  using I8 = std::integral_constant<int, 8>;
+  using I16 = std::integral_constant<int, 16>;
+  using I4 = std::integral_constant<int, 4>;
+  using I1 = std::integral_constant<int, 1>;
+  // rows of LDS to memory, 16 bytes a thread
+  auto save = [&](uint16_t *to) {
+    for (int x = tid; x < R * (kHid / 8); x += 256) {
+      const int r = x / (kHid / 8), c = (x - r * (kHid / 8)) * 8;
+      if (r0 + r < A.n) *reinterpret_cast<u32x4 *>(to + (int64_t)(r0 + r) * kHid + c) = *reinterpret_cast<const u32x4 *>(&act[r][c]);
+    }
+  };
+  // act = relu(acc + bias); bit 16 a + 4 c + t of the returned mask: positive
+  auto relu = [&](const float *bias, bool keep) {
+    uint64_t m = 0;
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int col = 16 * (w + 4 * c) + j;
+        const float b = bias[col];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          float v = acc[a][c][t] + b;
+          v = v > 0.f ? v : 0.f;
+          if (v > 0.f) m |= 1ull << (16 * a + 4 * c + t);
+          if (keep) acc[a][c][t] = v;
+          else act[16 * a + 4 * q + t][col] = f2bf(v);
+        }
+      }
+    __syncthreads();
+    return m;
+  };
+  fetch(A.p1, I3{}, I16{}, I4{});
+  product(I3{}, I4{});
+  fetch(A.p2, I8{}, I16{}, I4{});
+  const uint64_t m1 = relu(A.b1, false);
+  if (TRAIN) save(A.H1b);
+  product(I8{}, I4{});
+  fetch(A.p3, I8{}, I16{}, I4{});
+  const uint64_t m2 = relu(A.b2, false);
+  if (TRAIN) save(A.H2b);
+  product(I8{}, I4{});
+  if (TRAIN) fetch(A.p3t, I8{}, I16{}, I4{});
+  relu(A.b3, true);
+  // output: 64 sums over columns l, l + 64, l + 128, l + 192 per row, then a fixed tree
+  float w4c[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) w4c[c] = A.w4[16 * (w + 4 * c) + j];
+#pragma unroll
+  for (int a = 0; a < RT; ++a)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float s = 0.f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s = fmaf(acc[a][c][t], w4c[c], s);
+      sred[16 * a + 4 * q + t][16 * w + j] = s;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < R / 4; ++i) {
+    const int r = w * (R / 4) + i, row = r0 + r;
+    float s = sred[r][lane];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    s += *A.b4;
+    if (lane == 0) {
+      float d = 0.f;
+      if (row < A.n) {
+        A.y[row] = s;
+        if (TRAIN) {
+          const float e = s - A.tgt[A.perm ? A.perm[row] : row];
+          d = 2.f * e / A.n;
+          A.err[row] = e;
+          A.dy[row] = d;
+        }
+      }
+      if (TRAIN) dys[r] = d;
+    }
+  }
+  if constexpr (TRAIN) {
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int col = 16 * (w + 4 * c) + j;
+#pragma unroll
+      for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const int r = 16 * a + 4 * q + t;
+          const float v = acc[a][c][t];
+          if (r0 + r < A.n) A.Z3[(int64_t)(r0 + r) * kHid + col] = v;
+          act[r][col] = f2bf(v > 0.f ? dys[r] * w4c[c] : 0.f);
+        }
+    }
+    __syncthreads();
+    save(A.dZ3b);
+    // act = acc where the layer's output was positive
+    auto masked = [&](uint64_t m, float *to) {
+      __syncthreads();
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const int col = 16 * (w + 4 * c) + j;
+#pragma unroll
+        for (int a = 0; a < RT; ++a)
+#pragma unroll
+          for (int t = 0; t < 4; ++t) {
+            const int r = 16 * a + 4 * q + t;
+            const float v = (m >> (16 * a + 4 * c + t)) & 1 ? acc[a][c][t] : 0.f;
+            if (r0 + r < A.n) to[(int64_t)(r0 + r) * kHid + col] = v;
+            act[r][col] = f2bf(v);
+          }
+      }
+      __syncthreads();
+    };
+    product(I8{}, I4{});
+    fetch(A.p2t, I8{}, I16{}, I4{});
+    masked(m2, A.dZ2);
+    save(A.dZ2b);
+    product(I8{}, I4{});
+    fetch(A.p1t, I8{}, I5{}, I1{});
+    masked(m1, A.dZ1);
+    save(A.dZ1b);
+    // gradient of the 64 embedding features; the others are data
+    product(I8{}, I1{});
+    const int f = 16 * w + j;
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int r = 16 * a + 4 * q + t;
+        if (r0 + r < A.n) A.dX[(int64_t)(r0 + r) * 64 + f] = acc[a][0][t];
+      }
+  }
+}
+
+// The sums over the batch, in one launch: the slices of the three weight
+// gradients, the column sums (gradients of w4, b3, b2, b1) by row chunks, the
+// embedding gradient and the output bias.  Every sum but the embeddings' has a fixed order: a small change of a gradient
+// that nearly cancels changes the sign of its first Adam step.
+struct GradArgs {
+  GemmArgs g[3];
+  int blocks[3];              // of each product: tiles x slices, slice-major
+  const float *Z3, *dZ2, *dZ1, *dy, *w4;
+  int n, chunk, np;           // rows per chunk, chunks
+  float *part;                // [4][np][256]
+  float *gb4;
+  const float *dX;            // [n][64]
+  const int *perm, *desc;
+  float *demb;
+  int n_orb, ne;              // ne: chunks of kEmbRows rows
+};
+constexpr int kEmbRows = 256, kMaxOrb = 256;
+__global__ __launch_bounds__(256) void grad_kernel(GradArgs S) {
+  __shared__ float red[256];
+  __shared__ double es[kMaxOrb * 8];
+  int t = (int)blockIdx.x;
+#pragma unroll
+  for (int w = 0; w < 3; ++w) {
+    if (t < S.blocks[w]) {
+      const GemmArgs &g = S.g[w];
+      const int nbx = (g.N + TN - 1) / TN, nby = (g.M + TM - 1) / TM, z = t / (nbx * nby);
+      t -= z * nbx * nby;
+      gemm_tile(g, t % nbx, t / nbx, z);
+      return;
+    }
+    t -= S.blocks[w];
+  }
+  const int tid = threadIdx.x;
+  if (t < 16 * S.np) {
+    // sum `which` of 64 columns over a chunk: four row phases per column, combined in phase order
+    const int which = t / (4 * S.np), u = t - which * 4 * S.np, p = u >> 2, k = (u & 3) * 64 + (tid & 63), g = tid >> 6;
+    const int r0 = p * S.chunk, r1 = min(S.n, r0 + S.chunk);
+    const float w4 = S.w4[k];
+    float s = 0.f;
+    if (which == 0) {
+#pragma unroll 4
+      for (int i = r0 + g; i < r1; i += 4) s = fmaf(S.Z3[(int64_t)i * kHid + k], S.dy[i], s);
+    } else if (which == 1) {
+#pragma unroll 4
+      for (int i = r0 + g; i < r1; i += 4) {
+#pragma clang fp contract(off)
+        const float d = S.dy[i] * w4;
+        s += S.Z3[(int64_t)i * kHid + k] > 0.f ? d : 0.f;
+      }
+    } else {
+      const float *A = which == 2 ? S.dZ2 : S.dZ1;
+#pragma unroll 4
+      for (int i = r0 + g; i < r1; i += 4) s += A[(int64_t)i * kHid + k];
+    }
+    red[tid] = s;
+    __syncthreads();
+    if (g == 0) S.part[((int64_t)which * S.np + p) * kHid + k] = (red[tid] + red[64 + tid]) + (red[128 + tid] + red[192 + tid]);
+    return;
+  }
+  t -= 16 * S.np;
+  if (t < 4 * S.ne) {
+    // embedding gradient of 8 of the 32 components over a chunk of rows: both
+    // holes' features of a row go to its orbitals' sums, in FP64 (ds_add_f64 is
+    // 17 times as fast as ds_add_f32), and one atomic per component and orbital
+    // leaves the workgroup (one per row and feature took 21 us at 4096 rows)
+    const int g = t & 3, r0 = (t >> 2) * kEmbRows, r1 = min(S.n, r0 + kEmbRows);
+    for (int x = tid; x < S.n_orb * 8; x += 256) es[x] = 0.0;
+    __syncthreads();
+    for (int x = tid; x < (r1 - r0) * 16; x += 256) {
+      const int row = r0 + (x >> 4), which = (x >> 3) & 1, f = x & 7;
+      const int64_t i = S.perm ? S.perm[row] : row;
+      const int h = S.desc[4 * i + which];
+      unsafeAtomicAdd(&es[h * 8 + f], (double)S.dX[(int64_t)row * 64 + which * 32 + g * 8 + f]);
+    }
+    __syncthreads();
+    for (int x = tid; x < S.n_orb * 8; x += 256) {
+      const float v = (float)es[x];
+      if (v != 0.f) atomicAdd(&S.demb[(x >> 3) * 32 + g * 8 + (x & 7)], v);
+    }
+    return;
+  }
+  float s = 0.f;
+  for (int i = tid; i < S.n; i += 256) s += S.dy[i];
+  red[tid] = s;
+  __syncthreads();
+  if (tid == 0) {
+    float b = 0.f;
+    for (int i = 0; i < 256; ++i) b += red[i];
+    *S.gb4 = b;
+  }
+}
+
+// The step after a batch: sums the weight gradients' slices and the column
+// sums' chunks, takes the embedding gradient, and (lr > 0) makes the Adam step
+// m = b1 m + (1 - b1) g, v = b2 v + (1 - b2) g^2,
+// p -= lr (m / c1) / (sqrt(v / c2) + eps), c1, c2 the bias corrections
+// 1 - b1^t, 1 - b2^t; the packed bf16 weights are refreshed.
+// Blocks [0, nelem) take 256 elements of W1, W2, W3, emb, the next a column
+// (w4, b3, b2, b1, b4) per wavefront: lane l adds chunks l, l + 64, ..., then
+// a fixed tree; the last one the loss.
+struct Param {
+  float *p, *g, *m, *v;
+};
+struct AdamArgs {
+  Param W[3], emb, col[4], b4;   // col: w4, b3, b2, b1
+  const float *wpart[3];
+  int ks[3], wrows[3];
+  uint16_t *pf[3], *pt[3];
+  float *demb;          // accumulated by atomics; taken and cleared here
+  int n_emb, nelem;
+  const float *part, *err;
+  int np, n;
+  float *loss_out;
+  float lr, b1, b2, eps, c1, c2;
+};
+
+__device__ inline float adam(const AdamArgs &A, const Param &P, int i, float g) {
+  P.g[i] = g;
+  float p = P.p[i];
+  if (A.lr > 0.f) {
+    const float mi = fmaf(1.f - A.b1, g, A.b1 * P.m[i]);
+    const float vi = fmaf(g, (1.f - A.b2) * g, A.b2 * P.v[i]);
+    P.m[i] = mi;
+    P.v[i] = vi;
+    p -= A.lr * (mi / A.c1) / (sqrtf(vi / A.c2) + A.eps);
+    P.p[i] = p;
+  }
+  return p;
+}
+
+__global__ __launch_bounds__(256) void adam_kernel(AdamArgs A) {
+  if ((int)blockIdx.x < A.nelem) {
+    int i = (int)blockIdx.x * 256 + (int)threadIdx.x;
+#pragma unroll
+    for (int w = 0; w < 3; ++w) {
+      const int cnt = A.wrows[w] * kHid;
+      if (i < cnt) {
+        float g = 0.f;
+#pragma unroll 8
+        for (int z = 0; z < A.ks[w]; ++z) g += A.wpart[w][(int64_t)z * cnt + i];
+        const float p = adam(A, A.W[w], i, g);
+        if (A.lr > 0.f) store_packed(A.pf[w], A.pt[w], A.wrows[w], i, p);
+        return;
+      }
+      i -= cnt;
+    }
+    if (i < A.n_emb) {
+      const float g = A.demb[i];
+      A.demb[i] = 0.f;
+      adam(A, A.emb, i, g);
+    }
+    return;
+  }
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int k = ((int)blockIdx.x - A.nelem) * 4 + wv;
+  if ((int)blockIdx.x == (int)gridDim.x - 1) {
+    __shared__ float red[4];
+    float s = 0.f;
+    for (int i = threadIdx.x; i < A.n; i += 256) s = fmaf(A.err[i], A.err[i], s);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if (lane == 0) red[wv] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) *A.loss_out = ((red[0] + red[1]) + (red[2] + red[3])) / (float)A.n;
+    return;
+  }
+  if (k > 4 * kHid) return;
+  float s = 0.f;
+  if (k < 4 * kHid) {
+    const float *src = A.part + (int64_t)(k / kHid) * A.np * kHid + k % kHid;
+    for (int z = lane; z < A.np; z += 64) s += src[(int64_t)z * kHid];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  } else {
+    s = A.b4.g[0];
+  }
+  if (lane == 0) adam(A, k < 4 * kHid ? A.col[k / kHid] : A.b4, k < 4 * kHid ? k % kHid : 0, s);
 }
 
 }  // namespace
 
 // ---------------------------------------------------------------------------
 // Scratch of the allocation-free prediction (qpx_mlp_predict_static): the
-// staged descriptors, the features and the three layers' activations of at
-// most kStaticRows blocks, in one file-scope device array.  Each GPU the
-// library runs on holds its own copy until the process ends; its device
-// address is looked up once per device (scratch_address) and only that
-// address is handed to kernels and copies.
+// staged descriptors and the predictions of at most kStaticRows blocks, in
+// one file-scope device array.  Each GPU the library runs on holds its own
+// copy until the process ends; its device address is looked up once per
+// device (scratch_address) and only that address is handed to kernels and
+// copies.
 namespace {
 constexpr int kStaticRows = 2048;
-constexpr int kDin = 80, kHid = 256;
 constexpr size_t al256(size_t x) { return (x + 255) & ~size_t(255); }
-constexpr size_t kScratchBytes =
-    al256(sizeof(int) * 4 * kStaticRows) + al256(sizeof(float) * 3 * kStaticRows) +
-    al256(sizeof(float) * kDin * kStaticRows) + al256(sizeof(uint16_t) * kDin * kStaticRows) +
-    3 * al256(sizeof(float) * kHid * kStaticRows) + 3 * al256(sizeof(uint16_t) * kHid * kStaticRows) +
-    al256(sizeof(float) * kStaticRows);
+constexpr size_t kScratchBytes = al256(sizeof(int) * 4 * kStaticRows) + al256(sizeof(float) * 3 * kStaticRows) +
+                                 al256(sizeof(float) * kStaticRows);
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -423,18 +685,19 @@ struct qpx_mlp {
   int din = 80, hid = 256, n_orb = 0;
   hipStream_t st = nullptr;
   int device = 0;
-  // parameters (fp32 master) and bf16 copies; layer l: W (in x out) row-major
+  // parameters (fp32 master; layer l: W (in x out) row-major) and the weights
+  // packed as right factors, straight and transposed
   DBuf<float> W1, W2, W3, b1, b2, b3, w4, emb;
-  DBuf<uint16_t> W1b, W2b, W3b;
+  DBuf<uint16_t> p1, p2, p3, p1t, p2t, p3t;
   DBuf<float> gW1, gW2, gW3, gb1, gb2, gb3, gw4, gemb, gb4;
-  DBuf<float> ws;   // split-K partial products of the weight gradients (sized once)
+  DBuf<float> demb;                     // embedding gradient being accumulated; zero between steps
+  DBuf<float> ws1, ws2, ws3;            // slices of the weight gradients
   DBuf<float> mW1, mW2, mW3, mb1, mb2, mb3, mw4, memb, vW1, vW2, vW3, vb1, vb2, vb3, vw4, vemb;
   DBuf<float> b4, mb4, vb4;   // the output bias and its Adam moments (one element each, on the device)
   int step = 0;
-  // activations for a batch
-  int cap = 0;
-  DBuf<float> X, Z1, Z2, Z3, y, dy, dZ3, dZ2, dZ1, dX, lossp;
-  DBuf<uint16_t> Xb, H1b, H2b, H3b, dZ3b, dZ2b, dZ1b;
+  int cap = 0, tcap = 0;      // rows held: descriptors and predictions; training operands
+  DBuf<float> y, part, Z3, dZ2, dZ1, dX, rerr, dy, lossp;
+  DBuf<uint16_t> Xb, H1b, H2b, dZ3b, dZ2b, dZ1b;
   DBuf<int> desc;
   DBuf<float> fdesc, tgt;
   void *scratch = nullptr;   // device address of this device's prediction scratch
@@ -458,7 +721,7 @@ void gemm(hipStream_t st, const uint16_t *A, int64_t ars, int64_t acs, const uin
     return 0;
   };
   GemmArgs g{A, ars, acs, B, brs, bcs, C, crs, M, N, K, bias, relu, Cb, beta, nullptr, 1,
-             run_of(A, ars, acs), run_of(B, bcs, brs), mask};
+             run_of(A, ars, acs), run_of(B, bcs, brs), mask, 0};
   dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
   const int tiles = (int)(grid.x * grid.y);
   constexpr int kGrain = 16;   // split-K sizing unit (slices are then rounded up to TK)
@@ -481,175 +744,134 @@ void gemm(hipStream_t st, const uint16_t *A, int64_t ars, int64_t acs, const uin
   }
 }
 
-// out[k] = sum_i A[i][k] w[i] (w null: 1) over the n x mc row-major A; the
-// wide case uses the workspace for its per-chunk partial sums
-void colsum(hipStream_t st, const float *A, const float *w, int n, int mc, float *out, DBuf<float> &ws) {
-  if (mc < 32) {
-    hipLaunchKernelGGL(colsum_kernel, dim3(colsum_grid(mc)), dim3(256), 0, st, A, w, n, mc, out);
-    QPX_HIP(hipGetLastError());
-    return;
-  }
-  const int nb = (mc + 63) / 64;
-  int np = std::max(1, std::min(256 / nb, (n + 63) / 64));
-  np = (int)std::max<int64_t>(1, std::min<int64_t>(np, (int64_t)(ws.n / (size_t)mc)));
-  const int chunk = std::max(1, (n + np - 1) / np);
-  np = std::max(1, (n + chunk - 1) / chunk);
-  hipLaunchKernelGGL(colsum_part_kernel, dim3(nb, np), dim3(256), 0, st, A, w, n, mc, chunk, ws.p);
-  hipLaunchKernelGGL(colsum_final_kernel, dim3((mc + 3) / 4), dim3(256), 0, st, (const float *)ws.p, np, mc, out);
-  QPX_HIP(hipGetLastError());
-}
+constexpr int kSlices = 32;      // most slices of a weight gradient
+constexpr int kChunks = 64;      // most row chunks of a column sum
 
 void ensure(qpx_mlp *m, int n) {
   if (n <= m->cap) return;
-  int c = n;
-  m->X.alloc((size_t)c * m->din); m->Xb.alloc((size_t)c * m->din); m->dX.alloc((size_t)c * m->din);
-  m->Z1.alloc((size_t)c * m->hid); m->Z2.alloc((size_t)c * m->hid); m->Z3.alloc((size_t)c * m->hid);
-  m->H1b.alloc((size_t)c * m->hid); m->H2b.alloc((size_t)c * m->hid); m->H3b.alloc((size_t)c * m->hid);
-  m->dZ1.alloc((size_t)c * m->hid); m->dZ2.alloc((size_t)c * m->hid); m->dZ3.alloc((size_t)c * m->hid);
-  m->dZ1b.alloc((size_t)c * m->hid); m->dZ2b.alloc((size_t)c * m->hid); m->dZ3b.alloc((size_t)c * m->hid);
-  m->y.alloc(c); m->dy.alloc(c); m->lossp.alloc(1025);   // head partials + one loss slot
-  m->desc.alloc((size_t)4 * c); m->fdesc.alloc((size_t)3 * c); m->tgt.alloc(c);
-  if (!m->ws.p) m->ws.alloc((size_t)32 * m->hid * m->hid);   // the largest split: 32 x hid x hid
-  m->cap = c;
+  m->desc.alloc((size_t)4 * n);
+  m->fdesc.alloc((size_t)3 * n);
+  m->tgt.alloc(n);
+  m->y.alloc(n);
+  m->cap = n;
 }
 
-int grid1(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 16384); }
-
-// the buffers of one forward pass over n rows
-struct FwdBufs {
-  const int *desc;
-  const float *fdesc;
-  float *X, *Z1, *Z2, *Z3, *y;
-  uint16_t *Xb, *H1b, *H2b, *H3b;
-};
-
-void forward_bufs(qpx_mlp *m, int n, const FwdBufs &b) {
-  hipStream_t st = m->st;
-  const int D = m->din, Hd = m->hid;
-  hipLaunchKernelGGL(features_kernel, dim3(grid1((int64_t)n * D)), dim3(256), 0, st, b.desc, b.fdesc, m->emb.p, n, D,
-                     b.X, b.Xb);
-  // Z = act(X W + b): A = X (n x D, row-major), B = W (D x H, row-major)
-  gemm(st, b.Xb, D, 1, m->W1b.p, Hd, 1, b.Z1, Hd, n, Hd, D, m->b1.p, 1, b.H1b, 0.f);
-  gemm(st, b.H1b, Hd, 1, m->W2b.p, Hd, 1, b.Z2, Hd, n, Hd, Hd, m->b2.p, 1, b.H2b, 0.f);
-  gemm(st, b.H2b, Hd, 1, m->W3b.p, Hd, 1, b.Z3, Hd, n, Hd, Hd, m->b3.p, 1, b.H3b, 0.f);
+void ensure_train(qpx_mlp *m, int n) {
+  ensure(m, n);
+  if (n <= m->tcap) return;
+  const int Hd = m->hid;
+  m->Xb.alloc((size_t)n * m->din);
+  for (DBuf<uint16_t> *b : {&m->H1b, &m->H2b, &m->dZ1b, &m->dZ2b, &m->dZ3b}) b->alloc((size_t)n * Hd);
+  for (DBuf<float> *b : {&m->Z3, &m->dZ2, &m->dZ1}) b->alloc((size_t)n * Hd);
+  m->dX.alloc((size_t)n * 64);
+  m->rerr.alloc(n);
+  m->dy.alloc(n);
+  m->part.alloc((size_t)4 * kChunks * Hd);
+  m->lossp.alloc(1);
+  m->ws1.alloc((size_t)kSlices * m->din * Hd);
+  m->ws2.alloc((size_t)kSlices * Hd * Hd);
+  m->ws3.alloc((size_t)kSlices * Hd * Hd);
+  m->tcap = n;
 }
 
-void forward(qpx_mlp *m, int n) {
-  forward_bufs(m, n, FwdBufs{m->desc.p, m->fdesc.p, m->X.p, m->Z1.p, m->Z2.p, m->Z3.p, m->y.p, m->Xb.p, m->H1b.p,
-                             m->H2b.p, m->H3b.p});
+// the rows of the given arrays (rows perm[0..n) of them with perm)
+RowArgs row_args(qpx_mlp *m, int n, const int *perm, const int *desc, const float *fdesc, const float *tgt, float *y) {
+  RowArgs A{};
+  A.perm = perm; A.desc = desc; A.fdesc = fdesc; A.tgt = tgt; A.emb = m->emb.p;
+  A.p1 = m->p1.p; A.p2 = m->p2.p; A.p3 = m->p3.p; A.p1t = m->p1t.p; A.p2t = m->p2t.p; A.p3t = m->p3t.p;
+  A.b1 = m->b1.p; A.b2 = m->b2.p; A.b3 = m->b3.p; A.w4 = m->w4.p; A.b4 = m->b4.p;
+  A.n = n; A.y = y;
+  A.Xb = m->Xb.p; A.H1b = m->H1b.p; A.H2b = m->H2b.p; A.dZ3b = m->dZ3b.p; A.dZ2b = m->dZ2b.p; A.dZ1b = m->dZ1b.p;
+  A.Z3 = m->Z3.p; A.dZ2 = m->dZ2.p; A.dZ1 = m->dZ1.p; A.err = m->rerr.p; A.dy = m->dy.p; A.dX = m->dX.p;
+  return A;
 }
 
-// the forward buffers carved out of the prediction scratch at its device
-// address base (the layout kScratchBytes is sized for)
-FwdBufs static_bufs(void *base) {
-  unsigned char *p = static_cast<unsigned char *>(base);
-  auto take = [&](size_t bytes) {
-    unsigned char *q = p;
-    p += al256(bytes);
-    return q;
-  };
-  FwdBufs b{};
-  b.desc = reinterpret_cast<const int *>(take(sizeof(int) * 4 * kStaticRows));
-  b.fdesc = reinterpret_cast<const float *>(take(sizeof(float) * 3 * kStaticRows));
-  b.X = reinterpret_cast<float *>(take(sizeof(float) * kDin * kStaticRows));
-  b.Xb = reinterpret_cast<uint16_t *>(take(sizeof(uint16_t) * kDin * kStaticRows));
-  b.Z1 = reinterpret_cast<float *>(take(sizeof(float) * kHid * kStaticRows));
-  b.Z2 = reinterpret_cast<float *>(take(sizeof(float) * kHid * kStaticRows));
-  b.Z3 = reinterpret_cast<float *>(take(sizeof(float) * kHid * kStaticRows));
-  b.H1b = reinterpret_cast<uint16_t *>(take(sizeof(uint16_t) * kHid * kStaticRows));
-  b.H2b = reinterpret_cast<uint16_t *>(take(sizeof(uint16_t) * kHid * kStaticRows));
-  b.H3b = reinterpret_cast<uint16_t *>(take(sizeof(uint16_t) * kHid * kStaticRows));
-  b.y = reinterpret_cast<float *>(take(sizeof(float) * kStaticRows));
-  return b;
-}
-
-// One Adam step on the batch in place, enqueued on the network's stream
-// without waiting for it; the batch's mean squared error goes to *loss_out
-// (device memory).
-void train_step_async(qpx_mlp *m, int n, float lr, float *loss_out) {
-  hipStream_t st = m->st;
-  const int D = m->din, Hd = m->hid;
-  forward(m, n);
-  const int nb = head_blocks(n);
-  hipLaunchKernelGGL(head_kernel, dim3(nb), dim3(256), 0, st, m->Z3.p, m->w4.p, m->b4.p, n, Hd, m->tgt.p, m->y.p,
-                     m->dy.p, m->lossp.p);
-  // head grads
-  colsum(st, m->Z3.p, m->dy.p, n, Hd, m->gw4.p, m->ws);
-  colsum(st, m->dy.p, nullptr, n, 1, m->gb4.p, m->ws);
-  hipLaunchKernelGGL(head_back_kernel, dim3(grid1((int64_t)n * Hd)), dim3(256), 0, st, m->Z3.p, m->w4.p, m->dy.p,
-                     n, Hd, m->dZ3.p, m->dZ3b.p);
-  // layer 3: dW3 = H2^T dZ3 (H x H, K = n); db3 = colsum dZ3; dH2 = dZ3 W3^T
-  gemm(st, m->H2b.p, 1, Hd, m->dZ3b.p, Hd, 1, m->gW3.p, Hd, Hd, Hd, n, nullptr, 0, nullptr, 0.f, &m->ws);
-  colsum(st, m->dZ3.p, nullptr, n, Hd, m->gb3.p, m->ws);
-  // dZ2 = (dZ3 W3^T) masked by Z2 > 0, with its bf16 copy, in the epilogue
-  gemm(st, m->dZ3b.p, Hd, 1, m->W3b.p, 1, Hd, m->dZ2.p, Hd, n, Hd, Hd, nullptr, 0, m->dZ2b.p, 0.f, nullptr, m->Z2.p);
-  // layer 2
-  gemm(st, m->H1b.p, 1, Hd, m->dZ2b.p, Hd, 1, m->gW2.p, Hd, Hd, Hd, n, nullptr, 0, nullptr, 0.f, &m->ws);
-  colsum(st, m->dZ2.p, nullptr, n, Hd, m->gb2.p, m->ws);
-  gemm(st, m->dZ2b.p, Hd, 1, m->W2b.p, 1, Hd, m->dZ1.p, Hd, n, Hd, Hd, nullptr, 0, m->dZ1b.p, 0.f, nullptr, m->Z1.p);
-  // layer 1: dW1 = X^T dZ1 (D x H); dX = dZ1 W1^T (n x D)
-  gemm(st, m->Xb.p, 1, D, m->dZ1b.p, Hd, 1, m->gW1.p, Hd, D, Hd, n, nullptr, 0, nullptr, 0.f, &m->ws);
-  colsum(st, m->dZ1.p, nullptr, n, Hd, m->gb1.p, m->ws);
-  gemm(st, m->dZ1b.p, Hd, 1, m->W1b.p, 1, Hd, m->dX.p, D, n, D, Hd, nullptr, 0, nullptr, 0.f);
-  QPX_HIP(hipMemsetAsync(m->gemb.p, 0, sizeof(float) * m->emb.n, st));
-  hipLaunchKernelGGL(emb_grad_kernel, dim3(grid1((int64_t)n * 64)), dim3(256), 0, st, m->desc.p, m->dX.p, n, D,
-                     m->gemb.p);
+// predictions of n rows: 64 rows per workgroup where that still fills the
+// chip twice over (half the weight traffic of 32 or 16), fewer below
+void predict_rows(qpx_mlp *m, int n, const int *desc, const float *fdesc, float *y) {
+  const RowArgs A = row_args(m, n, nullptr, desc, fdesc, nullptr, y);
+  if (n >= 64 * 512) hipLaunchKernelGGL((mlp_rows_kernel<4, false>), dim3((n + 63) / 64), dim3(256), 0, m->st, A);
+  else if (n >= 32 * 256) hipLaunchKernelGGL((mlp_rows_kernel<2, false>), dim3((n + 31) / 32), dim3(256), 0, m->st, A);
+  else hipLaunchKernelGGL((mlp_rows_kernel<1, false>), dim3((n + 15) / 16), dim3(256), 0, m->st, A);
   QPX_HIP(hipGetLastError());
+}
+
+// One Adam step on n rows, enqueued on the network's stream without waiting
+// for it; the batch's mean squared error goes to *loss_out (device memory).
+void train_step_async(qpx_mlp *m, int n, const int *perm, const int *desc, const float *fdesc, const float *tgt,
+                      float lr, float *loss_out) {
+  hipStream_t st = m->st;
+  const int D = m->din, Hd = m->hid;
+  // 16 rows per workgroup until every CU has one, 32 above
+  const RowArgs R = row_args(m, n, perm, desc, fdesc, tgt, m->y.p);
+  if (n <= 16 * 256) hipLaunchKernelGGL((mlp_rows_kernel<1, true>), dim3((n + 15) / 16), dim3(256), 0, st, R);
+  else hipLaunchKernelGGL((mlp_rows_kernel<2, true>), dim3((n + 31) / 32), dim3(256), 0, st, R);
+  // weight gradients dW1 = X^T dZ1, dW2 = H1^T dZ2, dW3 = H2^T dZ3 over the
+  // batch, in slices of at least 64 rows, up to 256 workgroups a product;
+  // column sums in chunks of at least 64 rows, up to kChunks of them
+  GradArgs S{};
+  const uint16_t *a[3] = {m->Xb.p, m->H1b.p, m->H2b.p}, *b[3] = {m->dZ1b.p, m->dZ2b.p, m->dZ3b.p};
+  float *ws[3] = {m->ws1.p, m->ws2.p, m->ws3.p};
+  const int rows[3] = {D, Hd, Hd};
+  int ks[3], blocks = 0;
+  for (int w = 0; w < 3; ++w) {
+    const int tiles = ((rows[w] + TM - 1) / TM) * (Hd / TN);
+    ks[w] = n >= 128 ? std::max(1, std::min({256 / tiles, n / 64, kSlices})) : 1;
+    // one slice, too, goes through the slices' buffer
+    S.g[w] = GemmArgs{a[w], 1, rows[w], b[w], Hd, 1, nullptr, Hd, rows[w], Hd, n, nullptr, 0, nullptr, 0.f, ws[w],
+                      ks[w], 2, 2, nullptr, 1};
+    S.blocks[w] = tiles * ks[w];
+    blocks += S.blocks[w];
+  }
+  S.Z3 = m->Z3.p; S.dZ2 = m->dZ2.p; S.dZ1 = m->dZ1.p; S.dy = m->dy.p; S.w4 = m->w4.p;
+  S.n = n;
+  S.np = std::max(1, std::min(kChunks, (n + 63) / 64));
+  S.chunk = (n + S.np - 1) / S.np;
+  S.np = (n + S.chunk - 1) / S.chunk;
+  S.part = m->part.p;
+  S.gb4 = m->gb4.p;
+  S.dX = m->dX.p; S.perm = perm; S.desc = desc; S.demb = m->demb.p;
+  S.n_orb = m->n_orb;
+  S.ne = (n + kEmbRows - 1) / kEmbRows;
+  hipLaunchKernelGGL(grad_kernel, dim3(blocks + 16 * S.np + 4 * S.ne + 1), dim3(256), 0, st, S);
+  AdamArgs P{};
+  auto par = [](DBuf<float> &p, DBuf<float> &g, DBuf<float> &mm, DBuf<float> &v) { return Param{p.p, g.p, mm.p, v.p}; };
+  P.W[0] = par(m->W1, m->gW1, m->mW1, m->vW1);
+  P.W[1] = par(m->W2, m->gW2, m->mW2, m->vW2);
+  P.W[2] = par(m->W3, m->gW3, m->mW3, m->vW3);
+  P.emb = par(m->emb, m->gemb, m->memb, m->vemb);
+  P.col[0] = par(m->w4, m->gw4, m->mw4, m->vw4);
+  P.col[1] = par(m->b3, m->gb3, m->mb3, m->vb3);
+  P.col[2] = par(m->b2, m->gb2, m->mb2, m->vb2);
+  P.col[3] = par(m->b1, m->gb1, m->mb1, m->vb1);
+  P.b4 = par(m->b4, m->gb4, m->mb4, m->vb4);
+  uint16_t *pf[3] = {m->p1.p, m->p2.p, m->p3.p}, *pt[3] = {m->p1t.p, m->p2t.p, m->p3t.p};
+  int elems = 0;
+  for (int w = 0; w < 3; ++w) {
+    P.wpart[w] = ws[w];
+    P.wrows[w] = rows[w];
+    P.pf[w] = pf[w];
+    P.pt[w] = pt[w];
+    elems += rows[w] * Hd;
+  }
+  for (int w = 0; w < 3; ++w) P.ks[w] = ks[w];
+  P.demb = m->demb.p;
+  P.n_emb = (int)m->emb.n;
+  P.nelem = (elems + P.n_emb + 255) / 256;
+  P.part = m->part.p;
+  P.err = m->rerr.p;
+  P.np = S.np;
+  P.n = n;
+  P.loss_out = loss_out;
+  P.lr = lr;
   if (lr > 0.f) {
     m->step++;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float c1 = 1.f - std::pow(b1, (float)m->step), c2 = 1.f - std::pow(b2, (float)m->step);
-    AdamSet S{};
-    int nq = 0;
-    auto ad = [&](DBuf<float> &p, DBuf<float> &g, DBuf<float> &mm, DBuf<float> &vv, uint16_t *pb) {
-      S.p[nq] = p.p;
-      S.g[nq] = g.p;
-      S.m[nq] = mm.p;
-      S.v[nq] = vv.p;
-      S.pb[nq] = pb;
-      S.start[nq + 1] = S.start[nq] + (int64_t)p.n;
-      ++nq;
-    };
-    ad(m->W1, m->gW1, m->mW1, m->vW1, m->W1b.p);
-    ad(m->W2, m->gW2, m->mW2, m->vW2, m->W2b.p);
-    ad(m->W3, m->gW3, m->mW3, m->vW3, m->W3b.p);
-    ad(m->b1, m->gb1, m->mb1, m->vb1, nullptr);
-    ad(m->b2, m->gb2, m->mb2, m->vb2, nullptr);
-    ad(m->b3, m->gb3, m->mb3, m->vb3, nullptr);
-    ad(m->w4, m->gw4, m->mw4, m->vw4, nullptr);
-    ad(m->emb, m->gemb, m->memb, m->vemb, nullptr);
-    ad(m->b4, m->gb4, m->mb4, m->vb4, nullptr);
-    QPX_REQUIRE(nq == kAdamTensors, "Adam tensor count");
-    hipLaunchKernelGGL(adam_multi_kernel, dim3(grid1(S.start[kAdamTensors])), dim3(256), 0, st, S, lr, b1, b2, eps,
-                       c1, c2);
-    QPX_HIP(hipGetLastError());
+    P.b1 = 0.9f; P.b2 = 0.999f; P.eps = 1e-8f;
+    P.c1 = 1.f - std::pow(P.b1, (float)m->step);
+    P.c2 = 1.f - std::pow(P.b2, (float)m->step);
   }
-  // the step's mean squared error, left on the device
-  hipLaunchKernelGGL(loss_reduce_kernel, dim3(1), dim3(256), 0, st, m->lossp.p, nb, n, loss_out);
+  hipLaunchKernelGGL(adam_kernel, dim3(P.nelem + (4 * Hd + 1 + 3) / 4 + 1), dim3(256), 0, st, P);
   QPX_HIP(hipGetLastError());
-}
-
-// one step with its loss returned (synchronises the stream)
-float train_step(qpx_mlp *m, int n, float lr) {
-  train_step_async(m, n, lr, m->lossp.p + 1024);
-  float l = 0.f;
-  QPX_HIP(hipMemcpyAsync(&l, m->lossp.p + 1024, sizeof(float), hipMemcpyDeviceToHost, m->st));
-  QPX_HIP(hipStreamSynchronize(m->st));
-  return l;
-}
-
-// batch rows of the device-resident training set, in permutation order
-__global__ void gather_batch_kernel(const int *__restrict__ perm, int nb, const int *__restrict__ desc_all,
-                                    const float *__restrict__ fdesc_all, const float *__restrict__ tgt_all,
-                                    int *__restrict__ desc, float *__restrict__ fdesc, float *__restrict__ tgt) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nb) return;
-  const int64_t r = perm[i];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) desc[4 * (int64_t)i + q] = desc_all[4 * r + q];
-#pragma unroll
-  for (int q = 0; q < 3; ++q) fdesc[3 * (int64_t)i + q] = fdesc_all[3 * r + q];
-  tgt[i] = tgt_all[r];
 }
 
 template <typename F>
@@ -673,10 +895,13 @@ int mguard(qpx_mlp *m, F &&f) {
 // bounds, so it is rejected on the host before anything is uploaded.
 void check_desc(const qpx_mlp *m, int64_t n, const int *desc) {
   QPX_REQUIRE(desc, "null descriptor array");
+  const unsigned lim[4] = {(unsigned)m->n_orb, (unsigned)m->n_orb, 3u, 5u};   // negative values wrap above them
+  unsigned bad = 0;
+  for (int64_t i = 0; i < 4 * n; ++i) bad |= (unsigned)desc[i] >= lim[i & 3];   // no early exit: this vectorises
+  if (!bad) return;
   for (int64_t i = 0; i < n; ++i) {
     const int *d = desc + 4 * i;
-    if (d[0] < 0 || d[0] >= m->n_orb || d[1] < 0 || d[1] >= m->n_orb || d[2] < 0 || d[2] > 2 || d[3] < 0 ||
-        d[3] > 4) {
+    if ((unsigned)d[0] >= lim[0] || (unsigned)d[1] >= lim[1] || (unsigned)d[2] >= lim[2] || (unsigned)d[3] >= lim[3]) {
       char buf[160];
       std::snprintf(buf, sizeof buf, "descriptor row %lld = (%d, %d, %d, %d) out of range (n_orb = %d)",
                     (long long)i, d[0], d[1], d[2], d[3], m->n_orb);
@@ -701,7 +926,7 @@ extern "C" int qpx_mlp_create(int device, int n_orb, uint64_t seed, qpx_mlp **ou
   if (!out) return 1;
   qpx_mlp *m = new qpx_mlp();
   int rc = mguard(m, [&] {
-    QPX_REQUIRE(n_orb > 0 && n_orb <= 256, "n_orb must be in 1..256");
+    QPX_REQUIRE(n_orb > 0 && n_orb <= kMaxOrb, "n_orb must be in 1..256");
     QPX_HIP(hipSetDevice(device));
     m->device = device;
     m->n_orb = n_orb;
@@ -727,10 +952,12 @@ extern "C" int qpx_mlp_create(int device, int n_orb, uint64_t seed, qpx_mlp **ou
     m->b1.upload(z, m->st);
     m->b2.upload(z, m->st);
     m->b3.upload(z, m->st);
-    m->W1b.alloc((size_t)D * Hd); m->W2b.alloc((size_t)Hd * Hd); m->W3b.alloc((size_t)Hd * Hd);
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(64), dim3(256), 0, m->st, m->W1.p, m->W1b.p, (int64_t)D * Hd);
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(64), dim3(256), 0, m->st, m->W2.p, m->W2b.p, (int64_t)Hd * Hd);
-    hipLaunchKernelGGL(to_bf16_kernel, dim3(64), dim3(256), 0, m->st, m->W3.p, m->W3b.p, (int64_t)Hd * Hd);
+    m->p1.alloc(kPack1); m->p2.alloc(kPack); m->p3.alloc(kPack);
+    m->p1t.alloc(kPack1t); m->p2t.alloc(kPack); m->p3t.alloc(kPack);
+    QPX_HIP(hipMemsetAsync(m->p1.p, 0, sizeof(uint16_t) * kPack1, m->st));   // features 80..95 of the last step
+    hipLaunchKernelGGL(pack_kernel, dim3(64), dim3(256), 0, m->st, m->W1.p, D, m->p1.p, m->p1t.p);
+    hipLaunchKernelGGL(pack_kernel, dim3(64), dim3(256), 0, m->st, m->W2.p, Hd, m->p2.p, m->p2t.p);
+    hipLaunchKernelGGL(pack_kernel, dim3(64), dim3(256), 0, m->st, m->W3.p, Hd, m->p3.p, m->p3t.p);
     auto zero = [&](DBuf<float> &p, size_t n) {
       p.alloc(n);
       QPX_HIP(hipMemsetAsync(p.p, 0, sizeof(float) * n, m->st));
@@ -738,7 +965,7 @@ extern "C" int qpx_mlp_create(int device, int n_orb, uint64_t seed, qpx_mlp **ou
     zero(m->gW1, (size_t)D * Hd); zero(m->gW2, (size_t)Hd * Hd); zero(m->gW3, (size_t)Hd * Hd);
     zero(m->gb1, Hd); zero(m->gb2, Hd); zero(m->gb3, Hd); zero(m->gw4, Hd); zero(m->gb4, 1);
     zero(m->b4, 1); zero(m->mb4, 1); zero(m->vb4, 1);
-    zero(m->gemb, (size_t)n_orb * 32);
+    zero(m->gemb, (size_t)n_orb * 32); zero(m->demb, (size_t)n_orb * 32);
     zero(m->mW1, (size_t)D * Hd); zero(m->mW2, (size_t)Hd * Hd); zero(m->mW3, (size_t)Hd * Hd);
     zero(m->vW1, (size_t)D * Hd); zero(m->vW2, (size_t)Hd * Hd); zero(m->vW3, (size_t)Hd * Hd);
     zero(m->mb1, Hd); zero(m->mb2, Hd); zero(m->mb3, Hd); zero(m->mw4, Hd);
@@ -783,11 +1010,14 @@ extern "C" int qpx_mlp_train_step(qpx_mlp *m, int n, const int *desc, const floa
     QPX_REQUIRE(n > 0, "empty batch");
     QPX_REQUIRE(fdesc && target, "null argument");
     check_desc(m, n, desc);
-    ensure(m, n);
+    ensure_train(m, n);
     QPX_HIP(hipMemcpyAsync(m->desc.p, desc, sizeof(int) * 4 * n, hipMemcpyHostToDevice, m->st));
     QPX_HIP(hipMemcpyAsync(m->fdesc.p, fdesc, sizeof(float) * 3 * n, hipMemcpyHostToDevice, m->st));
     QPX_HIP(hipMemcpyAsync(m->tgt.p, target, sizeof(float) * n, hipMemcpyHostToDevice, m->st));
-    float l = train_step(m, n, lr);
+    train_step_async(m, n, nullptr, m->desc.p, m->fdesc.p, m->tgt.p, lr, m->lossp.p);
+    float l = 0.f;
+    QPX_HIP(hipMemcpyAsync(&l, m->lossp.p, sizeof(float), hipMemcpyDeviceToHost, m->st));
+    QPX_HIP(hipStreamSynchronize(m->st));
     if (loss) *loss = l;
   });
 }
@@ -799,7 +1029,7 @@ extern "C" int qpx_mlp_train_epochs(qpx_mlp *m, int n, const int *desc, const fl
     QPX_REQUIRE(n > 0 && batch >= 1 && batch <= n && epochs >= 1, "need 1 <= batch <= n and epochs >= 1");
     QPX_REQUIRE(desc && fdesc && target && epoch_loss, "null argument");
     check_desc(m, n, desc);
-    ensure(m, batch);
+    ensure_train(m, batch);
     DBuf<int> desc_all, perm_d;
     DBuf<float> fdesc_all, tgt_all;
     desc_all.upload(desc, (size_t)4 * n, m->st);
@@ -820,11 +1050,8 @@ extern "C" int qpx_mlp_train_epochs(qpx_mlp *m, int n, const int *desc, const fl
       }
       QPX_HIP(hipMemcpyAsync(perm_d.p, perm.data(), sizeof(int) * n, hipMemcpyHostToDevice, m->st));
       for (int q = 0; q < steps; ++q) {
-        hipLaunchKernelGGL(gather_batch_kernel, dim3((batch + 255) / 256), dim3(256), 0, m->st,
-                           perm_d.p + (size_t)q * batch, batch, desc_all.p, fdesc_all.p, tgt_all.p, m->desc.p,
-                           m->fdesc.p, m->tgt.p);
-        QPX_HIP(hipGetLastError());
-        train_step_async(m, batch, lr, step_loss.p + q);
+        train_step_async(m, batch, perm_d.p + (size_t)q * batch, desc_all.p, fdesc_all.p, tgt_all.p, lr,
+                         step_loss.p + q);
       }
       QPX_HIP(hipMemcpyAsync(sl.data(), step_loss.p, sizeof(float) * steps, hipMemcpyDeviceToHost, m->st));
       QPX_HIP(hipStreamSynchronize(m->st));
@@ -847,11 +1074,7 @@ extern "C" int qpx_mlp_predict(qpx_mlp *m, int n, const int *desc, const float *
       ensure(m, c);
       QPX_HIP(hipMemcpyAsync(m->desc.p, desc + 4 * (size_t)i0, sizeof(int) * 4 * c, hipMemcpyHostToDevice, m->st));
       QPX_HIP(hipMemcpyAsync(m->fdesc.p, fdesc + 3 * (size_t)i0, sizeof(float) * 3 * c, hipMemcpyHostToDevice, m->st));
-      forward(m, c);
-      const int nb = head_blocks(c);
-      hipLaunchKernelGGL(head_kernel, dim3(nb), dim3(256), 0, m->st, m->Z3.p, m->w4.p, m->b4.p, c, m->hid,
-                         (const float *)nullptr, m->y.p, (float *)nullptr, (float *)nullptr);
-      QPX_HIP(hipGetLastError());
+      predict_rows(m, c, m->desc.p, m->fdesc.p, m->y.p);
       QPX_HIP(hipMemcpyAsync(out + i0, m->y.p, sizeof(float) * c, hipMemcpyDeviceToHost, m->st));
     }
     QPX_HIP(hipStreamSynchronize(m->st));
@@ -869,14 +1092,14 @@ extern "C" int qpx_mlp_predict_static(qpx_mlp *m, int n, const int *desc, const 
     check_desc(m, n, desc);
     QPX_HIP(hipSetDevice(m->device));
     QPX_REQUIRE(m->scratch, "no prediction scratch on this device");
-    const FwdBufs b = static_bufs(m->scratch);
-    QPX_HIP(hipMemcpyAsync(const_cast<int *>(b.desc), desc, sizeof(int) * 4 * n, hipMemcpyHostToDevice, m->st));
-    QPX_HIP(hipMemcpyAsync(const_cast<float *>(b.fdesc), fdesc, sizeof(float) * 3 * n, hipMemcpyHostToDevice, m->st));
-    forward_bufs(m, n, b);
-    hipLaunchKernelGGL(head_kernel, dim3(head_blocks(n)), dim3(256), 0, m->st, b.Z3, m->w4.p, m->b4.p, n, m->hid,
-                       (const float *)nullptr, b.y, (float *)nullptr, (float *)nullptr);
-    QPX_HIP(hipGetLastError());
-    QPX_HIP(hipMemcpyAsync(out, b.y, sizeof(float) * n, hipMemcpyDeviceToHost, m->st));
+    unsigned char *base = static_cast<unsigned char *>(m->scratch);
+    int *dd = reinterpret_cast<int *>(base);
+    float *df = reinterpret_cast<float *>(base + al256(sizeof(int) * 4 * kStaticRows));
+    float *dy = reinterpret_cast<float *>(base + al256(sizeof(int) * 4 * kStaticRows) + al256(sizeof(float) * 3 * kStaticRows));
+    QPX_HIP(hipMemcpyAsync(dd, desc, sizeof(int) * 4 * n, hipMemcpyHostToDevice, m->st));
+    QPX_HIP(hipMemcpyAsync(df, fdesc, sizeof(float) * 3 * n, hipMemcpyHostToDevice, m->st));
+    predict_rows(m, n, dd, df, dy);
+    QPX_HIP(hipMemcpyAsync(out, dy, sizeof(float) * n, hipMemcpyDeviceToHost, m->st));
     QPX_HIP(hipStreamSynchronize(m->st));
   });
 }
@@ -909,8 +1132,8 @@ extern "C" int qpx_mlp_param(qpx_mlp *m, int which, int grad, int set, float *da
     if (set) {
       QPX_REQUIRE(!grad, "gradients are read-only");
       QPX_HIP(hipMemcpyAsync(b.p, data, sizeof(float) * n, hipMemcpyHostToDevice, m->st));
-      uint16_t *bb = which == 0 ? m->W1b.p : which == 1 ? m->W2b.p : which == 2 ? m->W3b.p : nullptr;
-      if (bb) hipLaunchKernelGGL(to_bf16_kernel, dim3(64), dim3(256), 0, m->st, b.p, bb, (int64_t)n);
+      uint16_t *pf[3] = {m->p1.p, m->p2.p, m->p3.p}, *pt[3] = {m->p1t.p, m->p2t.p, m->p3t.p};
+      if (which < 3) hipLaunchKernelGGL(pack_kernel, dim3(64), dim3(256), 0, m->st, b.p, (int)(n / m->hid), pf[which], pt[which]);
     } else {
       QPX_HIP(hipMemcpyAsync(data, b.p, sizeof(float) * n, hipMemcpyDeviceToHost, m->st));
     }
