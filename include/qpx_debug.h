@@ -19,7 +19,8 @@ extern "C" {
 /* Force the sigma path of later qpx_sigma / qpx_sigma_device / qpx_davidson
  * calls: 0 automatic, 1 string-driven kernels (product spaces) or else the
  * dense-map kernels (full-CI-like spaces), 2 scanning kernel, 3 sub-string
- * bucket kernel, 4 dense-map kernels.  *last_path reads 1 for both kinds of 1.  *last_path (may be NULL) receives the
+ * bucket kernels, 4 dense-map kernels, 5 sub-string buckets walked determinant
+ * by determinant.  *last_path reads 1 for 1 and 4, 3 for 3 and 5.  *last_path (may be NULL) receives the
  * path the previous sigma call took.  A forced path that does not apply to
  * the wavefunction makes the sigma call fail. */
 int qpx_debug_force_sigma_path(qpx_ctx *ctx, int path, int *last_path);

@@ -24,7 +24,7 @@ FLAGS = [
     "-ffp-contract=fast",
 ]
 
-SOURCES = ["context.hip", "wavefunction.hip", "sigma.hip", "sigma_fci.hip", "sigma_sparse.hip", "davidson.hip", "selection.hip", "mlp.hip",
+SOURCES = ["context.hip", "wavefunction.hip", "sigma.hip", "sigma_fci.hip", "sigma_sparse.hip", "sigma_pairs.hip", "davidson.hip", "selection.hip", "mlp.hip",
            "psi_update.hip", "s2_complete.hip"]
 
 

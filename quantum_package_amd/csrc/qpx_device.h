@@ -87,6 +87,32 @@ __device__ inline void double_hp(const uint64_t *a, const uint64_t *b, int *h1, 
   }
 }
 
+// the k-th set bit (0-based) of a string
+template <int NI>
+__device__ inline int kth_bit(const uint64_t *x, int k) {
+#pragma unroll
+  for (int w = 0; w < NI; ++w) {
+    const int c = __popcll(x[w]);
+    if (k < c) {
+      uint64_t y = x[w];
+      for (int q = 0; q < k; ++q) y &= y - 1;
+      return 64 * w + __ffsll((unsigned long long)y) - 1;
+    }
+    k -= c;
+  }
+  return -1;
+}
+
+__device__ inline void pair_of(int sl, int ne, int *i, int *j) {   // lexicographic (i < j) of slot sl
+  int a = 0;
+  while (sl >= ne - 1 - a) {
+    sl -= ne - 1 - a;
+    ++a;
+  }
+  *i = a;
+  *j = a + 1 + sl;
+}
+
 // <I|H|I> from orbital occupations: one-electron terms, same-spin pairs
 // J-K, opposite-spin pairs J.
 template <int NI>

@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 #include <cstdint>
 #include <string>
+#include <memory>
 #include <vector>
 #include <stdexcept>
 #include "../../include/qpx.h"
@@ -82,6 +83,10 @@ struct Ham {
   // the sparse sigma path when M <= kG4MaxOrb (ensure_g4)
   DBuf<double> G4;
   DBuf<float> G4f;
+  // integrals and HF elements of the bucket-by-bucket sparse sigma, per
+  // precision on first use (sigma_pairs.hip)
+  DBuf<double> Pt, Pf;
+  DBuf<float> Ptf, Pff;
   double ref_energy = 0.0;        // ref_bitmask_energy of the HF determinant
 };
 
@@ -152,6 +157,24 @@ struct FciPlan {
   }
 };
 
+// Entries of the bucket-by-bucket sparse sigma (sigma_pairs.hip): double
+// excitations [0, n_dbl), those of buckets of 64 and more in front, alpha singles [n_dbl, alpha_end), beta singles
+// [alpha_end, n_all).
+struct PairIdx {
+  bool valid = false, failed = false;
+  int64_t n_big = 0, n_dbl = 0, alpha_end = 0, n_all = 0;
+  int S = 0;                  // slots of a determinant
+  DBuf<uint2> ent;
+  DBuf<uint32_t> off, xlist;
+  DBuf<int2> wave;            // buckets of a wavefront's 64 entries
+  DBuf<int> slotpos, xptr;    // entry of each slot; spin exchanges of each determinant
+  void clear() { valid = failed = false; }   // the next wavefunction may take the arrays
+  void release() {
+    clear();
+    ent.release(); off.release(); xlist.release(); wave.release(); slotpos.release(); xptr.release();
+  }
+};
+
 struct Wfn {
   int64_t n_det = 0;
   int nint = 0;
@@ -172,6 +195,7 @@ struct Wfn {
   std::vector<int> col_len_h, row_len_h;
   int max_col = 0, max_row = 0;
   SparseIdx sp;                           // built on first use of the sparse path
+  PairIdx pr;                             // built on first use of the sparse path
   FciPlan fci;                            // built on first use of the product-space path
 };
 
@@ -193,15 +217,50 @@ struct StreamWorkspace {
   ~StreamWorkspace() {
     if (done) (void)hipEventDestroy(done);
   }
-  static bool capturing(hipStream_t s) {
+  // A captured graph owns its scratch (one buffer per capture and stream, till
+  // the wavefunction it was captured for goes): it may be replayed on any
+  // stream, beside other calls and after calls that need more.
+  struct Captured {
+    hipStream_t s;
+    unsigned long long id;
+    DBuf<char> buf;
+  };
+  std::vector<std::unique_ptr<Captured>> graphs;
+  static bool capturing(hipStream_t s, unsigned long long *id = nullptr) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return hipStreamIsCapturing(s, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+    unsigned long long x = 0;
+    if (hipStreamGetCaptureInfo(s, &cs, &x) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    if (id) *id = x;
+    return cs != hipStreamCaptureStatusNone;
   }
   char *get(size_t bytes, hipStream_t s) {
-    if (pending && last != s && !capturing(s)) QPX_HIP(hipStreamWaitEvent(s, done, 0));
+    unsigned long long id = 0;
+    if (capturing(s, &id)) {
+      for (auto &g : graphs)
+        if (g->s == s && g->id == id && g->buf.n >= bytes) return g->buf.p;
+      auto g = std::make_unique<Captured>();
+      g->s = s;
+      g->id = id;
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // lets this thread allocate
+      QPX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+      const hipError_t e = hipMalloc((void **)&g->buf.p, bytes);
+      QPX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+      QPX_HIP(e);
+      g->buf.n = bytes;
+      graphs.push_back(std::move(g));
+      return graphs.back()->buf.p;
+    }
+    if (pending && last != s) QPX_HIP(hipStreamWaitEvent(s, done, 0));
     // hipFree waits for the device, so the old buffer is not in use any more
     if (buf.n < bytes) buf.alloc(bytes);
     return buf.p;
+  }
+  void release() {
+    buf.release();
+    pending = false;
   }
   void used(hipStream_t s) {
     if (capturing(s)) return;
@@ -226,6 +285,7 @@ struct qpx_ctx {
   qpx::Workspace ws_sigma_io;   // host-order u/v/s staging for qpx_sigma
   qpx::Workspace ws_sigma_t;    // transposed u_t/v_t/s_t
   qpx::Workspace ws_misc;
+  qpx::StreamWorkspace ws_pairs;  // sums of the entries (sigma_pairs.hip)
   qpx::StreamWorkspace ws_fci;  // planes of u and the same-spin part (sigma_fci.hip)
   int64_t sel_stats[4] = {0, 0, 0, 0};
   std::vector<int64_t> sel_ticks;   // per-block durations of the last selection (benchmark hook)
@@ -246,6 +306,8 @@ void build_wavefunction(qpx_ctx *c, int n_int, int64_t n_det, const uint64_t *ps
 void ensure_conn(qpx_ctx *c);
 // implemented in sigma.hip
 void sigma_device(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, void *s_t, hipStream_t s);
+// implemented in sigma_pairs.hip
+bool sigma_pairs(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, void *s_t, hipStream_t s);
 // implemented in sigma_fci.hip
 bool fci_ok(qpx_ctx *c, int n_st, size_t tsize);
 bool sigma_fci(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, void *s_t, hipStream_t s);

@@ -695,6 +695,13 @@ static bool dense_ok(qpx_ctx *c, int nst, size_t tsize) {
   return W.ca.max_singles <= 96;
 }
 
+// gives back what the sparse path keeps for later wavefunctions once one takes another path
+static void release_pairs(qpx_ctx *c, hipStream_t st) {
+  if (c->W.pr.valid || !c->W.pr.ent.p || StreamWorkspace::capturing(st)) return;
+  c->W.pr.release();
+  c->ws_pairs.release();
+}
+
 void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, hipStream_t st) {
   QPX_REQUIRE(c->W.valid, "no wavefunction set");
   QPX_REQUIRE(nst >= 1 && nst <= GMAXST, "n_st must be in 1..8");
@@ -705,17 +712,19 @@ void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s
   if ((c->force_path == 0 || c->force_path == 1) && fci_ok(c, nst, ts) &&
       sigma_fci(c, prec, nst, u, v, s, st)) {
     c->sigma_path = 1;
+    release_pairs(c, st);
     return;
   }
   bool dense = dense_ok(c, nst, ts);
-  if (c->force_path == 2 || c->force_path == 3) dense = false;
+  if (c->force_path == 2 || c->force_path == 3 || c->force_path == 5) dense = false;
   if (c->force_path == 1 || c->force_path == 4) QPX_REQUIRE(dense, "dense-map sigma path not applicable to this wavefunction");
   if (!dense && c->force_path != 2 && sparse_ok(c, nst)) {
     c->sigma_path = 3;
     sigma_sparse(c, prec, nst, u, v, s, st);
     return;
   }
-  QPX_REQUIRE(c->force_path != 3, "sparse sigma path not applicable to this wavefunction");
+  release_pairs(c, st);
+  QPX_REQUIRE(c->force_path != 3 && c->force_path != 5, "sparse sigma path not applicable to this wavefunction");
   const Wfn &W = c->W;
   if (dense) {
     c->sigma_path = 1;
@@ -854,8 +863,8 @@ extern "C" int qpx_debug_lds_bandwidth(qpx_ctx *c, double *bytes_per_s) {
 // test hook: the sigma path of later calls (include/qpx_debug.h)
 extern "C" int qpx_debug_force_sigma_path(qpx_ctx *c, int path, int *last_path) {
   return qpx_guard(c, [&] {
-    QPX_REQUIRE(path >= 0 && path <= 4, "path must be 0 (automatic), 1 (string-driven or dense map), 2 (generic scan), "
-                                        "3 (sparse buckets) or 4 (dense map)");
+    QPX_REQUIRE(path >= 0 && path <= 5, "path must be 0 (automatic), 1 (string-driven or dense map), 2 (generic scan), "
+                                        "3 (sparse buckets), 4 (dense map) or 5 (sparse buckets, walked by determinant)");
     c->force_path = path;
     if (last_path) *last_path = c->sigma_path;
   });

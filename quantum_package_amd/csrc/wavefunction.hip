@@ -350,6 +350,9 @@ void build_wavefunction(qpx_ctx *c, int nint, int64_t n_det, const uint64_t *psi
   W.valid = false;
   W.sp.clear();
   W.fci.clear();
+  W.pr.clear();
+  c->ws_fci.graphs.clear();
+  c->ws_pairs.graphs.clear();
   W.perm.clear();
   W.n_det = n_det;
   W.nint = nint;

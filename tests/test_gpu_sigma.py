@@ -6,6 +6,8 @@ vector norm.
 """
 from __future__ import annotations
 
+import os
+import subprocess
 import sys
 
 import numpy as np
@@ -273,3 +275,103 @@ def test_sigma_product_space(ctx, M, na, nb, drop, nst):
     ctx._force_sigma_path(0)
     assert np.linalg.norm(v - vo) < 2e-5 * np.linalg.norm(vo)
     assert np.linalg.norm(s - so) < 2e-5 * max(1.0, np.linalg.norm(so))
+
+
+def _singles_space(M, na, nb, keep, seed):
+    """determinants whose alpha and beta strings are HF or single excitations
+    of it, a share `keep` of them, in random order: the buckets of HF less one
+    orbital of each spin hold keep * (M - na + 1) * (M - nb + 1) members"""
+    rng = np.random.default_rng(seed)
+    n_int = (M + 63) // 64
+    def strings(ne):
+        occ = list(range(1, ne + 1))
+        out = [occ] + [sorted([o for o in occ if o != h] + [p]) for h in occ for p in range(ne + 1, M + 1)]
+        return [list_to_bitstring(o, n_int) for o in out]
+    a, b = strings(na), strings(nb)
+    pick = np.flatnonzero(rng.random(len(a) * len(b)) < keep)
+    pick = np.union1d(pick, [0])
+    rng.shuffle(pick)
+    return np.array([[a[k // len(b)], b[k % len(b)]] for k in pick], dtype=np.uint64)
+
+
+# largest bucket: 4, 20, about 100 (64..255 members), 300 (256 and more, one to
+# three words of a spin string)
+BUCKETS = [(6, 2, 1, 0.7), (8, 3, 2, 0.6), (14, 3, 2, 0.7), (20, 3, 2, 0.9), (20, 1, 1, 0.9), (70, 2, 1, 0.25),
+           (130, 1, 1, 0.03)]
+
+
+@pytest.mark.parametrize("M,na,nb,keep", BUCKETS)
+@pytest.mark.parametrize("nst", [1, 3, 4, 8])
+def test_sigma_sparse_buckets(ctx, M, na, nb, keep, nst):
+    """The sums by bucket (3) and by determinant (5) against the oracle, and
+    the automatic choice between them (0): the bounds of the tests above."""
+    dets = _singles_space(M, na, nb, keep, M + nst)
+    _say(f"[sigma buckets] M={M} {na}a{nb}b n_det={dets.shape[0]} nst={nst}")
+    H = synthetic_hamiltonian(M, na, nb, seed=M)
+    ctx.set_hamiltonian(H)
+    ctx.set_wavefunction(dets)
+    u = np.random.default_rng(nst).standard_normal((dets.shape[0], nst))
+    vo, so = O.sigma(O.Ham(H), O.Bilinear(dets), u)
+    for path in (3, 5, 0):
+        ctx._force_sigma_path(path)
+        v, s = ctx.H_S2_u_0_nstates(u)
+        assert np.max(np.abs(v - vo)) < 1e-11 * max(1.0, np.max(np.abs(vo)))
+        assert np.max(np.abs(s - so)) < 1e-11 * max(1.0, np.max(np.abs(so)))
+        w, t = ctx.H_S2_u_0_nstates(u)
+        assert np.array_equal(v, w) and np.array_equal(s, t)     # every sum has a fixed order
+        v, s = ctx.H_S2_u_0_nstates(u, prec=1)
+        assert np.linalg.norm(v - vo) < 2e-5 * np.linalg.norm(vo)
+        assert np.linalg.norm(s - so) < 2e-5 * max(1.0, np.linalg.norm(so))
+    ctx._force_sigma_path(0)
+
+
+@pytest.mark.parametrize("path", [1, 3])
+def test_sigma_captured(path):
+    """A captured sigma keeps its scratch: replays between eager calls that
+    need more, on another stream, give the eager call's bits.  In a process of
+    its own, where torch starts the HIP runtime."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    code = f"import sys, torch; torch.cuda.init(); sys.path[:0] = {[here, os.path.dirname(here)]!r}; " \
+           f"import test_gpu_sigma as t; t._captured({path})"
+    r = subprocess.run([sys.executable, "-u", "-c", code], capture_output=True, text=True, timeout=100)
+    _say(r.stdout + r.stderr)
+    assert r.returncode == 0
+
+
+def _captured(path):
+    import torch
+    from quantum_package_amd.api import Context
+    ctx = Context(0)
+    dets = fci_space(10, 4, 3) if path == 1 else _singles_space(20, 3, 2, 0.9, 1)
+    ctx.set_hamiltonian(synthetic_hamiltonian(10 if path == 1 else 20, 4 if path == 1 else 3, 3 if path == 1 else 2, seed=4))
+    ctx.set_wavefunction(dets)
+    ctx._force_sigma_path(path)
+    n = dets.shape[0]
+
+    def run(nst, u, v, s, stream):
+        ctx._check(ctx.L.qpx_sigma_device(ctx.ptr, 0, nst, u.data_ptr(), v.data_ptr(), s.data_ptr(), stream.cuda_stream))
+
+    u = torch.randn(n, dtype=torch.float64, device="cuda")
+    big = torch.randn(4 * n, dtype=torch.float64, device="cuda")
+    v, s, ve, se = (torch.zeros_like(u) for _ in range(4))
+    vb, sb = torch.zeros_like(big), torch.zeros_like(big)
+    st, other = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    _say(f"[sigma captured] path={path} n_det={n}")
+    run(1, u, ve, se, st)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=st):
+        run(1, u, v, s, st)
+    for _ in range(3):
+        run(4, big, vb, sb, other)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(v, ve) and torch.equal(s, se)
+        v.zero_()
+        s.zero_()
+        u.copy_(torch.randn(n, dtype=torch.float64, device="cuda"))
+        torch.cuda.synchronize()
+        run(1, u, ve, se, other)
+        torch.cuda.synchronize()
+    ctx.close()
