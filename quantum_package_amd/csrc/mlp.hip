@@ -64,14 +64,9 @@ struct GemmArgs {
   float *C;           // C(i,j) = C[i*c_rs + j]
   int64_t c_rs;
   int M, N, K;
-  const float *bias;  // per column j (nullable)
-  int relu;           // epilogue: C = relu(C + bias)
-  uint16_t *Cb;       // optional bf16 copy of C (same layout)
-  float beta;         // C = acc + beta * C_old (gradient accumulation)
   float *part;        // split-K partial products (ksplit x M x N), or null
   int ksplit;         // K is cut into ksplit chunks (blockIdx.z); 1 = no split
   int a_run, b_run;   // staging: 1 = runs along k, 2 = along i (A) / j (B), 0 = element by element
-  const float *mask;  // optional: C(i,j) = 0 where mask(i,j) <= 0 (same layout as C; a ReLU's backward)
   int to_part;        // write slices to part whatever their number
 };
 
@@ -169,14 +164,7 @@ __device__ inline void gemm_tile(const GemmArgs &g, int bx, int by, int bz) {
         if (gi < g.M && gj < g.N && (g.ksplit > 1 || g.to_part)) {
           g.part[((int64_t)bz * g.M + gi) * g.N + gj] = acc[a][b][t];
         } else if (gi < g.M && gj < g.N) {
-          float v = acc[a][b][t];
-          float *c = g.C + gi * g.c_rs + gj;
-          if (g.beta != 0.f) v += g.beta * (*c);
-          if (g.bias) v += g.bias[gj];
-          if (g.relu) v = v > 0.f ? v : 0.f;
-          if (g.mask) v = g.mask[gi * g.c_rs + gj] > 0.f ? v : 0.f;
-          *c = v;
-          if (g.Cb) g.Cb[gi * g.c_rs + gj] = f2bf(v);
+          g.C[gi * g.c_rs + gj] = acc[a][b][t];
         }
       }
 }
@@ -185,7 +173,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_kernel(GemmArgs g) {
   gemm_tile(g, (int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z);
 }
 
-// split-K: C = sum of the partial products in slice order, then the epilogue
+// split-K: C = sum of the partial products in slice order
 __global__ void gemm_splitk_reduce_kernel(GemmArgs g) {
   const int64_t mn = (int64_t)g.M * g.N;
   for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < mn; x += (int64_t)gridDim.x * blockDim.x) {
@@ -194,13 +182,7 @@ __global__ void gemm_splitk_reduce_kernel(GemmArgs g) {
     // unrolled so that the slice loads are in flight together; the adds stay in slice order
 #pragma unroll 8
     for (int z = 0; z < g.ksplit; ++z) v += g.part[(int64_t)z * mn + x];
-    float *c = g.C + gi * g.c_rs + gj;
-    if (g.beta != 0.f) v += g.beta * (*c);
-    if (g.bias) v += g.bias[gj];
-    if (g.relu) v = v > 0.f ? v : 0.f;
-    if (g.mask) v = g.mask[gi * g.c_rs + gj] > 0.f ? v : 0.f;
-    *c = v;
-    if (g.Cb) g.Cb[gi * g.c_rs + gj] = f2bf(v);
+    g.C[gi * g.c_rs + gj] = v;
   }
 }
 
@@ -706,12 +688,11 @@ struct qpx_mlp {
 
 namespace {
 
-// C = A B (+ epilogue).  With a workspace, a product whose tile grid
+// C = A B.  With a workspace, a product whose tile grid
 // leaves most CUs idle and whose K is long (the weight gradients, K = batch)
 // is cut along K across workgroups and reduced in slice order.
 void gemm(hipStream_t st, const uint16_t *A, int64_t ars, int64_t acs, const uint16_t *B, int64_t brs, int64_t bcs,
-          float *C, int64_t crs, int M, int N, int K, const float *bias, int relu, uint16_t *Cb, float beta,
-          DBuf<float> *ws = nullptr, const float *mask = nullptr) {
+          float *C, int64_t crs, int M, int N, int K, DBuf<float> *ws = nullptr) {
   // 16-byte runs need a 16-byte-aligned base and a multiple-of-8 stride
   // across runs
   const auto run_of = [](const uint16_t *P, int64_t rs, int64_t cs) {
@@ -720,8 +701,8 @@ void gemm(hipStream_t st, const uint16_t *A, int64_t ars, int64_t acs, const uin
     if (rs == 1 && cs % 8 == 0) return 2;
     return 0;
   };
-  GemmArgs g{A, ars, acs, B, brs, bcs, C, crs, M, N, K, bias, relu, Cb, beta, nullptr, 1,
-             run_of(A, ars, acs), run_of(B, bcs, brs), mask, 0};
+  GemmArgs g{A, ars, acs, B, brs, bcs, C, crs, M, N, K, nullptr, 1,
+             run_of(A, ars, acs), run_of(B, bcs, brs), 0};
   dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
   const int tiles = (int)(grid.x * grid.y);
   constexpr int kGrain = 16;   // split-K sizing unit (slices are then rounded up to TK)
@@ -818,8 +799,8 @@ void train_step_async(qpx_mlp *m, int n, const int *perm, const int *desc, const
     const int tiles = ((rows[w] + TM - 1) / TM) * (Hd / TN);
     ks[w] = n >= 128 ? std::max(1, std::min({256 / tiles, n / 64, kSlices})) : 1;
     // one slice, too, goes through the slices' buffer
-    S.g[w] = GemmArgs{a[w], 1, rows[w], b[w], Hd, 1, nullptr, Hd, rows[w], Hd, n, nullptr, 0, nullptr, 0.f, ws[w],
-                      ks[w], 2, 2, nullptr, 1};
+    S.g[w] = GemmArgs{a[w], 1, rows[w], b[w], Hd, 1, nullptr, Hd, rows[w], Hd, n, ws[w],
+                      ks[w], 2, 2, 1};
     S.blocks[w] = tiles * ks[w];
     blocks += S.blocks[w];
   }
@@ -1165,7 +1146,7 @@ extern "C" int qpx_debug_mlp_gemm(qpx_mlp *m, int M, int N, int K, const float *
     hipLaunchKernelGGL(to_bf16_kernel, dim3(64), dim3(256), 0, m->st, b.p, bb.p, (int64_t)K * N);
     const int64_t ars = ta ? 1 : K, acs = ta ? M : 1;
     const int64_t brs = tb ? 1 : N, bcs = tb ? K : 1;
-    gemm(m->st, ab.p, ars, acs, bb.p, brs, bcs, c.p, N, M, N, K, nullptr, 0, nullptr, 0.f, split ? &ws : nullptr);
+    gemm(m->st, ab.p, ars, acs, bb.p, brs, bcs, c.p, N, M, N, K, split ? &ws : nullptr);
     QPX_HIP(hipMemcpyAsync(C, c.p, sizeof(float) * M * N, hipMemcpyDeviceToHost, m->st));
     QPX_HIP(hipStreamSynchronize(m->st));
   });
@@ -1183,7 +1164,7 @@ extern "C" int qpx_mlp_gemm_check(qpx_mlp *m, int M, int N, int K, const float *
     c.alloc((size_t)M * N);
     hipLaunchKernelGGL(to_bf16_kernel, dim3(64), dim3(256), 0, m->st, a.p, ab.p, (int64_t)M * K);
     hipLaunchKernelGGL(to_bf16_kernel, dim3(64), dim3(256), 0, m->st, b.p, bb.p, (int64_t)K * N);
-    gemm(m->st, ab.p, K, 1, bb.p, N, 1, c.p, N, M, N, K, nullptr, 0, nullptr, 0.f);
+    gemm(m->st, ab.p, K, 1, bb.p, N, 1, c.p, N, M, N, K);
     QPX_HIP(hipMemcpyAsync(C, c.p, sizeof(float) * M * N, hipMemcpyDeviceToHost, m->st));
     QPX_HIP(hipStreamSynchronize(m->st));
   });

@@ -153,3 +153,38 @@ def test_out_of_range_descriptors_are_rejected(mlp):
             mlp.train_epochs(d, fdesc, y, 1e-3, 1, 16, 0)
     assert np.array_equal(mlp.get("W1"), before)
     assert np.isfinite(mlp.predict(desc, fdesc)).all()
+
+
+# a workgroup's rows (16, 32, 64) less and plus one, and both sides of the sizes
+# at which the number of rows per workgroup changes
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 33, 63, 65, 4097, 8191, 8192, 32767, 32769])
+def test_predict_row_tiles(mlp, n):
+    """The bound of test_gradients_vs_reference; and a row's prediction does
+    not depend on the rows beside it beyond that bound."""
+    rng = np.random.default_rng(n)
+    desc, fdesc, y = _random_batch(n, 40, rng)
+    P = {k: mlp.get(k).astype(np.float64) for k in ["W1", "W2", "W3", "b1", "b2", "b3", "w4", "emb", "b4"]}
+    P["b4"] = float(np.ravel(P["b4"])[0])
+    _say(f"[mlp row tiles] predict n={n}")
+    yr, _, _ = mlp_ref.forward_backward(P, desc, fdesc.astype(np.float64), y.astype(np.float64))
+    bound = 2e-2 * np.max(np.abs(yr)) + 1e-3
+    assert np.max(np.abs(mlp.predict(desc, fdesc) - yr)) <= bound
+    k = min(n, 20)
+    assert np.max(np.abs(mlp.predict(desc[-k:], fdesc[-k:]) - yr[-k:])) <= bound
+
+
+@pytest.mark.parametrize("n", [15, 17, 33, 4096, 4097])
+def test_gradients_row_tiles(mlp, n):
+    """The bounds of test_gradients_vs_reference at the edges of the row tiles."""
+    rng = np.random.default_rng(n)
+    desc, fdesc, y = _random_batch(n, 40, rng)
+    keys = ["W1", "W2", "W3", "b1", "b2", "b3", "w4", "emb", "b4"]
+    P = {k: mlp.get(k).astype(np.float64) for k in keys}
+    P["b4"] = float(np.ravel(P["b4"])[0])
+    _say(f"[mlp row tiles] gradients n={n}")
+    loss = mlp.train_step(desc, fdesc, y, lr=0.0)
+    _, lr_, g = mlp_ref.forward_backward(P, desc, fdesc.astype(np.float64), y.astype(np.float64))
+    assert abs(loss - lr_) <= 1e-2 * abs(lr_)
+    for k in keys:
+        gg = mlp.get(k, grad=True).astype(np.float64).reshape(np.shape(g[k]))
+        assert np.linalg.norm(gg - g[k]) < 3e-2 * np.linalg.norm(g[k]), k
