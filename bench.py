@@ -6,11 +6,11 @@ determinants, N_int = 1) with 4 vectors (3 roots + 1 extra, the Davidson
 block size) in FP64, inputs resident in HBM.  value = determinants / s.
 
 The JSON line also carries:
-  roofline      the dominant (column) kernel against its bound, the LDS
-                read bandwidth measured on this GPU: the alpha-beta pairs'
-                u-row and integral bytes it reads from LDS per launch over
-                its event-timed duration; with its measured HBM traffic
-                (rocprofv3 counters, calibrated) and the whole call's;
+  roofline      the dominant (alpha/beta) kernel against its bound, the
+                matrix cores: the multiply-adds of its products per launch
+                over its event-timed duration, against the dense MFMA peak
+                of the precision; with the whole call's measured HBM traffic
+                (rocprofv3 counters, calibrated);
   cpu_baseline  the CPU oracle (a C/OpenMP restatement of the reference's
                 H_S2_u_0_nstates_openmp_work, the reference itself cannot be
                 built here) timed on a bounded, strided sample of the same
@@ -159,28 +159,23 @@ def main():
                                                       __import__("ctypes").c_float)), 3))
     P = fci_pairs(M, na) * n_det
     B = sigma_alg_bytes(n_det, P, nst, w, 1)
-    traffic = traffic_col = None
-    tpath = os.path.join(ROOT, "profiles", "sigma_dense_fci14_traffic.json")
+    traffic = traffic_ab = None
+    tpath = os.path.join(ROOT, "profiles", "sigma_fci14_traffic.json")
     if os.path.exists(tpath):
         with open(tpath) as f:
             tj = json.load(f)
-        traffic = tj.get("hbm_bytes_per_sigma")
-        for name, kv in tj.get("kernels", {}).items():
-            if "sigma_dense_col_kernel" in name and ("double" if prec == FP64 else "float") in name:
-                traffic_col = kv.get("hbm_bytes")
-    # Roofline of the dominant kernel, the column kernel (about 80 % of the
-    # call).  It serves the alpha-beta pairs' reads -- per pair a row of u
-    # (8 N_st w bytes) and an integral (8 w) -- from LDS, where the survey's
-    # gather model counts them as HBM gathers; its bound is the LDS read
-    # bandwidth, measured on this GPU by a conflict-free LDS read kernel.
-    lds_peak = __import__("ctypes").c_double(0.0)
-    ctx._check(ctx.L.qpx_debug_lds_bandwidth(ctx.ptr, __import__("ctypes").byref(lds_peak)))
-    lds_peak = lds_peak.value
+        if prec == FP64:
+            traffic = tj.get("hbm_bytes_per_sigma")
+            for name, kv in tj.get("kernels", {}).items():
+                if "sigma_fci_ab_kernel" in name:
+                    traffic_ab = kv.get("hbm_bytes")
+    # Roofline of the dominant kernel, the alpha/beta one.  Per column of u and
+    # state it multiplies the integrals (orbital pairs p < q x beta singles)
+    # with rows of u: 2 N_det N_st n_s M (M - 1) / 2 flop.
     n_s = na * (M - na)
-    P_ab = n_det * n_s * n_s
-    lds_bytes = P_ab * (8 * nst + 8) * w
-    t_col = float(kms[0]) * 1e-3
-    achieved = lds_bytes / t_col
+    flop = 2.0 * n_det * nst * n_s * (M * (M - 1) // 2)
+    peak = MFMA_FP64_PEAK if prec == FP64 else MFMA_FP32_PEAK
+    t_ab = float(kms[1]) * 1e-3
 
     out = {
         "metric": METRIC,
@@ -199,17 +194,17 @@ def main():
                                "6 alpha + 6 beta electrons, 9,018,009 determinants, N_int=1, 4 vectors "
                                "(3 roots + 1, Davidson block)",
                    "n_det": n_det, "n_states_per_call": nst, "connected_pairs": P,
-                   "kernel_ms": {"sigma_dense_col": float(kms[0]), "sigma_dense_row": float(kms[1])}},
-        "roofline": {"bound": "lds", "kernel": f"sigma_dense_col_kernel ({'FP64' if prec == FP64 else 'FP32'}, "
-                                               f"{nst} vectors, {n_s} alpha singles per string)",
-                     "achieved": achieved / 1e9, "peak": lds_peak / 1e9, "unit": "GB/s", "frac": achieved / lds_peak,
-                     "traffic": traffic_col,
-                     "hbm_frac": (traffic_col / t_col / HBM_PEAK) if traffic_col else None,
-                     "alg_bytes_per_launch": lds_bytes,
-                     "note": ("achieved = alpha-beta pairs x (u row + integral) bytes read from LDS per launch / "
-                              "the column kernel's event-timed duration; peak = LDS read bandwidth measured on this "
-                              "GPU; traffic = the launch's HBM bytes (rocprofv3 FETCH_SIZE + WRITE_SIZE, "
-                              "calibrated), hbm_frac = traffic / duration / 8 TB/s"),
+                   "kernel_ms": {"sigma_fci_spin": float(kms[0]), "sigma_fci_ab": float(kms[1])}},
+        "roofline": {"bound": "mfma", "kernel": f"sigma_fci_ab_kernel ({'FP64' if prec == FP64 else 'FP32'}, "
+                                                f"{nst} vectors, {n_s} beta singles per string)",
+                     "achieved": flop / t_ab / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s", "frac": flop / t_ab / peak,
+                     "traffic": traffic_ab,
+                     "hbm_frac": (traffic_ab / t_ab / HBM_PEAK) if traffic_ab else None,
+                     "alg_flop_per_launch": flop,
+                     "note": ("achieved = multiply-adds of the integral x u products per launch / the alpha/beta "
+                              "kernel's event-timed duration; peak = dense MFMA peak of the precision; traffic = the "
+                              "launch's HBM bytes (rocprofv3 FETCH_SIZE + WRITE_SIZE, calibrated), hbm_frac = "
+                              "traffic / duration / 8 TB/s"),
                      "call": {"survey_gather_model_bytes": B, "traffic": traffic,
                               "hbm_frac": (traffic / (ms * 1e-3) / HBM_PEAK) if traffic else None}},
     }
@@ -314,6 +309,8 @@ def davidson_leg(ctx, H, dets, log):
 
 
 MFMA_BF16_PEAK = 2.5e15   # MI355X dense bf16 FLOP/s
+MFMA_FP64_PEAK = 78.6e12  # dense FP64 and FP32 matrix FLOP/s
+MFMA_FP32_PEAK = 157.3e12
 
 
 def mlp_leg(args, log):
@@ -363,9 +360,10 @@ def sparse_alg_bytes(n_det, visited, na, nb, nst, w):
     pairs (S_b likewise); a pair of alpha singles shares n_b ab buckets and
     n_a - 1 aa buckets, a determinant meets itself in every slot, so the
     connected pairs are ab = V_ab - N na nb - S_b na - S_a nb and
-    aa = V_aa - N na(na-1)/2 - S_a (na-1).  Bytes: 8 per visited payload, 8 per
-    (determinant, slot) range, an nst*w row of u per connected pair, w per
-    ab integral, 2w per same-spin double, (na+nb+1) w per single, and the
+    aa = V_aa - N na(na-1)/2 - S_a (na-1).  Bytes: w per double (its integral),
+    per (determinant, slot) 16 for the entry and its position and 3 nst*w for
+    the row of u and the entry's sums (written and read; slots whose bucket has
+    no second member are counted too), (na+nb+1) w per single, and the
     determinant's own u, v, s rows."""
     V = visited
     sa = V["a1"] - n_det * na
@@ -375,7 +373,7 @@ def sparse_alg_bytes(n_det, visited, na, nb, nst, w):
     bb = V["b2"] - n_det * nb * (nb - 1) // 2 - sb * (nb - 1)
     slots = na * nb + na + nb + na * (na - 1) // 2 + nb * (nb - 1) // 2
     pairs = ab + aa + bb + sa + sb
-    b = (8 * sum(V.values()) + 8 * n_det * slots + pairs * nst * w + ab * w + 2 * (aa + bb) * w
+    b = ((ab + aa + bb) * w + n_det * slots * (16 + 3 * nst * w)
          + (sa + sb) * (na + nb + 1) * w + 3 * n_det * nst * w)
     return b, {"ab": ab, "aa": aa, "bb": bb, "a": sa, "b": sb}
 
@@ -423,7 +421,7 @@ def selected_davidson_leg(args, log):
     # call (rocprofv3 FETCH_SIZE/WRITE_SIZE of this leg, calibrated) when the
     # committed summary is for this psi
     traffic = {}
-    tpath = os.path.join(ROOT, "profiles", "sigma_sparse_selected_m96_traffic.json")
+    tpath = os.path.join(ROOT, "profiles", "sigma_pairs_selected_m96_traffic.json")
     if os.path.exists(tpath):
         with open(tpath) as f:
             tj = json.load(f)

@@ -31,13 +31,13 @@
 // integral is read once for both of its determinants.
 //
 // 262,144 determinants, 96 orbitals, 10 + 10 electrons, FP64, 4 states: 7.6 ms
-// by determinant, here 2.3 (doubles 1.62, singles 0.21, collection 0.46);
-// 40,003, 50 orbitals, FP32, 2 states: 459 and 125 us.  The doubles read
-// 3.7 GB that miss L2 (an integral table of 0.85 GB in an order without
-// reuse), bound by those misses and the L1 look-ups of the scattered words: half
+// by determinant, here 2.3 (doubles 1.59, singles 0.21, collection 0.46);
+// 40,003, 50 orbitals, FP32, 2 states: 459 and 125 us.  The doubles read 7.5 GB
+// from HBM at 4.6 TB/s (an integral table of 0.85 GB in an order with little
+// reuse), the collection 3.2 GB at 7 TB/s: both at what the card gives, so half
 // the occupancy or twice the loads in flight changes nothing.  The table
 // packed by pair symmetry (0.34 GB) was slower, 1.82 ms: neighbouring lanes
-// no longer read neighbouring words.  The collection reads 1.6 GB at 3.5 TB/s.
+// no longer read neighbouring words.
 #include <algorithm>
 #include <type_traits>
 #include <vector>
@@ -525,6 +525,10 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
                                                            const T *__restrict__ tab, const T *__restrict__ u,
                                                            T *__restrict__ part) {
   __shared__ T row_u[256 * NST];
+  // 16 workgroups in a row to an XCD: they share a bucket's members and rows of the
+  // table in its L2 (1.62 -> 1.59 ms above; 2.1M determinants, the call 113 -> 107 ms)
+  int blk = (int)blockIdx.x;
+  if ((blk | 127) < (int)gridDim.x) blk = (blk & ~127) | (blk & 7) << 4 | (blk & 127) >> 3;
   __shared__ uint32_t row_base[256];
   const int lane = threadIdx.x & 63;
   const int sub = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -532,10 +536,10 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
   T acc[NST];
 #pragma unroll
   for (int st = 0; st < NST; ++st) acc[st] = T(0);
-  if ((int)blockIdx.x < nbig) {
+  if (blk < nbig) {
     // 64 entries of a bucket of kSplit and more: a quarter of the members each
-    const int64_t p = (int64_t)blockIdx.x * 64 + lane;
-    const int2 d = wave[blockIdx.x];
+    const int64_t p = (int64_t)blk * 64 + lane;
+    const int2 d = wave[blk];
     add_members<T, NST>(ent, d.x + (int)((int64_t)d.y * sub / 4), d.x + (int)((int64_t)d.y * (sub + 1) / 4), tab + off[p],
                         u, ru, acc);
 #pragma unroll
@@ -551,7 +555,7 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
     }
     return;
   }
-  const int wv = nbig + ((int)blockIdx.x - nbig) * 4 + sub;
+  const int wv = nbig + (blk - nbig) * 4 + sub;
   if (wv >= nwave) return;
   const int2 d = wave[wv];
   if (d.y == 0) return;
