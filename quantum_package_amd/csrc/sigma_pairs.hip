@@ -97,7 +97,7 @@ __device__ inline uint64_t sub_word(const uint64_t *str, int ne, int drop, int n
 template <int NI>
 __global__ void sub_key_kernel(const uint64_t *__restrict__ str, int ne, int drop, int nslot, int n, int w,
                                const int *__restrict__ ord, uint64_t *__restrict__ key) {
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x)
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
     key[t] = sub_word<NI>(str, ne, drop, nslot, ord[t], w);
 }
 __global__ void iota_kernel(int *__restrict__ v, int64_t n) {
@@ -106,7 +106,7 @@ __global__ void iota_kernel(int *__restrict__ v, int64_t n) {
 template <int NI>
 __global__ void sub_head_kernel(const uint64_t *__restrict__ str, int ne, int drop, int nslot, int n,
                                 const int *__restrict__ ord, int *__restrict__ head) {
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) {
     bool h = t == 0;
     for (int w = 0; w < NI && !h; ++w)
       h = sub_word<NI>(str, ne, drop, nslot, ord[t], w) != sub_word<NI>(str, ne, drop, nslot, ord[t - 1], w);
@@ -114,7 +114,7 @@ __global__ void sub_head_kernel(const uint64_t *__restrict__ str, int ne, int dr
   }
 }
 __global__ void sub_id_kernel(const int *__restrict__ ord, const int *__restrict__ sid, int n, int *__restrict__ id) {
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) id[ord[t]] = sid[t] - 1;
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x) id[ord[t]] = sid[t] - 1;
 }
 
 int grid_for(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 1 << 16)); }
@@ -878,7 +878,11 @@ bool build(qpx_ctx *c) {
       sort_class(c, A, Z, B[q], pass ? (uint64_t)std::max(1, hi[q]) * (uint64_t)B[q].C.mult : ~0ULL, d_cnt + 4 + q);
     if (pass) read_ints(d_cnt + 4, 5, nseg, s);
     for (int q = 0; q < 5; ++q) place_class(A, Z, B[q], pass ? nseg[q] : (int)B[q].n, first, d_cnt + 9 + 2 * q, s);
-    if (pass) read_ints(d_cnt + 9, 10, room, s);
+    if (pass) {
+      read_ints(d_cnt + 9, 10, room, s);
+      for (int q = 0; q < 5; ++q)
+        if (room[2 * q] < 0) return false;   // less than twice the entries, but 2^31 and more
+    }
     if (!pass) scan<false>(A, cx, cx, W.n_det + 1, s);
   }
   // the doubles' large buckets, their small ones, the singles
@@ -932,9 +936,8 @@ bool build(qpx_ctx *c) {
   QPX_HIP(hipMemsetAsync(cx + W.n_det, 0, sizeof(int), s));
   QPX_HIP(hipGetLastError());
   scan<false>(A, cx, X.xptr.p, W.n_det + 1, s);
-  int nx = 0;
+  int nx = 0;   // at most as many as alpha/beta slots
   read_ints(X.xptr.p + W.n_det, 1, &nx, s);
-  if (nx < 0) return false;   // more than 2^31 of them
   reserve(X.xlist, std::max(nx, 1));
   hipLaunchKernelGGL(exchange_kernel<NI>, dim3(g), dim3(256), 0, s, W.csc_a.p, W.csc_b.p, W.col_ptr.p, W.astr.p, W.n_a,
                      W.bstr.p, W.n_b, W.n_det, (const int *)X.xptr.p, cx, X.xlist.p);
