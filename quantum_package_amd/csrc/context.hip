@@ -145,6 +145,8 @@ extern "C" int qpx_set_hamiltonian(qpx_ctx *c, int M, int na, int nb, const doub
     QPX_REQUIRE(h_core && eri, "null Hamiltonian array");
     int64_t npair = (int64_t)M * (M + 1) / 2;
     QPX_REQUIRE(n8 == npair * (npair + 1) / 2, "eri_packed length must be npair*(npair+1)/2");
+    // sigma calls enqueued on a caller's stream may still read the integrals
+    QPX_HIP(hipDeviceSynchronize());
     Ham &H = c->H;
     H.M = M;
     H.na = na;

@@ -1,0 +1,96 @@
+"""Device sigma calls on callers' streams: what later calls of the context may
+and may not do to calls that are still queued and to captured graphs."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from quantum_package_amd.hamiltonian import fci_space, synthetic_hamiltonian
+from hip_rt import Arr, Hip
+from test_gpu_sigma import _random_space, _say, _singles_space
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def hip():
+    return Hip()
+
+
+@pytest.fixture()
+def ctx():
+    from quantum_package_amd.api import Context
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def _space(kind):
+    """(M, na, nb, determinants): a product space or a selected one"""
+    if kind == "product":
+        return 10, 4, 3, fci_space(10, 4, 3)
+    return 20, 3, 2, _singles_space(20, 3, 2, 0.9, 1)
+
+
+class Vectors:
+    """u, v, s of a device sigma call (bilinear order, state-fastest)"""
+
+    def __init__(self, hip, n, nst, prec, seed):
+        dt = np.float64 if prec == 0 else np.float32
+        a = np.random.default_rng(seed).standard_normal((n, nst)).astype(dt)
+        self.nst, self.prec = nst, prec
+        self.u, self.v, self.s = Arr(hip, a), Arr(hip, np.zeros_like(a)), Arr(hip, np.zeros_like(a))
+
+    def sigma(self, ctx, stream):
+        ctx._check(ctx.L.qpx_sigma_device(ctx.ptr, self.prec, self.nst, self.u.p, self.v.p, self.s.p, stream))
+
+    def out(self):
+        return self.v.get(), self.s.get()
+
+    def clear(self):
+        z = np.zeros(self.v.shape, dtype=self.v.dtype)
+        self.v.put(z)
+        self.s.put(z)
+
+    def free(self):
+        for a in (self.u, self.v, self.s):
+            a.free()
+
+
+def _same(x, y):
+    return all(np.array_equal(a, b) for a, b in zip(x, y))
+
+
+@pytest.mark.parametrize("what", ["wavefunction", "hamiltonian"])
+@pytest.mark.parametrize("path", [1, 3, 4, 5])
+def test_new_inputs_wait_for_queued_calls(ctx, hip, path, what):
+    """A wavefunction of the same sizes (every array is reused) or another
+    Hamiltonian, set while calls are queued on a caller's stream: the queued
+    calls give what they give alone, bit for bit."""
+    M, na, nb, dets = _space("product" if path in (1, 4) else "selected")
+    other = dets[:, :, 0].copy()
+    lo, hi = np.uint64(1) << np.uint64(M - 2), np.uint64(1) << np.uint64(M - 1)
+    swap = ((other & lo) != 0) ^ ((other & hi) != 0)       # the two highest orbitals trade places
+    other = np.where(swap, other ^ lo ^ hi, other)[:, :, None]
+    _say(f"[sigma queued] path={path} new {what} n_det={dets.shape[0]}")
+    ctx.set_hamiltonian(synthetic_hamiltonian(M, na, nb, seed=4))
+    ctx.set_wavefunction(dets)
+    ctx._force_sigma_path(path)
+    st = hip.stream()
+    x = Vectors(hip, dets.shape[0], 4, 0, 1)
+    x.sigma(ctx, st)
+    hip.sync()
+    alone = x.out()
+    for _ in range(3):
+        x.clear()
+        ctx.set_hamiltonian(synthetic_hamiltonian(M, na, nb, seed=4))
+        ctx.set_wavefunction(dets)
+        for _ in range(50):
+            x.sigma(ctx, st)
+        if what == "wavefunction":
+            ctx.set_wavefunction(other)
+        else:
+            ctx.set_hamiltonian(synthetic_hamiltonian(M, na, nb, seed=5))
+        hip.sync()
+        assert _same(x.out(), alone)
+    x.free()
