@@ -17,13 +17,23 @@ extern "C" {
 #endif
 
 /* Force the sigma path of later qpx_sigma / qpx_sigma_device / qpx_davidson
- * calls: 0 automatic, 1 string-driven kernels (product spaces) or else the
- * dense-map kernels (full-CI-like spaces), 2 scanning kernel, 3 sub-string
- * bucket kernels, 4 dense-map kernels, 5 sub-string buckets walked determinant
- * by determinant.  *last_path reads 1 for 1 and 4, 3 for 3 and 5.  *last_path (may be NULL) receives the
- * path the previous sigma call took.  A forced path that does not apply to
- * the wavefunction makes the sigma call fail. */
+ * calls: 0 automatic, 1 string-driven kernels or, where they do not apply,
+ * the dense-map kernels, 2 scanning kernel, 3 sub-string bucket kernels or,
+ * where they do not apply, the buckets walked determinant by determinant,
+ * 4 dense-map kernels, 5 the walk.  A forced path that does not apply to the
+ * wavefunction makes the sigma call fail.  *last_path (may be NULL) receives
+ * the path the previous sigma call took: 1 for the kernels 1 and 4, 2, or 3
+ * for the kernels 3 and 5. */
 int qpx_debug_force_sigma_path(qpx_ctx *ctx, int path, int *last_path);
+
+/* The kernels of the previous sigma call: 1 string-driven, 2 scan, 3 bucket by
+ * bucket, 4 dense map, 5 walk by determinant. */
+int qpx_debug_sigma_kernels(qpx_ctx *ctx, int *kernels);
+
+/* Makes device allocations of the calling thread above `above` bytes end with
+ * hip_error (a hipError_t; 0: out of memory) without asking the device; above
+ * < 0 ends it.  For the paths that need less memory and for error paths. */
+int qpx_debug_fail_alloc(int64_t above, int hip_error);
 
 /* One qpx_sigma_device call per repetition on `stream`; ms (2) receives the
  * average duration of its two kernel phases (string-driven path: same-spin

@@ -57,6 +57,8 @@ SIGNATURES = [
 # include/qpx_debug.h: test and benchmark hooks
 DEBUG = [
     ("qpx_debug_force_sigma_path", C.c_int, [c_vp, C.c_int, c_ip]),
+    ("qpx_debug_sigma_kernels", C.c_int, [c_vp, c_ip]),
+    ("qpx_debug_fail_alloc", C.c_int, [C.c_int64, C.c_int]),
     ("qpx_debug_sigma_kernel_times", C.c_int, [c_vp, C.c_int, C.c_int, c_vp, c_vp, c_vp, c_vp,
                                                C.POINTER(C.c_float), C.c_int]),
     ("qpx_debug_sparse_stats", C.c_int, [c_vp, c_i64p]),

@@ -253,6 +253,13 @@ class Context:
         self._check(self.L.qpx_debug_force_sigma_path(self.ptr, path, C.byref(last)))
         return last.value
 
+    def _sigma_kernels(self) -> int:
+        """The kernels of the last sigma call: 1 string-driven, 2 scan, 3 bucket by
+        bucket, 4 dense map, 5 walk by determinant."""
+        k = C.c_int(0)
+        self._check(self.L.qpx_debug_sigma_kernels(self.ptr, C.byref(k)))
+        return k.value
+
     def _select_block_ticks(self, n_blocks: int):
         """Per-block workgroup durations (100 MHz ticks) of the last selection
         call, in block enumeration order."""

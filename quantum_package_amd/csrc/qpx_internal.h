@@ -15,6 +15,12 @@ struct Error : std::runtime_error {
   Error(int c, const std::string &m) : std::runtime_error(m), code(c) {}
 };
 
+// No device memory for an allocation: a sigma call then takes a path that
+// needs less.  Every other error reaches the caller.
+struct OutOfMemory : Error {
+  using Error::Error;
+};
+
 #define QPX_HIP(call)                                                                          \
   do {                                                                                         \
     hipError_t e_ = (call);                                                                    \
@@ -34,6 +40,21 @@ constexpr int NINT_MAX = 4;
 // the pair matrix
 constexpr int kG4MaxOrb = 160;
 
+// Test hook (qpx_debug_fail_alloc): allocations of this thread above
+// fail_above bytes end with fail_with.
+inline thread_local size_t fail_above = SIZE_MAX;
+inline thread_local hipError_t fail_with = hipErrorOutOfMemory;
+
+inline void device_alloc(void **p, size_t bytes) {
+  const hipError_t e = bytes > fail_above ? fail_with : hipMalloc(p, bytes);
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    *p = nullptr;
+    throw OutOfMemory(2, "HIP error out of memory: " + std::to_string(bytes) + " bytes of device memory");
+  }
+  QPX_HIP(e);
+}
+
 // Device buffer with RAII.
 template <typename T>
 struct DBuf {
@@ -52,7 +73,7 @@ struct DBuf {
     if (count == n && p) return;
     release();
     if (count == 0) return;
-    QPX_HIP(hipMalloc(&p, count * sizeof(T)));
+    device_alloc((void **)&p, count * sizeof(T));
     n = count;
   }
   void upload(const T *h, size_t count, hipStream_t s) {
@@ -246,10 +267,13 @@ struct StreamWorkspace {
       g->id = id;
       hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // lets this thread allocate
       QPX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-      const hipError_t e = hipMalloc((void **)&g->buf.p, bytes);
+      try {
+        g->buf.alloc(bytes);
+      } catch (...) {
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+        throw;
+      }
       QPX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-      QPX_HIP(e);
-      g->buf.n = bytes;
       graphs.push_back(std::move(g));
       return graphs.back()->buf.p;
     }
@@ -289,7 +313,8 @@ struct qpx_ctx {
   qpx::StreamWorkspace ws_fci;  // planes of u and the same-spin part (sigma_fci.hip)
   int64_t sel_stats[4] = {0, 0, 0, 0};
   std::vector<int64_t> sel_ticks;   // per-block durations of the last selection (benchmark hook)
-  int sigma_path = 0;           // last sigma path: 1 = dense-map, 2 = generic scan, 3 = sparse buckets
+  int sigma_path = 0;           // last sigma path: 1 = string-driven or dense map, 2 = generic scan, 3 = sparse buckets
+  int sigma_kernels = 0;        // its kernels, numbered as the forced paths (qpx_debug.h)
   int force_path = 0;           // 0 auto, else the path to use (tests)
   int verbosity = 0;            // 1: Davidson iteration table on stderr
   hipEvent_t kev[3] = {nullptr, nullptr, nullptr};  // per-kernel timing (benchmark hook)

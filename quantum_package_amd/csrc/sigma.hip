@@ -711,7 +711,7 @@ void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s
   // 9.0M determinants, FP64, 4 states; 35 against 86 us for 4900)
   if ((c->force_path == 0 || c->force_path == 1) && fci_ok(c, nst, ts) &&
       sigma_fci(c, prec, nst, u, v, s, st)) {
-    c->sigma_path = 1;
+    c->sigma_path = c->sigma_kernels = 1;
     release_pairs(c, st);
     return;
   }
@@ -728,6 +728,7 @@ void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s
   const Wfn &W = c->W;
   if (dense) {
     c->sigma_path = 1;
+    c->sigma_kernels = 4;
     const int maxs = W.ca.max_singles;
     if (prec == QPX_FP64) {
       if (W.nint == 1) launch_dense_nst<double, 1>(c, nst, maxs, (const double *)u, (double *)v, (double *)s, st);
@@ -737,7 +738,7 @@ void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s
       else launch_dense_nst<float, 2>(c, nst, maxs, (const float *)u, (float *)v, (float *)s, st);
     }
   } else {
-    c->sigma_path = 2;
+    c->sigma_path = c->sigma_kernels = 2;
     ensure_conn(c);
     if (prec == QPX_FP64) launch_generic<double>(c, nst, (const double *)u, (double *)v, (double *)s, st);
     else launch_generic<float>(c, nst, (const float *)u, (float *)v, (float *)s, st);
@@ -868,6 +869,21 @@ extern "C" int qpx_debug_force_sigma_path(qpx_ctx *c, int path, int *last_path) 
     c->force_path = path;
     if (last_path) *last_path = c->sigma_path;
   });
+}
+
+// test hook: the kernels of the previous sigma call (include/qpx_debug.h)
+extern "C" int qpx_debug_sigma_kernels(qpx_ctx *c, int *kernels) {
+  return qpx_guard(c, [&] {
+    QPX_REQUIRE(kernels, "null output");
+    *kernels = c->sigma_kernels;
+  });
+}
+
+// test hook: makes this thread's larger device allocations fail
+extern "C" int qpx_debug_fail_alloc(int64_t above, int hip_error) {
+  fail_above = above < 0 ? SIZE_MAX : (size_t)above;
+  fail_with = hip_error > 0 ? (hipError_t)hip_error : hipErrorOutOfMemory;
+  return 0;
 }
 
 // benchmark hook: average duration (ms) of the sigma kernels over `reps`

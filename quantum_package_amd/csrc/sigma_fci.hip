@@ -881,8 +881,7 @@ bool sigma_fci(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, h
     if (prec == QPX_FP64) build_tables<double>(c);
     else build_tables<float>(c);
     ws = prec == QPX_FP64 ? scratch_for<double>(c, nst, st) : scratch_for<float>(c, nst, st);
-  } catch (const Error &) {
-    (void)hipGetLastError();
+  } catch (const OutOfMemory &) {
     c->W.fci.clear();
     return false;
   }

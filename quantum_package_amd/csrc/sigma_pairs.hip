@@ -1038,8 +1038,7 @@ bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s,
       }
     }
     if (ok) ws = c->ws_pairs.get((f64 ? 8 : 4) * (size_t)nst * std::max<int64_t>(W.pr.n_all, 1), st);
-  } catch (const Error &) {
-    (void)hipGetLastError();
+  } catch (const OutOfMemory &) {
     ok = false;
   }
   if (!ok) {

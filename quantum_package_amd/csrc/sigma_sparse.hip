@@ -512,7 +512,11 @@ bool sparse_ok(qpx_ctx *c, int nst) {
 void sigma_sparse(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, hipStream_t st) {
   // by bucket where that fits and pays (2.3 against 7.6 ms for 262,144
   // determinants of 96 orbitals, FP64, 4 states)
-  if (c->force_path != 5 && sigma_pairs(c, prec, nst, u, v, s, st)) return;
+  if (c->force_path != 5 && sigma_pairs(c, prec, nst, u, v, s, st)) {
+    c->sigma_kernels = 3;
+    return;
+  }
+  c->sigma_kernels = 5;
   Wfn &W = c->W;
   ensure_g4(c);   // partners in a bucket then read neighbouring integrals
   if (!W.sp.valid) {

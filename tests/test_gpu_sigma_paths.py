@@ -1,0 +1,82 @@
+"""Which kernels a sigma call runs, and what becomes of errors on the way."""
+from __future__ import annotations
+
+import contextlib
+
+import numpy as np
+import pytest
+
+from quantum_package_amd.hamiltonian import fci_space, synthetic_hamiltonian
+from test_gpu_sigma import BUCKETS, PRODUCT, _product_space, _say, _singles_space
+
+pytestmark = pytest.mark.gpu
+
+STRINGS, SCAN, BUCKET, DENSE, WALK = 1, 2, 3, 4, 5
+LAUNCH_FAILURE = 719   # a hipError_t that is not about memory
+
+
+@pytest.fixture()
+def ctx():
+    from quantum_package_amd.api import Context
+    c = Context(0)
+    yield c
+    c.close()
+
+
+@contextlib.contextmanager
+def failing_allocations(ctx, above, error=0):
+    ctx.L.qpx_debug_fail_alloc(above, error)
+    try:
+        yield
+    finally:
+        ctx.L.qpx_debug_fail_alloc(-1, 0)
+
+
+def _set(ctx, M, na, nb, dets):
+    ctx.set_hamiltonian(synthetic_hamiltonian(M, na, nb, seed=4))
+    ctx.set_wavefunction(dets)
+    return np.random.default_rng(1).standard_normal((dets.shape[0], 2))
+
+
+# of PRODUCT, the space with 26 orbitals is the dense map's: the integrals of
+# 88 singles do not fit the string-driven kernel's LDS
+@pytest.mark.parametrize("kind,M,na,nb,arg", [("product", *p) for p in PRODUCT if p[0] < 26] +
+                         [("buckets", *p) for p in BUCKETS])
+def test_forced_kernels_run(ctx, kind, M, na, nb, arg):
+    """The spaces the kernels of sigma_fci.hip and sigma_pairs.hip are checked
+    on are computed by them, in both precisions."""
+    dets = _product_space(M, na, nb, arg, 7) if kind == "product" else _singles_space(M, na, nb, arg, M + 1)
+    u = _set(ctx, M, na, nb, dets)
+    _say(f"[sigma kernels] {kind} M={M} {na}a{nb}b n_det={dets.shape[0]}")
+    for path, kernels in ((1, STRINGS),) if kind == "product" else ((3, BUCKET), (5, WALK)):
+        ctx._force_sigma_path(path)
+        for prec in (0, 1):
+            ctx.H_S2_u_0_nstates(u, prec=prec)
+            assert ctx._sigma_kernels() == kernels
+
+
+def test_kernels_by_path(ctx):
+    dets = fci_space(8, 4, 4)
+    u = _set(ctx, 8, 4, 4, dets)
+    for path, kernels in ((0, STRINGS), (1, STRINGS), (2, SCAN), (3, BUCKET), (4, DENSE), (5, WALK)):
+        ctx._force_sigma_path(path)
+        ctx.H_S2_u_0_nstates(u)
+        assert ctx._sigma_kernels() == kernels
+
+
+@pytest.mark.parametrize("path", [1, 3])
+def test_errors_reach_the_caller(ctx, path):
+    """Only the want of memory sends a call to another path; any other error
+    of the set-up is the call's, and the next call is as if it had not been."""
+    from quantum_package_amd.api import QpxError
+    M, na, nb = (10, 4, 3) if path == 1 else (20, 3, 2)
+    dets = fci_space(M, na, nb) if path == 1 else _singles_space(M, na, nb, 0.9, 1)
+    u = _set(ctx, M, na, nb, dets)
+    ctx._force_sigma_path(path)
+    ctx.H_S2_u_0_nstates(u)
+    _say(f"[sigma errors] path={path} n_det={dets.shape[0]}")
+    with failing_allocations(ctx, 0, LAUNCH_FAILURE):
+        with pytest.raises(QpxError):
+            ctx.H_S2_u_0_nstates(u, prec=1)
+    ctx.H_S2_u_0_nstates(u, prec=1)
+    assert ctx._sigma_kernels() == path
