@@ -227,10 +227,7 @@ extern "C" int qpx_set_hamiltonian(qpx_ctx *c, int M, int na, int nb, const doub
     QPX_HIP(hipStreamSynchronize(c->stream));
     H.G4.release();   // rebuilt for the new integrals on the next sparse call
     H.G4f.release();
-    H.Pt.release();
-    H.Pf.release();
-    H.Ptf.release();
-    H.Pff.release();
+    H.release_pair_tables();
     c->ham_set = true;
     c->W.valid = false;
   });

@@ -108,6 +108,12 @@ struct Ham {
   // precision on first use (sigma_pairs.hip)
   DBuf<double> Pt, Pf;
   DBuf<float> Ptf, Pff;
+  void release_pair_tables() {
+    Pt.release();
+    Pf.release();
+    Ptf.release();
+    Pff.release();
+  }
   double ref_energy = 0.0;        // ref_bitmask_energy of the HF determinant
 };
 

@@ -726,20 +726,22 @@ void build_tables(qpx_ctx *c) {
   if (t.valid) return;
   hipStream_t s = c->stream;
   const int M = c->H.M, npo = M * (M - 1) / 2, nr = npo + M, mt = (nr + 15) / 16;
+  // memory first: a set of tables that does not fit is tried again by every call
+  t.coef_a.alloc(std::max<size_t>((size_t)128 * P.a.nchunk, 1));
+  t.coef_b.alloc(std::max<size_t>((size_t)128 * P.b.nchunk, 1));
+  t.tgt.alloc((size_t)mt * P.ldt * 4);
+  t.gb.alloc((size_t)npo * W.n_b);
+  t.vo.alloc((size_t)npo * nr);
   auto coefs = [&](const SpinConn &cc, int n, const SpinTiles &tl, DBuf<T> &out) {
-    out.alloc(std::max<size_t>((size_t)128 * tl.nchunk, 1));
     hipLaunchKernelGGL(fci_coef_kernel<T>, dim3(tl.ntile), dim3(256), 0, s, cc.s_ptr.p, cc.s_idx.p, Prec<T>::sval(cc),
                        cc.d_ptr.p, cc.d_idx.p, Prec<T>::dval(cc), n, tl.ptr.p, tl.idx.p, out.p);
     QPX_HIP(hipGetLastError());
   };
   coefs(W.ca, W.n_a, P.a, t.coef_a);
   coefs(W.cb, W.n_b, P.b, t.coef_b);
-  t.tgt.alloc((size_t)mt * P.ldt * 4);
   hipLaunchKernelGGL(fci_target_kernel<T>, dim3(1024), dim3(256), 0, s, P.map_a.p, W.astr.p, W.n_a, P.ldt, M, npo, mt, t.tgt.p);
-  t.gb.alloc((size_t)npo * W.n_b);
   hipLaunchKernelGGL(fci_coulomb_kernel<T>, dim3(1024), dim3(256), 0, s, W.bstr.p, Prec<T>::V(c->H), c->H.npair,
                      P.vrow.p, W.n_b, npo, t.gb.p);
-  t.vo.alloc((size_t)npo * nr);
   hipLaunchKernelGGL(fci_pairs_kernel<T>, dim3(256), dim3(256), 0, s, Prec<T>::V(c->H), c->H.npair, P.vrow.p, npo, nr,
                      t.vo.p);
   QPX_HIP(hipGetLastError());
@@ -872,9 +874,19 @@ bool fci_ok(qpx_ctx *c, int nst, size_t ts) {
 }
 
 // False when the tables or the scratch do not fit the device's memory: the
-// caller then takes a path that needs none.
+// caller then takes a path that needs none.  What the call began goes again;
+// what was there before it stays, for the calls and captured graphs that use it.
 bool sigma_fci(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, hipStream_t st) {
   ensure_conn(c);
+  FciPlan &P = c->W.fci;
+  const bool had_plan = P.valid, had_tables = prec == QPX_FP64 ? P.t64.valid : P.t32.valid;
+  auto drop = [&] {
+    if (!had_tables) {
+      if (prec == QPX_FP64) P.t64.clear();
+      else P.t32.clear();
+    }
+    if (!had_plan) P.clear();
+  };
   char *ws = nullptr;
   try {
     build_plan(c);
@@ -882,8 +894,11 @@ bool sigma_fci(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, h
     else build_tables<float>(c);
     ws = prec == QPX_FP64 ? scratch_for<double>(c, nst, st) : scratch_for<float>(c, nst, st);
   } catch (const OutOfMemory &) {
-    c->W.fci.clear();
+    drop();
     return false;
+  } catch (...) {
+    drop();
+    throw;
   }
   if (prec == QPX_FP64)
     run<double>(c, ab_shape(c, nst, 8, c->W.cb.max_singles), ws, nst, (const double *)u, (double *)v, (double *)s, st);

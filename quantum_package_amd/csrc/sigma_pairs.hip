@@ -954,9 +954,9 @@ void build_table(qpx_ctx *c, DBuf<T> &tab, DBuf<T> &fock) {
   const int M = H.M, npo = M * (M - 1) / 2;
   const int64_t n = (int64_t)M * M * M * M + (int64_t)npo * npo;
   fock.alloc((size_t)2 * M * M);
+  tab.alloc(n);
   hipLaunchKernelGGL(fock_table_kernel<T>, dim3(64), dim3(256), 0, c->stream, H.hcore.p, H.GS.p, H.GO.p, M, H.na, H.nb,
                      fock.p);
-  tab.alloc(n);
   hipLaunchKernelGGL(pair_table_kernel<T>, dim3(grid_for(n)), dim3(256), 0, c->stream, H.V.p, M, H.npair, npo, tab.p);
   QPX_HIP(hipGetLastError());
   QPX_HIP(hipStreamSynchronize(c->stream));
@@ -1014,6 +1014,10 @@ namespace qpx {
 
 // False when the entries, their sums or the integral table do not fit: the
 // caller then walks the buckets determinant by determinant (sigma_sparse.hip).
+// What the call began goes again; what was there before it stays, for the calls
+// and captured graphs that use it.  Entries that do not fit are not tried again
+// for this wavefunction; a table or sums (of a precision, of a number of
+// states) are, which costs an allocation.
 bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, hipStream_t st) {
   Wfn &W = c->W;
   Ham &H = c->H;
@@ -1024,28 +1028,46 @@ bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s,
   if (H.M > kG4MaxOrb || nst > kMaxState || H.na > kMaxElec || H.nb > kMaxElec || H.na < 1 || H.nb < 1) return false;
   if (W.pr.failed) return false;
   const bool f64 = prec == QPX_FP64;
+  const bool had_entries = W.pr.valid, had_table = f64 ? H.Pt.p != nullptr : H.Ptf.p != nullptr;
+  auto drop = [&] {
+    if (!had_entries) {
+      W.pr.release();
+      c->ws_pairs.release();
+    }
+    if (had_table) return;
+    if (f64) {
+      H.Pt.release();
+      H.Pf.release();
+    } else {
+      H.Ptf.release();
+      H.Pff.release();
+    }
+  };
   char *ws = nullptr;
-  bool ok = false;
+  bool ok = false, entries = had_entries, failed = false;   // failed: the entries do not fit
   try {
     if (f64) build_table<double>(c, H.Pt, H.Pf);
     else build_table<float>(c, H.Ptf, H.Pff);
-    ok = W.pr.valid;
-    if (!ok) {
+    if (!entries) {
+      failed = true;
       switch (W.nint) {
-        case 1: ok = build<1>(c); break;
-        case 2: ok = build<2>(c); break;
-        default: ok = build<3>(c); break;
+        case 1: entries = build<1>(c); break;
+        case 2: entries = build<2>(c); break;
+        default: entries = build<3>(c); break;
       }
+      failed = !entries;
     }
+    ok = entries;
     if (ok) ws = c->ws_pairs.get((f64 ? 8 : 4) * (size_t)nst * std::max<int64_t>(W.pr.n_all, 1), st);
   } catch (const OutOfMemory &) {
     ok = false;
+  } catch (...) {
+    drop();
+    throw;
   }
   if (!ok) {
-    W.pr.release();
-    if (f64) H.Pt.release();
-    else H.Ptf.release();
-    W.pr.failed = !StreamWorkspace::capturing(st);
+    drop();
+    W.pr.failed = failed && !StreamWorkspace::capturing(st);
     return false;
   }
   if (c->ktiming) QPX_HIP(hipEventRecord(c->kev[0], st));

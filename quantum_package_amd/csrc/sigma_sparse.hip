@@ -518,14 +518,27 @@ void sigma_sparse(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s
   }
   c->sigma_kernels = 5;
   Wfn &W = c->W;
-  ensure_g4(c);   // partners in a bucket then read neighbouring integrals
-  if (!W.sp.valid) {
+  auto set_up = [&] {
+    ensure_g4(c);   // partners in a bucket then read neighbouring integrals
+    if (W.sp.valid) return;
     switch (W.nint) {
       case 1: build_buckets<1>(c); break;
       case 2: build_buckets<2>(c); break;
       case 3: build_buckets<3>(c); break;
       default: build_buckets<4>(c); break;
     }
+  };
+  try {
+    set_up();
+  } catch (const OutOfMemory &) {
+    if (!W.sp.valid) W.sp.clear();
+    // what calls of another precision or number of vectors hold is given up,
+    // unless a captured graph may still use it
+    if (!W.pr.valid || !c->ws_pairs.graphs.empty()) throw;
+    W.pr.release();
+    c->ws_pairs.release();
+    c->H.release_pair_tables();
+    set_up();
   }
   if (prec == QPX_FP64) {
     switch (W.nint) {

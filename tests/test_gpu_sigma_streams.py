@@ -7,7 +7,8 @@ import pytest
 
 from quantum_package_amd.hamiltonian import fci_space, synthetic_hamiltonian
 from hip_rt import Arr, Hip
-from test_gpu_sigma import _random_space, _say, _singles_space
+from test_gpu_sigma import _say, _singles_space
+from test_gpu_sigma_paths import failing_allocations
 
 pytestmark = pytest.mark.gpu
 
@@ -61,6 +62,13 @@ def _same(x, y):
     return all(np.array_equal(a, b) for a, b in zip(x, y))
 
 
+def _prepare(ctx, kind):
+    M, na, nb, dets = _space(kind)
+    ctx.set_hamiltonian(synthetic_hamiltonian(M, na, nb, seed=4))
+    ctx.set_wavefunction(dets)
+    return dets.shape[0]
+
+
 @pytest.mark.parametrize("what", ["wavefunction", "hamiltonian"])
 @pytest.mark.parametrize("path", [1, 3, 4, 5])
 def test_new_inputs_wait_for_queued_calls(ctx, hip, path, what):
@@ -93,4 +101,92 @@ def test_new_inputs_wait_for_queued_calls(ctx, hip, path, what):
             ctx.set_hamiltonian(synthetic_hamiltonian(M, na, nb, seed=5))
         hip.sync()
         assert _same(x.out(), alone)
+    x.free()
+
+
+@pytest.mark.parametrize("kind,kernels", [("product", 1), ("selected", 3)])
+def test_failed_calls_leave_the_others_alone(ctx, hip, kind, kernels):
+    """Calls that find no memory for the tables of another precision, or for
+    the scratch of more vectors, fail or take another path; a graph captured
+    before and the eager calls give the same bits as before, from the same
+    kernels, and the calls that failed work once there is memory."""
+    from quantum_package_amd.api import QpxError
+    n = _prepare(ctx, kind)
+    _say(f"[sigma failing] {kind} n_det={n}")
+    ctx._force_sigma_path(kernels)
+    st = hip.stream()
+    x, single, more = Vectors(hip, n, 1, 0, 1), Vectors(hip, n, 1, 1, 2), Vectors(hip, n, 4, 0, 3)
+    x.sigma(ctx, st)
+    hip.sync()
+    want = x.out()
+    g = hip.capture(st, lambda: x.sigma(ctx, st))
+    for call in (single, more):
+        with failing_allocations(ctx, 1000):
+            try:
+                call.sigma(ctx, st)
+                assert ctx._sigma_kernels() != kernels
+            except QpxError as e:
+                assert "memory" in str(e)
+        hip.sync()
+        x.clear()
+        hip.replay(g, st)
+        hip.sync()
+        assert _same(x.out(), want)
+        x.clear()
+        x.sigma(ctx, st)
+        hip.sync()
+        assert ctx._sigma_kernels() == kernels and _same(x.out(), want)
+    for call in (single, more):
+        call.sigma(ctx, st)
+        assert ctx._sigma_kernels() == kernels
+    hip.sync()
+    x.clear()
+    hip.replay(g, st)
+    hip.sync()
+    assert _same(x.out(), want)
+    hip.drop(g)
+    for v in (x, single, more):
+        v.free()
+
+
+@pytest.mark.parametrize("what", ["sums", "entries"])
+def test_bucket_calls_without_memory_walk(ctx, hip, what):
+    """Sums that do not fit send that call alone to the walk; entries that do
+    not fit send the wavefunction's calls there.  FP64 against the walk."""
+    n = _prepare(ctx, "selected")
+    _say(f"[sigma walk] {what} n_det={n}")
+    x, st = Vectors(hip, n, 4, 0, 2), hip.stream()
+
+    def run(path):
+        x.clear()
+        ctx._force_sigma_path(path)
+        x.sigma(ctx, st)
+        hip.sync()
+        return x.out()
+
+    def close(out):
+        return all(np.max(np.abs(a - b)) < 1e-11 * np.max(np.abs(b)) for a, b in zip(out, want))
+
+    dets = _space("selected")[3]
+    ctx._force_sigma_path(3)
+    ctx.set_wavefunction(dets[:50])   # leaves the integral tables, not the room for more entries
+    ctx.H_S2_u_0_nstates(np.ones(50))
+    ctx.set_wavefunction(dets)
+    want = run(5)
+    if what == "sums":
+        assert close(run(3)) and ctx._sigma_kernels() == 3
+        with failing_allocations(ctx, 1000):   # a captured call's sums are memory of its own
+            g = hip.capture(st, lambda: x.sigma(ctx, st))
+            assert ctx._sigma_kernels() == 5
+        x.clear()
+        hip.replay(g, st)
+        hip.sync()
+        assert _same(x.out(), want)
+        hip.drop(g)
+    else:
+        with failing_allocations(ctx, 1 << 16):
+            assert close(run(3)) and ctx._sigma_kernels() == 5
+        assert close(run(3)) and ctx._sigma_kernels() == 5
+        ctx.set_wavefunction(dets)
+    assert close(run(3)) and ctx._sigma_kernels() == 3
     x.free()
