@@ -234,6 +234,33 @@ struct Workspace {
   }
 };
 
+inline bool capturing(hipStream_t s, unsigned long long *id = nullptr) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  unsigned long long x = 0;
+  if (hipStreamGetCaptureInfo(s, &cs, &x) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  if (id) *id = x;
+  return cs != hipStreamCaptureStatusNone;
+}
+
+// While s is captured, lets this thread allocate and wait on other streams:
+// tables and scratch that a captured call is the first to need are made beside
+// the graph.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  bool on;
+  explicit RelaxedCapture(hipStream_t s) : on(capturing(s)) {
+    if (on) QPX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  }
+  ~RelaxedCapture() {
+    if (on) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+  RelaxedCapture(const RelaxedCapture &) = delete;
+  RelaxedCapture &operator=(const RelaxedCapture &) = delete;
+};
+
 // Scratch of calls that are enqueued on a caller's stream and return before
 // they have run: a call on another stream first waits for the last user.
 struct StreamWorkspace {
@@ -253,16 +280,6 @@ struct StreamWorkspace {
     DBuf<char> buf;
   };
   std::vector<std::unique_ptr<Captured>> graphs;
-  static bool capturing(hipStream_t s, unsigned long long *id = nullptr) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    unsigned long long x = 0;
-    if (hipStreamGetCaptureInfo(s, &cs, &x) != hipSuccess) {
-      (void)hipGetLastError();
-      return false;
-    }
-    if (id) *id = x;
-    return cs != hipStreamCaptureStatusNone;
-  }
   char *get(size_t bytes, hipStream_t s) {
     unsigned long long id = 0;
     if (capturing(s, &id)) {
@@ -271,15 +288,7 @@ struct StreamWorkspace {
       auto g = std::make_unique<Captured>();
       g->s = s;
       g->id = id;
-      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // lets this thread allocate
-      QPX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
-      try {
-        g->buf.alloc(bytes);
-      } catch (...) {
-        (void)hipThreadExchangeStreamCaptureMode(&mode);
-        throw;
-      }
-      QPX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+      g->buf.alloc(bytes);
       graphs.push_back(std::move(g));
       return graphs.back()->buf.p;
     }

@@ -697,7 +697,7 @@ static bool dense_ok(qpx_ctx *c, int nst, size_t tsize) {
 
 // gives back what the sparse path keeps for later wavefunctions once one takes another path
 static void release_pairs(qpx_ctx *c, hipStream_t st) {
-  if (c->W.pr.valid || !c->W.pr.ent.p || StreamWorkspace::capturing(st)) return;
+  if (c->W.pr.valid || !c->W.pr.ent.p || capturing(st)) return;
   c->W.pr.release();
   c->ws_pairs.release();
 }
@@ -707,6 +707,7 @@ void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s
   QPX_REQUIRE(nst >= 1 && nst <= GMAXST, "n_st must be in 1..8");
   QPX_REQUIRE(prec == QPX_FP64 || prec == QPX_FP32, "prec must be QPX_FP64 or QPX_FP32");
   size_t ts = prec == QPX_FP64 ? sizeof(double) : sizeof(float);
+  RelaxedCapture relaxed(st);
   // a product space takes the string-driven path (12.2 against 32.8 ms for
   // 9.0M determinants, FP64, 4 states; 35 against 86 us for 4900)
   if ((c->force_path == 0 || c->force_path == 1) && fci_ok(c, nst, ts) &&

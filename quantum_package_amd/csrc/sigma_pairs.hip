@@ -1067,7 +1067,7 @@ bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s,
   }
   if (!ok) {
     drop();
-    W.pr.failed = failed && !StreamWorkspace::capturing(st);
+    W.pr.failed = failed;
     return false;
   }
   if (c->ktiming) QPX_HIP(hipEventRecord(c->kev[0], st));

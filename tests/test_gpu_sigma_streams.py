@@ -190,3 +190,40 @@ def test_bucket_calls_without_memory_walk(ctx, hip, what):
         ctx.set_wavefunction(dets)
     assert close(run(3)) and ctx._sigma_kernels() == 3
     x.free()
+
+
+@pytest.mark.parametrize("first", ["precision", "call"])
+@pytest.mark.parametrize("kind,path", [("product", 1), ("product", 4), ("selected", 3), ("selected", 5)])
+def test_captured_call_builds_its_tables(ctx, hip, kind, path, first):
+    """A captured call may be the first of its precision, or of the
+    wavefunction: replays give the bits of an eager call, which runs the same
+    kernels."""
+    n = _prepare(ctx, kind)
+    _say(f"[sigma captured] {kind} path={path} first {first} n_det={n}")
+    ctx._force_sigma_path(path)
+    st = hip.stream()
+    x, y = Vectors(hip, n, 2, 1, 1), Vectors(hip, n, 1, 0, 2)
+    if first == "precision":
+        y.sigma(ctx, st)
+        hip.sync()
+        before = y.out()
+    g = hip.capture(st, lambda: x.sigma(ctx, st))
+    assert ctx._sigma_kernels() == path
+    x.clear()
+    hip.replay(g, st)
+    hip.sync()
+    got = x.out()
+    x.sigma(ctx, st)
+    hip.sync()
+    assert ctx._sigma_kernels() == path and _same(x.out(), got)
+    for _ in range(3):
+        y.sigma(ctx, st)
+        x.clear()
+        hip.replay(g, st)
+        hip.sync()
+        assert _same(x.out(), got)
+    if first == "precision":
+        assert _same(y.out(), before)
+    hip.drop(g)
+    x.free()
+    y.free()
