@@ -104,15 +104,14 @@ struct Ham {
   // the sparse sigma path when M <= kG4MaxOrb (ensure_g4)
   DBuf<double> G4;
   DBuf<float> G4f;
-  // integrals and HF elements of the bucket-by-bucket sparse sigma, per
-  // precision on first use (sigma_pairs.hip)
+  // integrals (per precision, on first use) and HF elements of the
+  // bucket-by-bucket sparse sigma (sigma_pairs.hip)
   DBuf<double> Pt, Pf;
-  DBuf<float> Ptf, Pff;
+  DBuf<float> Ptf;
   void release_pair_tables() {
     Pt.release();
     Pf.release();
     Ptf.release();
-    Pff.release();
   }
   double ref_energy = 0.0;        // ref_bitmask_energy of the HF determinant
 };

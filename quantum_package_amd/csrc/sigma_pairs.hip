@@ -470,9 +470,9 @@ __global__ void pair_table_kernel(const double *__restrict__ V, int M, int npair
 }
 // single excitation i -> x from the HF occupation: h + sum over HF's orbitals,
 // [spin][x M + i]
-template <typename T>
 __global__ void fock_table_kernel(const double *__restrict__ hcore, const double *__restrict__ GS,
-                                  const double *__restrict__ GO, int M, int na, int nb, T *__restrict__ f) {
+                                  const double *__restrict__ GO, int M, int na, int nb,
+                                  double *__restrict__ f) {
   for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < 2 * M * M; q += gridDim.x * blockDim.x) {
     const int sp = q / (M * M), r = q - sp * M * M, x = r / M, i = r - x * M;
     const int ns = sp ? nb : na, no = sp ? na : nb;
@@ -480,7 +480,7 @@ __global__ void fock_table_kernel(const double *__restrict__ hcore, const double
     double v = hcore[i * M + x];
     for (int k = 0; k < ns; ++k) v += GS[row + k];
     for (int k = 0; k < no; ++k) v += GO[row + k];
-    f[q] = (T)v;
+    f[q] = v;
   }
 }
 
@@ -491,11 +491,15 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// Sums and the rows of u in LDS are FP64 in both precisions: a chain over a
+// bucket that holds one large coefficient (HF's) rounds every later term
+// against it.
+
 // adds members [c, end) of one bucket, 64 at a time: their rows of u, with the
 // members' signs, go to LDS (ru, this wavefront's)
 template <typename T, int NST>
-__device__ __forceinline__ void add_members(const uint2 *ent, int c, int end, const T *row, const T *u, T *ru,
-                                            T (&acc)[NST]) {
+__device__ __forceinline__ void add_members(const uint2 *ent, int c, int end, const T *row, const T *u,
+                                            double *ru, double (&acc)[NST]) {
   constexpr int B = 16;   // integrals in flight
   const int lane = threadIdx.x & 63;
   for (; c < end; c += 64) {
@@ -503,8 +507,8 @@ __device__ __forceinline__ void add_members(const uint2 *ent, int c, int end, co
     const uint2 e = ent[c + min(lane, n - 1)];
     const T *src = u + (int64_t)(e.x & ~kSign) * NST;
 #pragma unroll
-    for (int st = 0; st < NST; ++st) ru[lane * NST + st] = lane < n ? flip(src[st], e.x & kSign) : T(0);
-      wave_fence();
+    for (int st = 0; st < NST; ++st) ru[lane * NST + st] = lane < n ? (double)flip(src[st], e.x & kSign) : 0.0;
+    wave_fence();
     for (int r = 0; r < n; r += B) {
       T g[B];
 #pragma unroll
@@ -512,9 +516,9 @@ __device__ __forceinline__ void add_members(const uint2 *ent, int c, int end, co
 #pragma unroll
       for (int i = 0; i < B; ++i)
 #pragma unroll
-        for (int st = 0; st < NST; ++st) acc[st] += g[i] * ru[(r + i) * NST + st];
+        for (int st = 0; st < NST; ++st) acc[st] += (double)g[i] * ru[(r + i) * NST + st];
     }
-      wave_fence();
+    wave_fence();
   }
 }
 
@@ -524,7 +528,7 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
                                                            const int2 *__restrict__ wave, int nbig, int nwave,
                                                            const T *__restrict__ tab, const T *__restrict__ u,
                                                            T *__restrict__ part) {
-  __shared__ T row_u[256 * NST];
+  __shared__ double row_u[256 * NST];
   // 16 workgroups in a row to an XCD: they share a bucket's members and rows of the
   // table in its L2 (1.62 -> 1.59 ms above; 2.1M determinants, the call 113 -> 107 ms)
   int blk = (int)blockIdx.x;
@@ -532,10 +536,10 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
   __shared__ uint32_t row_base[256];
   const int lane = threadIdx.x & 63;
   const int sub = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  T *ru = row_u + sub * 64 * NST;
-  T acc[NST];
+  double *ru = row_u + sub * 64 * NST;
+  double acc[NST];
 #pragma unroll
-  for (int st = 0; st < NST; ++st) acc[st] = T(0);
+  for (int st = 0; st < NST; ++st) acc[st] = 0.0;
   if (blk < nbig) {
     // 64 entries of a bucket of kSplit and more: a quarter of the members each
     const int64_t p = (int64_t)blk * 64 + lane;
@@ -551,7 +555,7 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
     for (int st = 0; st < NST; ++st) {
 #pragma unroll
       for (int q = 1; q < 4; ++q) acc[st] += row_u[q * 64 * NST + st * 64 + lane];
-      part[p * NST + st] = flip(acc[st], own & kSign);
+      part[p * NST + st] = (T)flip(acc[st], own & kSign);
     }
     return;
   }
@@ -566,7 +570,7 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
     add_members<T, NST>(ent, d.x, d.x + d.y, row, u, ru, acc);
     if (p >= d.x + d.y) return;
 #pragma unroll
-    for (int st = 0; st < NST; ++st) part[p * NST + st] = flip(acc[st], own.x & kSign);
+    for (int st = 0; st < NST; ++st) part[p * NST + st] = (T)flip(acc[st], own.x & kSign);
     return;
   }
   // buckets of one size: their rows of u, with the members' signs, and table
@@ -592,7 +596,7 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
   };
   load(1);   // beside the rows of u
 #pragma unroll
-  for (int st = 0; st < NST; ++st) ru[lane * NST + st] = flip(x[st], own.x & kSign);
+  for (int st = 0; st < NST; ++st) ru[lane * NST + st] = (double)flip(x[st], own.x & kSign);
   wave_fence();
   for (int r0 = 1;;) {
 #pragma unroll
@@ -602,9 +606,9 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
       const int up = !on ? lane : m + r < z ? lane + r : lane + r - z;
       const int dn = !on ? lane : m >= r ? lane - r : lane - r + z;
 #pragma unroll
-      for (int st = 0; st < NST; ++st) acc[st] += g[i] * ru[up * NST + st];
+      for (int st = 0; st < NST; ++st) acc[st] += (double)g[i] * ru[up * NST + st];
       if (2 * r < z) {
-        const T h = __shfl(g[i], dn);
+        const double h = (double)__shfl(g[i], dn);
 #pragma unroll
         for (int st = 0; st < NST; ++st) acc[st] += h * ru[dn * NST + st];
       }
@@ -615,7 +619,7 @@ __global__ __launch_bounds__(256) void pair_doubles_kernel(const uint2 *__restri
   }
   if (!on) return;
 #pragma unroll
-  for (int st = 0; st < NST; ++st) part[p * NST + st] = flip(acc[st], own.x & kSign);
+  for (int st = 0; st < NST; ++st) part[p * NST + st] = (T)flip(acc[st], own.x & kSign);
 }
 
 struct SingleArgs {
@@ -626,11 +630,12 @@ struct SingleArgs {
 };
 
 // sums of the single excitations: HF's element plus the change of the
-// occupations (a few orbitals) instead of a sum over all electrons
+// occupations (a few orbitals) instead of a sum over all electrons; elements in
+// FP64 in both precisions, what HF's occupation adds being taken off again
 template <typename T, int NI, int NST>
 __global__ __launch_bounds__(256) void pair_singles_kernel(SingleArgs A, int64_t first, const uint2 *__restrict__ ent,
                                                            const uint32_t *__restrict__ off,
-                                                           const int2 *__restrict__ wave, const T *__restrict__ fock,
+                                                           const int2 *__restrict__ wave, const double *__restrict__ fock,
                                                            const T *__restrict__ GS, const T *__restrict__ GO,
                                                            const T *__restrict__ u, T *__restrict__ part) {
   const int64_t p = first + blockIdx.x * (int64_t)256 + threadIdx.x;
@@ -654,13 +659,13 @@ __global__ __launch_bounds__(256) void pair_singles_kernel(SingleArgs A, int64_t
     same[w] = (w == (i >> 6) ? x & ~(1ULL << (i & 63)) : x) ^ hs[w];
     other[w] = y ^ ho[w];
   }
-  T acc[NST];
+  double acc[NST];
 #pragma unroll
-  for (int st = 0; st < NST; ++st) acc[st] = T(0);
-  const T *f = fock + (beta ? M * M : 0) + i;
+  for (int st = 0; st < NST; ++st) acc[st] = 0.0;
+  const double *f = fock + (beta ? M * M : 0) + i;
   for (int k = b0; k < b1; k += 4) {
     uint2 e[4];
-    T h[4];
+    double h[4];
     const T *gs[4], *go[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -676,7 +681,7 @@ __global__ __launch_bounds__(256) void pair_singles_kernel(SingleArgs A, int64_t
         const int o = __ffsll((unsigned long long)y) - 1;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const T g = gs[q][64 * w + o];
+          const double g = (double)gs[q][64 * w + o];
           h[q] += (hs[w] >> o) & 1 ? -g : g;
         }
       }
@@ -684,7 +689,7 @@ __global__ __launch_bounds__(256) void pair_singles_kernel(SingleArgs A, int64_t
         const int o = __ffsll((unsigned long long)y) - 1;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const T g = go[q][64 * w + o];
+          const double g = (double)go[q][64 * w + o];
           h[q] += (ho[w] >> o) & 1 ? -g : g;
         }
       }
@@ -692,18 +697,20 @@ __global__ __launch_bounds__(256) void pair_singles_kernel(SingleArgs A, int64_t
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       if (k + q >= b1 || (int)e[q].y == i) continue;
-      const T t = flip(h[q], e[q].x & kSign);
+      const double t = flip(h[q], e[q].x & kSign);
       const T *src = u + (int64_t)(e[q].x & ~kSign) * NST;
 #pragma unroll
-      for (int st = 0; st < NST; ++st) acc[st] += t * src[st];
+      for (int st = 0; st < NST; ++st) acc[st] += t * (double)src[st];
     }
   }
 #pragma unroll
-  for (int st = 0; st < NST; ++st) part[p * NST + st] = flip(acc[st], own & kSign);
+  for (int st = 0; st < NST; ++st) part[p * NST + st] = (T)flip(acc[st], own & kSign);
 }
 
 // v and s of a determinant: 16 lanes add its entries' sums, slots l, l + 16,
-// ..., then a fixed tree
+// ..., then a fixed tree.  In FP64 in both precisions: an FP32 call's error
+// would otherwise be that of hundreds of sums and of the list of spin exchanges
+// added one by one.
 template <typename T, int NST>
 __global__ __launch_bounds__(256) void pair_collect_kernel(const int *__restrict__ slotpos, int S, int64_t n,
                                                            const T *__restrict__ part, const int *__restrict__ xptr,
@@ -714,9 +721,9 @@ __global__ __launch_bounds__(256) void pair_collect_kernel(const int *__restrict
   const int64_t k = blockIdx.x * (int64_t)16 + (threadIdx.x >> 4);
   const int l = threadIdx.x & 15;
   const bool on = k < n;
-  T acc[NST];
+  double acc[NST];
 #pragma unroll
-  for (int st = 0; st < NST; ++st) acc[st] = T(0);
+  for (int st = 0; st < NST; ++st) acc[st] = 0.0;
   if (on) {
     const int *sp = slotpos + k * S;
     for (int t = l; t < S; t += 64) {
@@ -727,7 +734,7 @@ __global__ __launch_bounds__(256) void pair_collect_kernel(const int *__restrict
       for (int q = 0; q < 4; ++q)
         if (at[q] >= 0)
 #pragma unroll
-          for (int st = 0; st < NST; ++st) acc[st] += part[(int64_t)at[q] * NST + st];
+          for (int st = 0; st < NST; ++st) acc[st] += (double)part[(int64_t)at[q] * NST + st];
     }
   }
 #pragma unroll
@@ -738,15 +745,15 @@ __global__ __launch_bounds__(256) void pair_collect_kernel(const int *__restrict
   // lane st writes state st of v, lane 8 + st of s
 #pragma unroll
   for (int st = 0; st < NST; ++st) {
-    const T x = u[k * NST + st];
-    if (l == st) v[k * NST + st] = acc[st] + (T)hdiag[k] * x;
+    const double x = (double)u[k * NST + st];
+    if (l == st) v[k * NST + st] = (T)(acc[st] + hdiag[k] * x);
     if (l == 8 + st) {
-      T t = (T)sdiag[k] * x;
+      double t = sdiag[k] * x;
       for (int q = xptr[k]; q < xptr[k + 1]; ++q) {
         const uint32_t e = xlist[q];
-        t += flip(u[(int64_t)(e & ~kSign) * NST + st], e & kSign);
+        t += (double)flip(u[(int64_t)(e & ~kSign) * NST + st], e & kSign);
       }
-      s[k * NST + st] = t;
+      s[k * NST + st] = (T)t;
     }
   }
 }
@@ -948,22 +955,24 @@ bool build(qpx_ctx *c) {
 }
 
 template <typename T>
-void build_table(qpx_ctx *c, DBuf<T> &tab, DBuf<T> &fock) {
+void build_table(qpx_ctx *c, DBuf<T> &tab) {
   Ham &H = c->H;
   if (tab.p) return;
   const int M = H.M, npo = M * (M - 1) / 2;
   const int64_t n = (int64_t)M * M * M * M + (int64_t)npo * npo;
-  fock.alloc((size_t)2 * M * M);
   tab.alloc(n);
-  hipLaunchKernelGGL(fock_table_kernel<T>, dim3(64), dim3(256), 0, c->stream, H.hcore.p, H.GS.p, H.GO.p, M, H.na, H.nb,
-                     fock.p);
+  if (!H.Pf.p) {
+    H.Pf.alloc((size_t)2 * M * M);
+    hipLaunchKernelGGL(fock_table_kernel, dim3(64), dim3(256), 0, c->stream, H.hcore.p, H.GS.p, H.GO.p, M, H.na, H.nb,
+                       H.Pf.p);
+  }
   hipLaunchKernelGGL(pair_table_kernel<T>, dim3(grid_for(n)), dim3(256), 0, c->stream, H.V.p, M, H.npair, npo, tab.p);
   QPX_HIP(hipGetLastError());
   QPX_HIP(hipStreamSynchronize(c->stream));
 }
 
 template <typename T, int NI, int NST>
-void launch(qpx_ctx *c, char *ws, const T *tab, const T *fock, const T *u, T *v, T *s, hipStream_t st) {
+void launch(qpx_ctx *c, char *ws, const T *tab, const double *fock, const T *u, T *v, T *s, hipStream_t st) {
   Wfn &W = c->W;
   PairIdx &X = W.pr;
   const bool f64 = std::is_same<T, double>::value;
@@ -986,7 +995,7 @@ void launch(qpx_ctx *c, char *ws, const T *tab, const T *fock, const T *u, T *v,
 }
 
 template <typename T, int NI>
-void launch_nst(qpx_ctx *c, int nst, char *ws, const T *tab, const T *fock, const T *u, T *v, T *s, hipStream_t st) {
+void launch_nst(qpx_ctx *c, int nst, char *ws, const T *tab, const double *fock, const T *u, T *v, T *s, hipStream_t st) {
   switch (nst) {
     case 1: launch<T, NI, 1>(c, ws, tab, fock, u, v, s, st); break;
     case 2: launch<T, NI, 2>(c, ws, tab, fock, u, v, s, st); break;
@@ -1000,7 +1009,7 @@ void launch_nst(qpx_ctx *c, int nst, char *ws, const T *tab, const T *fock, cons
 }
 
 template <typename T>
-void launch_ni(qpx_ctx *c, int nst, char *ws, const T *tab, const T *fock, const T *u, T *v, T *s, hipStream_t st) {
+void launch_ni(qpx_ctx *c, int nst, char *ws, const T *tab, const double *fock, const T *u, T *v, T *s, hipStream_t st) {
   switch (c->W.nint) {
     case 1: launch_nst<T, 1>(c, nst, ws, tab, fock, u, v, s, st); break;
     case 2: launch_nst<T, 2>(c, nst, ws, tab, fock, u, v, s, st); break;
@@ -1035,19 +1044,14 @@ bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s,
       c->ws_pairs.release();
     }
     if (had_table) return;
-    if (f64) {
-      H.Pt.release();
-      H.Pf.release();
-    } else {
-      H.Ptf.release();
-      H.Pff.release();
-    }
+    if (f64) H.Pt.release();
+    else H.Ptf.release();
   };
   char *ws = nullptr;
   bool ok = false, entries = had_entries, failed = false;   // failed: the entries do not fit
   try {
-    if (f64) build_table<double>(c, H.Pt, H.Pf);
-    else build_table<float>(c, H.Ptf, H.Pff);
+    if (f64) build_table<double>(c, H.Pt);
+    else build_table<float>(c, H.Ptf);
     if (!entries) {
       failed = true;
       switch (W.nint) {
@@ -1074,7 +1078,7 @@ bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s,
   if (f64)
     launch_ni<double>(c, nst, ws, H.Pt.p, H.Pf.p, (const double *)u, (double *)v, (double *)s, st);
   else
-    launch_ni<float>(c, nst, ws, H.Ptf.p, H.Pff.p, (const float *)u, (float *)v, (float *)s, st);
+    launch_ni<float>(c, nst, ws, H.Ptf.p, H.Pf.p, (const float *)u, (float *)v, (float *)s, st);
   if (c->ktiming) {
     QPX_HIP(hipEventRecord(c->kev[1], st));
     QPX_HIP(hipEventRecord(c->kev[2], st));

@@ -6,8 +6,8 @@ import contextlib
 import numpy as np
 import pytest
 
-from quantum_package_amd.hamiltonian import fci_space, synthetic_hamiltonian
-from test_gpu_sigma import BUCKETS, PRODUCT, _product_space, _say, _singles_space
+from quantum_package_amd.hamiltonian import fci_space, hf_determinant, synthetic_hamiltonian
+from test_gpu_sigma import BUCKETS, PRODUCT, _product_space, _random_space, _say, _singles_space
 
 pytestmark = pytest.mark.gpu
 
@@ -80,3 +80,25 @@ def test_errors_reach_the_caller(ctx, path):
             ctx.H_S2_u_0_nstates(u, prec=1)
     ctx.H_S2_u_0_nstates(u, prec=1)
     assert ctx._sigma_kernels() == path
+
+
+@pytest.mark.parametrize("vector", ["noise", "HF and a tail"])
+@pytest.mark.parametrize("M,na,nb,n", [(40, 5, 4, 6000), (96, 6, 6, 6000)])
+def test_bucket_fp32_error(ctx, M, na, nb, n, vector):
+    """An FP32 sigma by bucket is no further from the FP64 one than the walk's,
+    which spreads a determinant's terms over the lanes of a wavefront."""
+    dets = _random_space(M, na, nb, n, M)
+    _set(ctx, M, na, nb, dets)
+    rng = np.random.default_rng(2)
+    u = rng.standard_normal((n, 2)) / np.sqrt(n)
+    if vector != "noise":
+        u *= 0.3
+        u[np.nonzero((dets == hf_determinant(M, na, nb)).all((1, 2)))[0][0]] = 0.95
+    u = u.astype(np.float32).astype(np.float64)
+    _say(f"[sigma fp32 error] M={M} {na}a{nb}b n_det={n} {vector}")
+    ctx._force_sigma_path(3)
+    ref, by_bucket = ctx.H_S2_u_0_nstates(u), ctx.H_S2_u_0_nstates(u, prec=1)
+    ctx._force_sigma_path(5)
+    walk = ctx.H_S2_u_0_nstates(u, prec=1)
+    for x, y, r in zip(by_bucket, walk, ref):
+        assert np.linalg.norm(x - r) <= np.linalg.norm(y - r)
