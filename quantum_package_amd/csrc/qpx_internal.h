@@ -55,6 +55,11 @@ inline void device_alloc(void **p, size_t bytes) {
   QPX_HIP(e);
 }
 
+// What a context keeps of one wavefunction's arrays and scratch for the next, of
+// the bucket kernels and of the string-driven ones; more costs less to allocate
+// again than the set-up it serves (some 10^8 entries to sort).
+constexpr size_t kKeepBytes = (size_t)4 << 30;
+
 // Device buffer with RAII.
 template <typename T>
 struct DBuf {
@@ -195,6 +200,9 @@ struct PairIdx {
   DBuf<int2> wave;            // buckets of a wavefront's 64 entries
   DBuf<int> slotpos, xptr;    // entry of each slot; spin exchanges of each determinant
   void clear() { valid = failed = false; }   // the next wavefunction may take the arrays
+  size_t bytes() const {
+    return ent.n * sizeof(uint2) + wave.n * sizeof(int2) + (off.n + xlist.n + slotpos.n + xptr.n) * sizeof(int);
+  }
   void release() {
     clear();
     ent.release(); off.release(); xlist.release(); wave.release(); slotpos.release(); xptr.release();
@@ -299,6 +307,9 @@ struct StreamWorkspace {
   void release() {
     buf.release();
     pending = false;
+  }
+  void trim(size_t keep) {
+    if (buf.n > keep) release();
   }
   void used(hipStream_t s) {
     if (capturing(s)) return;

@@ -1062,7 +1062,9 @@ bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s,
       failed = !entries;
     }
     ok = entries;
-    if (ok) ws = c->ws_pairs.get((f64 ? 8 : 4) * (size_t)nst * std::max<int64_t>(W.pr.n_all, 1), st);
+    const size_t sums = (f64 ? 8 : 4) * (size_t)nst * std::max<int64_t>(W.pr.n_all, 1);
+    if (ok && !had_entries) c->ws_pairs.trim(std::max(kKeepBytes, sums));   // the set-up's scratch
+    if (ok) ws = c->ws_pairs.get(sums, st);
   } catch (const OutOfMemory &) {
     ok = false;
   } catch (...) {

@@ -354,6 +354,11 @@ void build_wavefunction(qpx_ctx *c, int nint, int64_t n_det, const uint64_t *psi
   W.sp.clear();
   W.fci.clear();
   W.pr.clear();
+  if (W.pr.bytes() + c->ws_pairs.buf.n > kKeepBytes) {
+    W.pr.release();
+    c->ws_pairs.release();
+  }
+  c->ws_fci.trim(kKeepBytes);
   c->ws_fci.graphs.clear();
   c->ws_pairs.graphs.clear();
   W.perm.clear();

@@ -227,3 +227,29 @@ def test_captured_call_builds_its_tables(ctx, hip, kind, path, first):
     hip.drop(g)
     x.free()
     y.free()
+
+
+def test_kept_memory_is_bounded(ctx, hip):
+    """811,801 determinants of 100 orbitals, 10a10b: 170M entries, whose set-up
+    sorts in 4.7 GB of scratch.  After the set-up the scratch is what the sums
+    need (1.4 GB); after the next wavefunction entries and scratch together are
+    no more than 4 GiB, as before the large one."""
+    M, na, nb = 100, 10, 10
+    dets = _singles_space(M, na, nb, 2.0, 1)
+    n = dets.shape[0]
+    assert n == (1 + na * (M - na)) ** 2
+    ctx.set_hamiltonian(synthetic_hamiltonian(M, na, nb, seed=4))
+    ctx._force_sigma_path(3)
+    ctx.set_wavefunction(dets[:50])
+    ctx.H_S2_u_0_nstates(np.ones(50))
+    small = hip.free_bytes()
+    _say(f"[sigma memory] n_det={n}")
+    ctx.set_wavefunction(dets)
+    before = hip.free_bytes()
+    ctx.H_S2_u_0_nstates(np.ones(n))
+    assert ctx._sigma_kernels() == 3
+    slots = n * (na * nb + na * (na - 1) + 2 * na)
+    # entries 12 bytes, positions 4, sums 8; host vectors' staging 6 x 8 per determinant; 10 % for whole wavefronts
+    assert before - hip.free_bytes() < 1.1 * 24 * slots + 48 * n + (256 << 20)
+    ctx.set_wavefunction(dets[:50])
+    assert small - hip.free_bytes() < (4 << 30) + 48 * n + (256 << 20)
