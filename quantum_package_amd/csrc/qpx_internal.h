@@ -269,10 +269,11 @@ struct RelaxedCapture {
 };
 
 // Scratch of calls that are enqueued on a caller's stream and return before
-// they have run: a call on another stream first waits for the last user.
+// they have run: every call first waits for the last user.  On one stream that
+// costs nothing; handles are not compared, since hipStreamPerThread stands for a
+// stream of each thread.
 struct StreamWorkspace {
   DBuf<char> buf;
-  hipStream_t last = nullptr;
   hipEvent_t done = nullptr;
   bool pending = false;
   ~StreamWorkspace() {
@@ -299,7 +300,7 @@ struct StreamWorkspace {
       graphs.push_back(std::move(g));
       return graphs.back()->buf.p;
     }
-    if (pending && last != s) QPX_HIP(hipStreamWaitEvent(s, done, 0));
+    if (pending) QPX_HIP(hipStreamWaitEvent(s, done, 0));
     // hipFree waits for the device, so the old buffer is not in use any more
     if (buf.n < bytes) buf.alloc(bytes);
     return buf.p;
@@ -315,7 +316,6 @@ struct StreamWorkspace {
     if (capturing(s)) return;
     if (!done) QPX_HIP(hipEventCreateWithFlags(&done, hipEventDisableTiming));
     QPX_HIP(hipEventRecord(done, s));
-    last = s;
     pending = true;
   }
 };

@@ -2,6 +2,9 @@
 and may not do to calls that are still queued and to captured graphs."""
 from __future__ import annotations
 
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 
@@ -253,3 +256,41 @@ def test_kept_memory_is_bounded(ctx, hip):
     assert before - hip.free_bytes() < 1.1 * 24 * slots + 48 * n + (256 << 20)
     ctx.set_wavefunction(dets[:50])
     assert small - hip.free_bytes() < (4 << 30) + 48 * n + (256 << 20)
+
+
+@pytest.mark.parametrize("kind,path", [("product", 1), ("selected", 3)])
+def test_calls_on_per_thread_streams(ctx, hip, kind, path):
+    """Calls of several threads, one after another, each on its thread's default
+    stream: one handle, as many streams, one scratch.  Every call gives what it
+    gives alone, bit for bit."""
+    n = _prepare(ctx, kind)
+    ctx._force_sigma_path(path)
+    _say(f"[sigma threads] {kind} n_det={n}")
+    per_thread = ctypes.c_void_p(2)   # hipStreamPerThread
+    xs = [Vectors(hip, n, 4, 0, seed) for seed in range(4)]
+    alone = []
+    for x in xs:
+        x.sigma(ctx, per_thread)
+        hip.sync()
+        alone.append(x.out())
+        x.clear()
+
+    turn = [threading.Event() for _ in range(len(xs) + 1)]
+
+    def enqueue(k):
+        turn[k].wait()
+        for _ in range(20):
+            xs[k].sigma(ctx, per_thread)
+        turn[k + 1].set()
+        turn[-1].wait()   # the thread, and with it its stream, lasts as long as its work
+        hip.sync()
+
+    threads = [threading.Thread(target=enqueue, args=(k,)) for k in range(len(xs))]
+    for t in threads:
+        t.start()
+    turn[0].set()
+    for t in threads:
+        t.join()
+    for x, want in zip(xs, alone):
+        assert _same(x.out(), want)
+        x.free()
