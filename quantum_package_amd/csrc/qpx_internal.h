@@ -360,6 +360,7 @@ void sigma_device(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, vo
 bool sigma_pairs(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, void *s_t, hipStream_t s);
 // implemented in sigma_fci.hip
 bool fci_ok(qpx_ctx *c, int n_st, size_t tsize);
+bool fci_pays(qpx_ctx *c, int n_st, size_t tsize);
 bool sigma_fci(qpx_ctx *c, int prec, int n_st, const void *u_t, void *v_t, void *s_t, hipStream_t s);
 // implemented in sigma_sparse.hip
 bool sparse_ok(qpx_ctx *c, int n_st);

@@ -709,8 +709,16 @@ void sigma_device(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s
   size_t ts = prec == QPX_FP64 ? sizeof(double) : sizeof(float);
   RelaxedCapture relaxed(st);
   // a product space takes the string-driven path (12.2 against 32.8 ms for
-  // 9.0M determinants, FP64, 4 states; 35 against 86 us for 4900)
-  if ((c->force_path == 0 || c->force_path == 1) && fci_ok(c, nst, ts) &&
+  // 9.0M determinants, FP64, 4 states; 35 against 86 us for 4900), but for some
+  // of few beta strings, and where a handful of alpha strings with more beta
+  // strings than the dense map takes leaves its column tiles empty (1 x 8008
+  // strings, FP64, 4 states: 840 us, 68 by bucket; 16 x 8008: 894, 1555)
+  auto strings = [&] {
+    if (c->force_path == 1) return true;
+    if (dense_ok(c, nst, ts)) return fci_pays(c, nst, ts);
+    return c->W.n_a >= 8 || !sparse_ok(c, nst);
+  };
+  if ((c->force_path == 0 || c->force_path == 1) && fci_ok(c, nst, ts) && strings() &&
       sigma_fci(c, prec, nst, u, v, s, st)) {
     c->sigma_path = c->sigma_kernels = 1;
     release_pairs(c, st);

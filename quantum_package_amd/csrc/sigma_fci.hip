@@ -873,6 +873,42 @@ bool fci_ok(qpx_ctx *c, int nst, size_t ts) {
   return true;
 }
 
+// Whether the string-driven kernels are the faster ones for a space that the
+// dense map could take too.  They give a beta string one workgroup of four
+// matrix wavefronts, the dense map one workgroup per 1024 alpha strings, and
+// their work does not shrink with the connections that an incomplete set
+// lacks: with fewer beta strings than CUs, many alpha strings and several
+// vectors the dense map can win (20 orbitals, 4a1b, 4845 x 20 strings, FP32, 2
+// vectors: 433 against 935 us; 14 orbitals, 6a1b, 3003 x 14, FP64, 1 vector: 263
+// against 206).  The two times, in microseconds, are fitted to 1072 spaces of
+// 1 to 256 beta strings (4 to 30 orbitals, 1, 2 and 4 vectors, both
+// precisions) within about 10 %.  By them no space is more than 8 % slower than
+// with the dense map, and the mean is 1 % above the faster of the two.  With more beta strings
+// the string-driven kernels were at most 4 % behind in incomplete sets, and 1.5
+// to 4 times as fast in complete ones.
+bool fci_pays(qpx_ctx *c, int nst, size_t ts) {
+  const Wfn &W = c->W;
+  if (W.n_b > 256 || W.n_a < 128) return true;
+  ensure_conn(c);
+  const Shape S = ab_shape(c, nst, ts, W.cb.max_singles);
+  if (!S.ks) return true;
+  const bool f64 = ts == 8;
+  const double n_a = W.n_a, n_b = W.n_b, groups = (W.n_a + 63) / 64, tiles = (double)S.mt / S.nrow;
+  const double strings = (f64 ? 18.4 : 20.6) + 5.0e-5 * nst * n_a * n_b +
+                         groups * (tiles * (f64 ? 0.103 + 0.161 * S.ks : 0.291 + 0.078 * S.ks) + (f64 ? 2.8 : 2.4));
+  // per string: beta singles k, alpha singles and same-spin partners
+  const double k = W.cb.n_singles / n_b, sa = W.ca.n_singles / n_a, same_a = sa + W.ca.n_doubles / n_a;
+  const double same_b = k + W.cb.n_doubles / n_b, rows = std::min(1.0, n_a / 1024);
+  const double rounds = (W.n_b * ((W.n_a + 1023) / 1024) + 255) / 256, row_rounds = n_a / 256;
+  const double stage = nst * n_a / 1024;
+  const double dense =
+      f64 ? 6.7 + 9.2 * nst + rounds * (k * (1.54 + 0.056 * stage + sa * rows * (0.014 + 0.067 * nst)) + 0.325 * rows * same_a) +
+                row_rounds * 0.110 * same_b
+          : 12.5 + 3.1 * nst + rounds * (k * (1.46 + 0.156 * stage + sa * rows * (0.110 + 0.016 * nst)) + 0.222 * rows * same_a) +
+                row_rounds * (1.72 + 0.054 * same_b);
+  return strings < 0.95 * dense;
+}
+
 // False when the tables or the scratch do not fit the device's memory: the
 // caller then takes a path that needs none.  What the call began goes again;
 // what was there before it stays, for the calls and captured graphs that use it.

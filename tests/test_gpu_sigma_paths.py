@@ -6,7 +6,7 @@ import contextlib
 import numpy as np
 import pytest
 
-from quantum_package_amd.hamiltonian import fci_space, hf_determinant, synthetic_hamiltonian
+from quantum_package_amd.hamiltonian import Hamiltonian, fci_space, hf_determinant, synthetic_hamiltonian
 from test_gpu_sigma import BUCKETS, PRODUCT, _product_space, _random_space, _say, _singles_space
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +102,28 @@ def test_bucket_fp32_error(ctx, M, na, nb, n, vector):
     walk = ctx.H_S2_u_0_nstates(u, prec=1)
     for x, y, r in zip(by_bucket, walk, ref):
         assert np.linalg.norm(x - r) <= np.linalg.norm(y - r)
+
+
+# complete spaces of few beta strings: measured 0.46, 0.92 and 0.73 of the
+# string-driven kernels' time with the dense map, then 1.8, 2.0 and 1.9 of it;
+# one alpha string and more beta strings than the dense map takes: 0.08 by bucket
+@pytest.mark.parametrize("M,na,nb,nst,prec,kernels", [
+    (20, 4, 1, 2, 1, DENSE), (14, 6, 1, 4, 0, DENSE), (14, 7, 0, 4, 0, DENSE), (16, 16, 6, 4, 0, BUCKET),
+    (12, 6, 1, 4, 0, STRINGS), (14, 6, 2, 4, 0, STRINGS), (8, 4, 4, 4, 1, STRINGS)])
+def test_few_beta_strings(ctx, M, na, nb, nst, prec, kernels):
+    """The automatic path takes the faster kernels; its values are those of the
+    forced paths (FP64: 1e-11 of the largest entry, FP32: 2e-5 of the norm)."""
+    H = synthetic_hamiltonian(M, na, max(nb, 1), seed=4)
+    ctx.set_hamiltonian(Hamiltonian(M=M, n_alpha=na, n_beta=nb, h=H.h, eri=H.eri, seed=H.seed))
+    dets = fci_space(M, na, nb)
+    ctx.set_wavefunction(dets)
+    u = np.random.default_rng(1).standard_normal((dets.shape[0], nst))
+    _say(f"[sigma few beta] M={M} {na}a{nb}b nst={nst} prec={prec} n_det={dets.shape[0]}")
+    got = ctx.H_S2_u_0_nstates(u, prec=prec)
+    assert ctx._sigma_kernels() == kernels
+    ctx._force_sigma_path(DENSE if kernels == STRINGS else STRINGS)
+    for x, r in zip(got, ctx.H_S2_u_0_nstates(u)):
+        if prec == 0:
+            assert np.max(np.abs(x - r)) < 1e-11 * max(1.0, np.max(np.abs(r)))
+        else:
+            assert np.linalg.norm(x - r) < 2e-5 * max(1.0, np.linalg.norm(r))
