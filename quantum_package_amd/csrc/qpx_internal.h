@@ -1,6 +1,7 @@
 // qpx_internal.h -- shared state of libqpx (MI355X / gfx950).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <memory>
@@ -59,6 +60,7 @@ inline void device_alloc(void **p, size_t bytes) {
 // the bucket kernels and of the string-driven ones; more costs less to allocate
 // again than the set-up it serves (some 10^8 entries to sort).
 constexpr size_t kKeepBytes = (size_t)4 << 30;
+constexpr size_t kKeepFci = (size_t)64 << 20;   // tables of a product space: what allocations cost shows in small ones
 
 // Device buffer with RAII.
 template <typename T>
@@ -121,15 +123,68 @@ struct Ham {
   double ref_energy = 0.0;        // ref_bitmask_energy of the HF determinant
 };
 
+// Small arrays laid out one after another in one allocation: a dozen allocations
+// cost as much as ten sigma calls of a small space.  Arrays of 1 MB and more get
+// memory of their own (one block of several MB took 0.2 ms longer).  lay() runs
+// twice, first to add up the size, then to hand out the addresses.
+template <typename T>
+struct View {
+  T *p = nullptr;
+};
+struct Block {
+  DBuf<char> mem;
+  std::vector<std::unique_ptr<DBuf<char>>> own;
+  size_t used = 0, n_own = 0;
+  bool sizing = true;
+  // memory that is large enough stays, unless it is far too large
+  static void reserve(DBuf<char> &b, size_t n) {
+    if (b.n < n || b.n / 4 > std::max(n, (size_t)1 << 20)) b.alloc(n);
+  }
+  template <typename T>
+  void lay(View<T> &v, size_t count) {
+    const size_t n = (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+    if (n >= (size_t)1 << 20) {
+      if (n_own == own.size()) own.push_back(std::make_unique<DBuf<char>>());
+      DBuf<char> &b = *own[n_own++];
+      if (sizing) reserve(b, n);
+      else v.p = reinterpret_cast<T *>(b.p);
+      return;
+    }
+    if (!sizing) v.p = reinterpret_cast<T *>(mem.p + used);
+    used += n;
+  }
+  size_t bytes() const {
+    size_t n = mem.n;
+    for (const auto &b : own) n += b->n;
+    return n;
+  }
+  void release() {
+    mem.release();
+    own.clear();
+  }
+  template <typename F>
+  void layout(F f) {   // f(): the lay() calls
+    for (bool first : {true, false}) {
+      sizing = first;
+      used = n_own = 0;
+      f();
+      if (first) {
+        reserve(mem, used);
+        own.resize(n_own);
+      }
+    }
+  }
+};
+
 // Connectivity of unique spin strings (within the unique set).
 struct SpinConn {
-  DBuf<int> s_ptr, s_idx;         // singles: CSR over strings
-  DBuf<uint32_t> s_info;          // h | p<<8 | (phase<0)<<16 (0-based orbitals)
-  DBuf<double> s_val;             // same-spin part of the single element, phase included
-  DBuf<float> s_valf;
-  DBuf<int> d_ptr, d_idx;         // doubles
-  DBuf<double> d_val;             // full same-spin double element, phase included
-  DBuf<float> d_valf;
+  View<int> s_ptr, s_idx;         // singles: CSR over strings
+  View<uint32_t> s_info;          // h | p<<8 | (phase<0)<<16 (0-based orbitals)
+  View<double> s_val;             // same-spin part of the single element, phase included
+  View<float> s_valf;
+  View<int> d_ptr, d_idx;         // doubles
+  View<double> d_val;             // full same-spin double element, phase included
+  View<float> d_valf;
   int max_singles = 0, max_doubles = 0;
   int64_t n_singles = 0, n_doubles = 0;
 };
@@ -158,33 +213,40 @@ struct SparseIdx {
 // on first use: partners of 16 strings at a time, their matrix elements and
 // the placement tables, per precision.
 struct SpinTiles {
-  int ntile = 0, nchunk = 0;
-  DBuf<int> ptr, idx;
+  int ntile = 0;
+  int64_t nchunk = 0;    // room for the partners of all tiles, in chunks of 8
+  View<int2> range;      // chunks of a tile
+  View<int> idx;
 };
 template <typename T>
 struct FciTables {
   bool valid = false;
-  DBuf<T> coef_a, coef_b, gb, vo;
-  DBuf<uint4> tgt;
-  void clear() {
+  Block mem;
+  View<T> coef_a, coef_b, gb, vo;
+  View<uint4> tgt;
+  void release() {
     valid = false;
-    coef_a.release(); coef_b.release(); gb.release(); vo.release(); tgt.release();
+    mem.release();
   }
 };
 struct FciPlan {
   bool valid = false;
   int lda = 0, ldb = 0, ldt = 0;
-  DBuf<int> vrow;
-  DBuf<uint32_t> map_a, map_b;
+  Block mem, lists;      // maps and ranges; partners
+  View<uint32_t> map_a, map_b;
   SpinTiles a, b;
   FciTables<double> t64;
   FciTables<float> t32;
-  void clear() {
+  void clear() {   // the next wavefunction may take the memory
+    valid = t64.valid = t32.valid = false;
+    if (mem.bytes() + lists.bytes() + t64.mem.bytes() + t32.mem.bytes() > kKeepFci) release();
+  }
+  void release() {
     valid = false;
-    vrow.release(); map_a.release(); map_b.release();
-    for (SpinTiles *t : {&a, &b}) { t->ptr.release(); t->idx.release(); t->ntile = t->nchunk = 0; }
-    t64.clear();
-    t32.clear();
+    mem.release();
+    lists.release();
+    t64.release();
+    t32.release();
   }
 };
 
@@ -225,7 +287,9 @@ struct Wfn {
   bool conn_valid = false;
   DBuf<double> hdiag, sdiag;              // bilinear order
   // per-string scan costs for the generic alpha/beta kernel
-  DBuf<int64_t> cost_a, cost_b;
+  View<int64_t> cost_a, cost_b;
+  DBuf<int> conn_count;                   // singles and doubles per string
+  Block conn;                             // ca, cb and the costs
   std::vector<int> col_len_h, row_len_h;
   int max_col = 0, max_row = 0;
   SparseIdx sp;                           // built on first use of the sparse path

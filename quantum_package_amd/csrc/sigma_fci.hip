@@ -96,12 +96,30 @@ constexpr uint32_t kNone = 0xffffffffu;
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------- tables
+// A set-up kernel does both spins, blocks [0, n of alpha) and the rest: in a
+// small space launches, allocations and waits are the time to the first result
+// (4900 determinants, 4 vectors: 395 us; 655 with a launch per table and spin, an
+// allocation per array and the partners' numbers read back, 480 with the dense
+// map, which needs no tables).
+struct SpinArgs {
+  const int *s_ptr, *s_idx, *d_ptr, *d_idx;
+  const uint32_t *s_info;
+  int n, ntile, room;   // room: chunks of 8 partners at a tile's disposal, 0 = as many as it needs
+  uint32_t *map;
+  int2 *range;
+  int *idx;
+};
+
 // map[i * npo + pair] = partner of string i through the single excitation
 // between the pair's orbitals | sign << 31; kNone when both or neither are
 // occupied
-__global__ void fci_map_kernel(const int *__restrict__ s_ptr, const int *__restrict__ s_idx,
-                               const uint32_t *__restrict__ s_info, int n, int npo, uint32_t *__restrict__ map) {
-  const int i = blockIdx.x;
+__global__ void fci_map_kernel(SpinArgs A, SpinArgs B, int npo) {
+  int i = blockIdx.x;
+  const bool beta = i >= A.n;
+  if (beta) i -= A.n;
+  const int *s_ptr = beta ? B.s_ptr : A.s_ptr, *s_idx = beta ? B.s_idx : A.s_idx;
+  const uint32_t *s_info = beta ? B.s_info : A.s_info;
+  uint32_t *map = beta ? B.map : A.map;
   for (int x = threadIdx.x; x < npo; x += blockDim.x) map[(int64_t)i * npo + x] = kNone;
   __syncthreads();
   for (int e = s_ptr[i] + (int)threadIdx.x; e < s_ptr[i + 1]; e += blockDim.x) {
@@ -118,60 +136,77 @@ __global__ void fci_map_kernel(const int *__restrict__ s_ptr, const int *__restr
 // without a target points at the lane's own spare word behind the column, so
 // that the placement needs no branch.  Rows npo + p are the diagonal pairs
 // (pp): their target is the string itself when it holds p.
+// Behind the targets, in the same launch: gb[i * npo + row], the sum over the
+// orbitals k of beta string i of (row|kk), and vo[npo][nr], the integrals of each
+// off-diagonal pair with all pairs.
 template <typename T>
-__global__ void fci_target_kernel(const uint32_t *__restrict__ map, const uint64_t *__restrict__ astr, int n_a,
-                                  int ldt, int M, int npo, int mt, uint4 *__restrict__ tgt) {
-  const int64_t n = (int64_t)mt * ldt * 4;
-  for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < n; x += (int64_t)gridDim.x * blockDim.x) {
-    const int q = (int)(x & 3);
-    const int a = (int)((x >> 2) % ldt), tile = (int)((x >> 2) / ldt);
-    uint32_t w[4];
+struct TableArgs {
+  const uint32_t *map_a;
+  const uint64_t *astr, *bstr;
+  const T *V;
+  int n_a, n_b, ldt, M, npo, nr, npair;
+  int64_t n_tgt, n_gb, n_vo;
+  uint4 *tgt;
+  T *gb, *vo;
+};
+// packed pair of row: off-diagonal pairs first, then the diagonal ones
+__device__ inline int64_t pair_of_row(int row, int npo) {
+  if (row >= npo) return pair_index(row - npo, row - npo);
+  int q = (int)((1.0 + sqrt(1.0 + 8.0 * row)) / 2.0);
+  while (q * (q - 1) / 2 > row) --q;
+  while ((q + 1) * q / 2 <= row) ++q;
+  return pair_index(row - q * (q - 1) / 2, q);
+}
+template <typename T>
+__global__ __launch_bounds__(256) void fci_tables_kernel(TableArgs<T> A) {
+  const int64_t n = A.n_tgt + A.n_gb + A.n_vo;
+  for (int64_t y = blockIdx.x * (int64_t)256 + threadIdx.x; y < n; y += (int64_t)gridDim.x * 256) {
+    int64_t x = y;
+    if (x < A.n_tgt) {
+      const int q = (int)(x & 3);
+      const int a = (int)((x >> 2) % A.ldt), tile = (int)((x >> 2) / A.ldt);
+      uint32_t w[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * tile + Mfma<T>::row(q, r);
-      w[r] = (a < n_a && row < npo) ? map[(int64_t)a * npo + row] : kNone;
-      if (a < n_a && row >= npo && row < npo + M && ((astr[a] >> (row - npo)) & 1)) w[r] = (uint32_t)a;
-      if (w[r] == kNone) w[r] = (uint32_t)(n_a + 16 * q + (a & 15));
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * tile + Mfma<T>::row(q, r);
+        w[r] = (a < A.n_a && row < A.npo) ? A.map_a[(int64_t)a * A.npo + row] : kNone;
+        if (a < A.n_a && row >= A.npo && row < A.npo + A.M && ((A.astr[a] >> (row - A.npo)) & 1)) w[r] = (uint32_t)a;
+        if (w[r] == kNone) w[r] = (uint32_t)(A.n_a + 16 * q + (a & 15));
+      }
+      A.tgt[x] = make_uint4(w[0], w[1], w[2], w[3]);
+      continue;
     }
-    tgt[x] = make_uint4(w[0], w[1], w[2], w[3]);
-  }
-}
-
-// out[i * npo + row] = sum over the orbitals k of string i of (row|kk)
-template <typename T>
-__global__ void fci_coulomb_kernel(const uint64_t *__restrict__ str, const T *__restrict__ V, int npair,
-                                   const int *__restrict__ vrow, int n, int npo, T *__restrict__ out) {
-  const int64_t m = (int64_t)npo * n;
-  for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < m; x += (int64_t)gridDim.x * blockDim.x) {
-    const int i = (int)(x / npo), row = (int)(x - (int64_t)i * npo);
-    T g = T(0);
-    for (uint64_t y = str[i]; y; y &= y - 1) {
-      const int k = __ffsll((unsigned long long)y) - 1;
-      g += V[(int64_t)vrow[row] * npair + pair_index(k, k)];
+    x -= A.n_tgt;
+    if (x < A.n_gb) {
+      const int i = (int)(x / A.npo), row = (int)(x - (int64_t)i * A.npo);
+      const int64_t P = pair_of_row(row, A.npo);
+      T g = T(0);
+      for (uint64_t z = A.bstr[i]; z; z &= z - 1) {
+        const int k = __ffsll((unsigned long long)z) - 1;
+        g += A.V[P * A.npair + pair_index(k, k)];
+      }
+      A.gb[x] = g;
+      continue;
     }
-    out[x] = g;
+    x -= A.n_gb;
+    A.vo[x] = A.V[pair_of_row((int)(x / A.nr), A.npo) * A.npair + pair_of_row((int)(x % A.nr), A.npo)];
   }
-}
-
-// integrals of each off-diagonal pair with all pairs, [npo][nr]
-template <typename T>
-__global__ void fci_pairs_kernel(const T *__restrict__ V, int npair, const int *__restrict__ vrow, int npo, int nr,
-                                 T *__restrict__ vo) {
-  for (int x = blockIdx.x * blockDim.x + threadIdx.x; x < npo * nr; x += gridDim.x * blockDim.x)
-    vo[x] = V[(int64_t)vrow[x / nr] * npair + vrow[x % nr]];
 }
 
 // Partners of 16 consecutive strings: a bitmap of the string set in LDS
-// collects the singles and doubles of the 16.  Without `idx` only their
-// number is written, rounded up to pairs of chunks of 8; with it the ascending
-// list (padded with its first entry).
-__global__ __launch_bounds__(256) void fci_union_kernel(const int *__restrict__ s_ptr, const int *__restrict__ s_idx,
-                                                        const int *__restrict__ d_ptr, const int *__restrict__ d_idx,
-                                                        int n, int *__restrict__ chunks, const int *__restrict__ ptr,
-                                                        int *__restrict__ idx) {
+// collects the singles and doubles of the 16; their number, rounded up to pairs
+// of chunks of 8, gives the tile's range and the ascending list (padded with its
+// first entry) goes to it.  With room for every tile one pass does both; without,
+// a first pass (write = false) leaves the numbers in range[].y and the host the
+// ranges for a second.
+__global__ __launch_bounds__(256) void fci_union_kernel(SpinArgs A, SpinArgs B, bool write) {
   extern __shared__ uint32_t bits[];
   __shared__ int part[256];
-  const int tile = blockIdx.x, tid = threadIdx.x, nw = (n + 31) >> 5;
+  int tile = blockIdx.x;
+  const SpinArgs &S = tile < A.ntile ? A : B;
+  if (tile >= A.ntile) tile -= A.ntile;
+  const int *s_ptr = S.s_ptr, *s_idx = S.s_idx, *d_ptr = S.d_ptr, *d_idx = S.d_idx;
+  const int n = S.n, tid = threadIdx.x, nw = (n + 31) >> 5;
   for (int x = tid; x < nw; x += 256) bits[x] = 0;
   __syncthreads();
   const int i0 = 16 * tile, i1 = min(n, i0 + 16);
@@ -190,11 +225,12 @@ __global__ __launch_bounds__(256) void fci_union_kernel(const int *__restrict__ 
     total += part[x];
   }
   const int nch = (total + 15) / 16 * 2;   // an even number: the product takes two at a time
-  if (!idx) {
-    if (tid == 0) chunks[tile] = nch;
+  if (S.room && tid == 0) S.range[tile] = make_int2(tile * S.room, tile * S.room + nch);
+  if (!write) {
+    if (tid == 0) S.range[tile].y = nch;
     return;
   }
-  int *out = idx + (int64_t)8 * ptr[tile];
+  int *out = S.idx + (int64_t)8 * (S.room ? tile * S.room : S.range[tile].x);
   for (int w = w0; w < w1; ++w)
     for (uint32_t y = bits[w]; y; y &= y - 1) out[before++] = 32 * w + __ffs(y) - 1;
   __syncthreads();
@@ -204,14 +240,24 @@ __global__ __launch_bounds__(256) void fci_union_kernel(const int *__restrict__ 
 // matrix elements of a tile: coef[(8 chunk + pos) * 16 + i % 16], zero where
 // string i and the partner are not connected
 template <typename T>
-__global__ __launch_bounds__(256) void fci_coef_kernel(const int *__restrict__ s_ptr, const int *__restrict__ s_idx,
-                                                       const T *__restrict__ s_val, const int *__restrict__ d_ptr,
-                                                       const int *__restrict__ d_idx, const T *__restrict__ d_val,
-                                                       int n, const int *__restrict__ ptr, const int *__restrict__ idx,
-                                                       T *__restrict__ coef) {
-  const int tile = blockIdx.x, tid = threadIdx.x;
-  const int64_t c0 = (int64_t)8 * ptr[tile];
-  const int np = 8 * (ptr[tile + 1] - ptr[tile]);
+struct CoefArgs {
+  const T *s_val, *d_val;
+  T *coef;
+};
+template <typename T>
+__global__ __launch_bounds__(256) void fci_coef_kernel(SpinArgs A, CoefArgs<T> CA, SpinArgs B, CoefArgs<T> CB) {
+  int tile = blockIdx.x;
+  const bool beta = tile >= A.ntile;
+  if (beta) tile -= A.ntile;
+  const SpinArgs &S = beta ? B : A;
+  const CoefArgs<T> &C = beta ? CB : CA;
+  const int *s_ptr = S.s_ptr, *s_idx = S.s_idx, *d_ptr = S.d_ptr, *d_idx = S.d_idx, *idx = S.idx;
+  const T *s_val = C.s_val, *d_val = C.d_val;
+  T *coef = C.coef;
+  const int n = S.n, tid = threadIdx.x;
+  const int2 range = S.range[tile];
+  const int64_t c0 = (int64_t)8 * range.x;
+  const int np = 8 * (range.y - range.x);
   for (int x = tid; x < 16 * np; x += 256) coef[c0 * 16 + x] = T(0);
   __syncthreads();
   const int i0 = 16 * tile, i1 = min(n, i0 + 16);
@@ -271,7 +317,7 @@ __global__ __launch_bounds__(256) void fci_planes_kernel(const T *__restrict__ u
 // The four wavefronts of a workgroup, and neighbouring workgroups, take the
 // string tiles of one column block, whose rows (n x 16 NT values) stay in L2.
 template <typename T, int NT, int W, bool ALPHA>
-__global__ __launch_bounds__(256, 2) void sigma_fci_spin_kernel(const int *__restrict__ ptr,
+__global__ __launch_bounds__(256, 2) void sigma_fci_spin_kernel(const int2 *__restrict__ range,
                                                                 const int *__restrict__ idx,
                                                                 const T *__restrict__ coef, int n, int ntile,
                                                                 int ld, int ncol, int ngrp, int nblk,
@@ -292,7 +338,7 @@ __global__ __launch_bounds__(256, 2) void sigma_fci_spin_kernel(const int *__res
   uint32_t col[NP];
 #pragma unroll
   for (int t = 0; t < NP; ++t) col[t] = min(c0 + 16 * W * t, ld - 16 * W) + W * j;   // past the end: the last columns again
-  const int k0 = ptr[tile], k1 = ptr[tile + 1];
+  const int k0 = range[tile].x, k1 = range[tile].y;
   v4 acc[NT];
 #pragma unroll
   for (int t = 0; t < NT; ++t) acc[t] = v4{T(0), T(0), T(0), T(0)};
@@ -696,59 +742,16 @@ Shape ab_shape(const qpx_ctx *c, int nst, size_t ts, int max_singles) {
   return S;
 }
 
-void build_tiles(qpx_ctx *c, const SpinConn &cc, int n, SpinTiles &t) {
-  hipStream_t s = c->stream;
-  t.ntile = (n + 15) / 16;
-  DBuf<int> chunks;
-  chunks.alloc(t.ntile);
-  const size_t lds = sizeof(uint32_t) * ((n + 31) / 32);
-  hipLaunchKernelGGL(fci_union_kernel, dim3(t.ntile), dim3(256), lds, s, cc.s_ptr.p, cc.s_idx.p, cc.d_ptr.p,
-                     cc.d_idx.p, n, chunks.p, (const int *)nullptr, (int *)nullptr);
-  QPX_HIP(hipGetLastError());
-  std::vector<int> h(t.ntile), p(t.ntile + 1, 0);
-  QPX_HIP(hipMemcpyAsync(h.data(), chunks.p, sizeof(int) * t.ntile, hipMemcpyDeviceToHost, s));
-  QPX_HIP(hipStreamSynchronize(s));
-  for (int i = 0; i < t.ntile; ++i) p[i + 1] = p[i] + h[i];
-  t.nchunk = p[t.ntile];
-  t.ptr.upload(p, s);
-  t.idx.alloc(std::max<size_t>((size_t)8 * t.nchunk, 1));
-  hipLaunchKernelGGL(fci_union_kernel, dim3(t.ntile), dim3(256), lds, s, cc.s_ptr.p, cc.s_idx.p, cc.d_ptr.p,
-                     cc.d_idx.p, n, chunks.p, (const int *)t.ptr.p, t.idx.p);
-  QPX_HIP(hipGetLastError());
-  QPX_HIP(hipStreamSynchronize(s));   // p and chunks go out of scope
+SpinArgs spin_args(const SpinConn &cc, int n, const SpinTiles &t, int room, const View<uint32_t> &map) {
+  return SpinArgs{cc.s_ptr.p, cc.s_idx.p, cc.d_ptr.p, cc.d_idx.p, cc.s_info.p, n, t.ntile, room, map.p, t.range.p, t.idx.p};
 }
 
-template <typename T>
-void build_tables(qpx_ctx *c) {
-  Wfn &W = c->W;
-  FciPlan &P = W.fci;
-  FciTables<T> &t = Prec<T>::tab(P);
-  if (t.valid) return;
-  hipStream_t s = c->stream;
-  const int M = c->H.M, npo = M * (M - 1) / 2, nr = npo + M, mt = (nr + 15) / 16;
-  // memory first: a set of tables that does not fit is tried again by every call
-  t.coef_a.alloc(std::max<size_t>((size_t)128 * P.a.nchunk, 1));
-  t.coef_b.alloc(std::max<size_t>((size_t)128 * P.b.nchunk, 1));
-  t.tgt.alloc((size_t)mt * P.ldt * 4);
-  t.gb.alloc((size_t)npo * W.n_b);
-  t.vo.alloc((size_t)npo * nr);
-  auto coefs = [&](const SpinConn &cc, int n, const SpinTiles &tl, DBuf<T> &out) {
-    hipLaunchKernelGGL(fci_coef_kernel<T>, dim3(tl.ntile), dim3(256), 0, s, cc.s_ptr.p, cc.s_idx.p, Prec<T>::sval(cc),
-                       cc.d_ptr.p, cc.d_idx.p, Prec<T>::dval(cc), n, tl.ptr.p, tl.idx.p, out.p);
-    QPX_HIP(hipGetLastError());
-  };
-  coefs(W.ca, W.n_a, P.a, t.coef_a);
-  coefs(W.cb, W.n_b, P.b, t.coef_b);
-  hipLaunchKernelGGL(fci_target_kernel<T>, dim3(1024), dim3(256), 0, s, P.map_a.p, W.astr.p, W.n_a, P.ldt, M, npo, mt, t.tgt.p);
-  hipLaunchKernelGGL(fci_coulomb_kernel<T>, dim3(1024), dim3(256), 0, s, W.bstr.p, Prec<T>::V(c->H), c->H.npair,
-                     P.vrow.p, W.n_b, npo, t.gb.p);
-  hipLaunchKernelGGL(fci_pairs_kernel<T>, dim3(256), dim3(256), 0, s, Prec<T>::V(c->H), c->H.npair, P.vrow.p, npo, nr,
-                     t.vo.p);
-  QPX_HIP(hipGetLastError());
-  QPX_HIP(hipStreamSynchronize(s));
-  t.valid = true;
+// most chunks of 8 partners (an even number, not 0) the 16 strings of a tile have
+int most_chunks(const SpinConn &cc, int n) {
+  return std::max(2, (int)((std::min<int64_t>(n, 16 * ((int64_t)cc.max_singles + cc.max_doubles)) + 15) / 16 * 2));
 }
 
+// Enqueued on the context's stream, as build_tables; the caller waits.
 void build_plan(qpx_ctx *c) {
   Wfn &W = c->W;
   FciPlan &P = W.fci;
@@ -759,22 +762,79 @@ void build_plan(qpx_ctx *c) {
   P.lda = round_up(W.n_a, W.n_a >= 256 ? 64 : 32);
   P.ldb = round_up(W.n_b, W.n_b >= 256 ? 64 : 32);
   P.ldt = round_up(W.n_a, 64);
-  std::vector<int> vrow(npo + M);
-  for (int q = 0; q < M; ++q) {
-    for (int p = 0; p < q; ++p) vrow[off_pair(p, q)] = (int)pair_index(p, q);
-    vrow[npo + q] = (int)pair_index(q, q);
+  P.a.ntile = (W.n_a + 15) / 16;
+  P.b.ntile = (W.n_b + 15) / 16;
+  P.mem.layout([&] {
+    P.mem.lay(P.map_a, (size_t)W.n_a * npo);
+    P.mem.lay(P.map_b, (size_t)W.n_b * npo);
+    P.mem.lay(P.a.range, P.a.ntile);
+    P.mem.lay(P.b.range, P.b.ntile);
+  });
+  // Room for the most partners a tile can have, where the FP64 elements (1 KB a
+  // chunk) then take at most 4 MB: the partners are listed without a look at
+  // their number.
+  int room_a = most_chunks(W.ca, W.n_a), room_b = most_chunks(W.cb, W.n_b);
+  P.a.nchunk = (int64_t)P.a.ntile * room_a;
+  P.b.nchunk = (int64_t)P.b.ntile * room_b;
+  const size_t lds = sizeof(uint32_t) * ((std::max(W.n_a, W.n_b) + 31) / 32);
+  const dim3 grid(P.a.ntile + P.b.ntile), block(256);
+  auto args = [&](bool beta) {
+    return beta ? spin_args(W.cb, W.n_b, P.b, room_b, P.map_b) : spin_args(W.ca, W.n_a, P.a, room_a, P.map_a);
+  };
+  if (P.a.nchunk + P.b.nchunk > 4096) {
+    room_a = room_b = 0;
+    hipLaunchKernelGGL(fci_union_kernel, grid, block, lds, s, args(false), args(true), false);
+    QPX_HIP(hipGetLastError());
+    for (SpinTiles *t : {&P.a, &P.b}) {
+      std::vector<int2> r(t->ntile);
+      QPX_HIP(hipMemcpyAsync(r.data(), t->range.p, sizeof(int2) * t->ntile, hipMemcpyDeviceToHost, s));
+      QPX_HIP(hipStreamSynchronize(s));
+      int64_t at = 0;
+      for (int2 &x : r) {
+        x = make_int2((int)at, (int)at + x.y);
+        at = x.y;
+      }
+      t->nchunk = at;
+      QPX_HIP(hipMemcpyAsync(t->range.p, r.data(), sizeof(int2) * t->ntile, hipMemcpyHostToDevice, s));
+      QPX_HIP(hipStreamSynchronize(s));   // r goes out of scope
+    }
   }
-  P.vrow.upload(vrow, s);
-  P.map_a.alloc((size_t)W.n_a * npo);
-  P.map_b.alloc((size_t)W.n_b * npo);
-  hipLaunchKernelGGL(fci_map_kernel, dim3(W.n_a), dim3(64), 0, s, W.ca.s_ptr.p, W.ca.s_idx.p, W.ca.s_info.p, W.n_a,
-                     npo, P.map_a.p);
-  hipLaunchKernelGGL(fci_map_kernel, dim3(W.n_b), dim3(64), 0, s, W.cb.s_ptr.p, W.cb.s_idx.p, W.cb.s_info.p, W.n_b,
-                     npo, P.map_b.p);
+  P.lists.layout([&] {
+    P.lists.lay(P.a.idx, (size_t)8 * P.a.nchunk);
+    P.lists.lay(P.b.idx, (size_t)8 * P.b.nchunk);
+  });
+  hipLaunchKernelGGL(fci_map_kernel, dim3(W.n_a + W.n_b), dim3(64), 0, s, args(false), args(true), npo);
+  hipLaunchKernelGGL(fci_union_kernel, grid, block, lds, s, args(false), args(true), true);
   QPX_HIP(hipGetLastError());
-  build_tiles(c, W.ca, W.n_a, P.a);
-  build_tiles(c, W.cb, W.n_b, P.b);
   P.valid = true;
+}
+
+template <typename T>
+void build_tables(qpx_ctx *c) {
+  Wfn &W = c->W;
+  FciPlan &P = W.fci;
+  FciTables<T> &t = Prec<T>::tab(P);
+  if (t.valid) return;
+  hipStream_t s = c->stream;
+  const int M = c->H.M, npo = M * (M - 1) / 2, nr = npo + M, mt = (nr + 15) / 16;
+  t.mem.layout([&] {
+    t.mem.lay(t.coef_a, (size_t)128 * P.a.nchunk);
+    t.mem.lay(t.coef_b, (size_t)128 * P.b.nchunk);
+    t.mem.lay(t.tgt, (size_t)mt * P.ldt * 4);
+    t.mem.lay(t.gb, (size_t)npo * W.n_b);
+    t.mem.lay(t.vo, (size_t)npo * nr);
+  });
+  const SpinArgs a = spin_args(W.ca, W.n_a, P.a, 0, P.map_a), b = spin_args(W.cb, W.n_b, P.b, 0, P.map_b);
+  hipLaunchKernelGGL(fci_coef_kernel<T>, dim3(P.a.ntile + P.b.ntile), dim3(256), 0, s, a,
+                     CoefArgs<T>{Prec<T>::sval(W.ca), Prec<T>::dval(W.ca), t.coef_a.p}, b,
+                     CoefArgs<T>{Prec<T>::sval(W.cb), Prec<T>::dval(W.cb), t.coef_b.p});
+  const TableArgs<T> A{P.map_a.p, W.astr.p, W.bstr.p, Prec<T>::V(c->H), W.n_a, W.n_b, P.ldt, M, npo, nr, c->H.npair,
+                       (int64_t)mt * P.ldt * 4, (int64_t)npo * W.n_b, (int64_t)npo * nr, t.tgt.p, t.gb.p, t.vo.p};
+  hipLaunchKernelGGL(fci_tables_kernel<T>, dim3((unsigned)std::min<int64_t>((A.n_tgt + A.n_gb + A.n_vo + 255) / 256, 4096)),
+                     dim3(256), 0, s, A);
+  QPX_HIP(hipGetLastError());
+  QPX_HIP(hipStreamSynchronize(s));   // the call may be on another stream
+  t.valid = true;
 }
 
 template <typename T, int KS>
@@ -801,9 +861,9 @@ void launch_spin(qpx_ctx *c, int nst, const T *pa, const T *pb, T *y, hipStream_
   FciTables<T> &t = Prec<T>::tab(P);
   const int ga = (P.ldb + 16 * NT - 1) / (16 * NT), gb = (P.lda + 16 * NT - 1) / (16 * NT);
   const int na = nst * ga * ((P.a.ntile + 3) / 4), nb = nst * gb * ((P.b.ntile + 3) / 4);
-  hipLaunchKernelGGL((sigma_fci_spin_kernel<T, NT, W, true>), dim3(na), dim3(256), 0, st, P.a.ptr.p, P.a.idx.p,
+  hipLaunchKernelGGL((sigma_fci_spin_kernel<T, NT, W, true>), dim3(na), dim3(256), 0, st, P.a.range.p, P.a.idx.p,
                      t.coef_a.p, F.n_a, P.a.ntile, P.ldb, F.n_b, ga, na, pa, y, P.lda, F.n_b);
-  hipLaunchKernelGGL((sigma_fci_spin_kernel<T, NT, W, false>), dim3(nb), dim3(256), 0, st, P.b.ptr.p, P.b.idx.p,
+  hipLaunchKernelGGL((sigma_fci_spin_kernel<T, NT, W, false>), dim3(nb), dim3(256), 0, st, P.b.range.p, P.b.idx.p,
                      t.coef_b.p, F.n_b, P.b.ntile, P.lda, F.n_a, gb, nb, pb, y, P.lda, F.n_b);
   QPX_HIP(hipGetLastError());
 }
@@ -918,10 +978,10 @@ bool sigma_fci(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, h
   const bool had_plan = P.valid, had_tables = prec == QPX_FP64 ? P.t64.valid : P.t32.valid;
   auto drop = [&] {
     if (!had_tables) {
-      if (prec == QPX_FP64) P.t64.clear();
-      else P.t32.clear();
+      if (prec == QPX_FP64) P.t64.release();
+      else P.t32.release();
     }
-    if (!had_plan) P.clear();
+    if (!had_plan) P.release();
   };
   char *ws = nullptr;
   try {

@@ -149,47 +149,40 @@ __global__ void scan_cost_kernel(const int *__restrict__ sptr, const int *__rest
 }
 
 // ---------------------------------------------------------------------------
-static void build_conn(qpx_ctx *c, const DBuf<uint64_t> &str, int n, int nint, SpinConn &cc) {
+// singles and doubles of every string among the n, to ns and nd
+static void count_conn(qpx_ctx *c, const DBuf<uint64_t> &str, int n, int nint, int *ns, int *nd) {
   hipStream_t s = c->stream;
-  DBuf<int> ns, nd;
-  ns.alloc(n);
-  nd.alloc(n);
-  int grid = (n + 255) / 256;
+  const int grid = (n + 255) / 256;
   switch (nint) {
-    case 1: hipLaunchKernelGGL(conn_count_kernel<1>, dim3(grid), dim3(256), 0, s, str.p, n, ns.p, nd.p); break;
-    case 2: hipLaunchKernelGGL(conn_count_kernel<2>, dim3(grid), dim3(256), 0, s, str.p, n, ns.p, nd.p); break;
-    case 3: hipLaunchKernelGGL(conn_count_kernel<3>, dim3(grid), dim3(256), 0, s, str.p, n, ns.p, nd.p); break;
-    default: hipLaunchKernelGGL(conn_count_kernel<4>, dim3(grid), dim3(256), 0, s, str.p, n, ns.p, nd.p); break;
+    case 1: hipLaunchKernelGGL(conn_count_kernel<1>, dim3(grid), dim3(256), 0, s, str.p, n, ns, nd); break;
+    case 2: hipLaunchKernelGGL(conn_count_kernel<2>, dim3(grid), dim3(256), 0, s, str.p, n, ns, nd); break;
+    case 3: hipLaunchKernelGGL(conn_count_kernel<3>, dim3(grid), dim3(256), 0, s, str.p, n, ns, nd); break;
+    default: hipLaunchKernelGGL(conn_count_kernel<4>, dim3(grid), dim3(256), 0, s, str.p, n, ns, nd); break;
   }
   QPX_HIP(hipGetLastError());
-  std::vector<int> hs(n), hd(n);
-  QPX_HIP(hipMemcpyAsync(hs.data(), ns.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
-  QPX_HIP(hipMemcpyAsync(hd.data(), nd.p, sizeof(int) * n, hipMemcpyDeviceToHost, s));
-  QPX_HIP(hipStreamSynchronize(s));
-  std::vector<int> ps(n + 1), pd(n + 1);
+}
+
+// running sums of the counts (n + 1 each) and their extent
+static void sum_conn(const int *ns, const int *nd, int n, int *ps, int *pd, SpinConn &cc) {
   ps[0] = pd[0] = 0;
   int64_t ts = 0, td = 0;
   cc.max_singles = cc.max_doubles = 0;
   for (int i = 0; i < n; ++i) {
-    ts += hs[i];
-    td += hd[i];
+    ts += ns[i];
+    td += nd[i];
     QPX_REQUIRE(ts < (1LL << 31) && td < (1LL << 31), "spin-string connectivity exceeds 2^31 entries");
     ps[i + 1] = (int)ts;
     pd[i + 1] = (int)td;
-    cc.max_singles = std::max(cc.max_singles, hs[i]);
-    cc.max_doubles = std::max(cc.max_doubles, hd[i]);
+    cc.max_singles = std::max(cc.max_singles, ns[i]);
+    cc.max_doubles = std::max(cc.max_doubles, nd[i]);
   }
   cc.n_singles = ts;
   cc.n_doubles = td;
-  cc.s_ptr.upload(ps, s);
-  cc.d_ptr.upload(pd, s);
-  cc.s_idx.alloc(std::max<int64_t>(ts, 1));
-  cc.s_info.alloc(std::max<int64_t>(ts, 1));
-  cc.s_val.alloc(std::max<int64_t>(ts, 1));
-  cc.s_valf.alloc(std::max<int64_t>(ts, 1));
-  cc.d_idx.alloc(std::max<int64_t>(td, 1));
-  cc.d_val.alloc(std::max<int64_t>(td, 1));
-  cc.d_valf.alloc(std::max<int64_t>(td, 1));
+}
+
+static void fill_conn(qpx_ctx *c, const DBuf<uint64_t> &str, int n, int nint, SpinConn &cc) {
+  hipStream_t s = c->stream;
+  const int grid = (n + 255) / 256;
   Ham &H = c->H;
 #define QPX_FILL(NI)                                                                                        \
   hipLaunchKernelGGL(conn_fill_kernel<NI>, dim3(grid), dim3(256), 0, s, str.p, n, H.M, H.V.p, H.npair,     \
@@ -509,11 +502,40 @@ void ensure_conn(qpx_ctx *c) {
   QPX_REQUIRE(W.valid, "no wavefunction set");
   if (W.conn_valid) return;
   hipStream_t s = c->stream;
-  build_conn(c, W.astr, W.n_a, W.nint, W.ca);
-  build_conn(c, W.bstr, W.n_b, W.nint, W.cb);
+  // both spins share the counts' transfer, the pointers' and the memory
+  const size_t na = W.n_a, nb = W.n_b;
+  W.conn_count.alloc(2 * (na + nb));
+  int *cnt = W.conn_count.p;
+  count_conn(c, W.astr, W.n_a, W.nint, cnt, cnt + na);
+  count_conn(c, W.bstr, W.n_b, W.nint, cnt + 2 * na, cnt + 2 * na + nb);
+  std::vector<int> h(2 * (na + nb)), p(2 * (na + nb) + 4);
+  QPX_HIP(hipMemcpyAsync(h.data(), cnt, sizeof(int) * h.size(), hipMemcpyDeviceToHost, s));
+  QPX_HIP(hipStreamSynchronize(s));
+  sum_conn(h.data(), h.data() + na, W.n_a, p.data(), p.data() + na + 1, W.ca);
+  sum_conn(h.data() + 2 * na, h.data() + 2 * na + nb, W.n_b, p.data() + 2 * (na + 1), p.data() + 2 * (na + 1) + nb + 1, W.cb);
+  View<int> ptrs;
+  W.conn.layout([&] {
+    W.conn.lay(ptrs, p.size());
+    for (SpinConn *q : {&W.ca, &W.cb}) {
+      W.conn.lay(q->s_idx, q->n_singles);
+      W.conn.lay(q->s_info, q->n_singles);
+      W.conn.lay(q->s_val, q->n_singles);
+      W.conn.lay(q->s_valf, q->n_singles);
+      W.conn.lay(q->d_idx, q->n_doubles);
+      W.conn.lay(q->d_val, q->n_doubles);
+      W.conn.lay(q->d_valf, q->n_doubles);
+    }
+    W.conn.lay(W.cost_a, na);
+    W.conn.lay(W.cost_b, nb);
+  });
+  W.ca.s_ptr.p = ptrs.p;
+  W.ca.d_ptr.p = ptrs.p + na + 1;
+  W.cb.s_ptr.p = ptrs.p + 2 * (na + 1);
+  W.cb.d_ptr.p = W.cb.s_ptr.p + nb + 1;
+  QPX_HIP(hipMemcpyAsync(ptrs.p, p.data(), sizeof(int) * p.size(), hipMemcpyHostToDevice, s));
+  fill_conn(c, W.astr, W.n_a, W.nint, W.ca);
+  fill_conn(c, W.bstr, W.n_b, W.nint, W.cb);
   // scan costs: alpha string a -> sum over its alpha singles a' of row length
-  W.cost_a.alloc(W.n_a);
-  W.cost_b.alloc(W.n_b);
   hipLaunchKernelGGL(scan_cost_kernel, dim3((W.n_a + 255) / 256), dim3(256), 0, s, W.ca.s_ptr.p, W.ca.s_idx.p,
                      W.row_ptr.p, W.n_a, W.cost_a.p);
   hipLaunchKernelGGL(scan_cost_kernel, dim3((W.n_b + 255) / 256), dim3(256), 0, s, W.cb.s_ptr.p, W.cb.s_idx.p,

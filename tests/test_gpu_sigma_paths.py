@@ -127,3 +127,24 @@ def test_few_beta_strings(ctx, M, na, nb, nst, prec, kernels):
             assert np.max(np.abs(x - r)) < 1e-11 * max(1.0, np.max(np.abs(r)))
         else:
             assert np.linalg.norm(x - r) < 2e-5 * max(1.0, np.linalg.norm(r))
+
+
+def test_product_spaces_in_turn(ctx):
+    """Tables and connections of one wavefunction are laid out in the memory of
+    the last: spaces of growing and shrinking string sets in one context, with
+    few and with many partners per string, give the bits of a context of their
+    own, in both precisions."""
+    from quantum_package_amd.api import Context
+    spaces = [(8, 4, 4), (4, 4, 2), (12, 4, 3), (6, 3, 1), (14, 6, 1), (8, 4, 4), (2, 1, 1), (12, 5, 3)]
+    for M, na, nb in spaces:
+        dets = fci_space(M, na, nb)
+        _say(f"[sigma in turn] M={M} {na}a{nb}b n_det={dets.shape[0]}")
+        own = Context(0)
+        got = []
+        for c in (ctx, own):
+            u = _set(c, M, na, nb, dets)
+            c._force_sigma_path(1)
+            got.append([x for prec in (0, 1) for x in c.H_S2_u_0_nstates(u, prec=prec)])
+            assert c._sigma_kernels() == STRINGS
+        own.close()
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
