@@ -212,6 +212,11 @@ struct SparseIdx {
 // Tables of the string-driven sigma of product spaces (sigma_fci.hip), built
 // on first use: partners of 16 strings at a time, their matrix elements and
 // the placement tables, per precision.
+struct FciConn {   // connections and elements, for sums that are not finite
+  const int *as_ptr, *as_idx, *ad_ptr, *ad_idx, *bd_ptr, *bd_idx;
+  const uint32_t *as_info;
+  const void *as_val, *ad_val, *bs_val, *bd_val;
+};
 struct SpinTiles {
   int ntile = 0;
   int64_t nchunk = 0;    // room for the partners of all tiles, in chunks of 8
@@ -224,6 +229,7 @@ struct FciTables {
   Block mem;
   View<T> coef_a, coef_b, gb, vo;
   View<uint4> tgt;
+  View<FciConn> conn;
   void release() {
     valid = false;
     mem.release();

@@ -148,6 +148,7 @@ struct TableArgs {
   int64_t n_tgt, n_gb, n_vo;
   uint4 *tgt;
   T *gb, *vo;
+  FciConn conn, *conn_to;
 };
 // packed pair of row: off-diagonal pairs first, then the diagonal ones
 __device__ inline int64_t pair_of_row(int row, int npo) {
@@ -160,6 +161,7 @@ __device__ inline int64_t pair_of_row(int row, int npo) {
 template <typename T>
 __global__ __launch_bounds__(256) void fci_tables_kernel(TableArgs<T> A) {
   const int64_t n = A.n_tgt + A.n_gb + A.n_vo;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *A.conn_to = A.conn;
   for (int64_t y = blockIdx.x * (int64_t)256 + threadIdx.x; y < n; y += (int64_t)gridDim.x * 256) {
     int64_t x = y;
     if (x < A.n_tgt) {
@@ -419,6 +421,7 @@ struct FciArgs {
   const uint64_t *astr;
   const uint32_t *map_a, *map_b;
   const double *hdiag, *sdiag;
+  const FciConn *conn;
   const void *vo, *gbs;   // integrals of off-diagonal pairs with all pairs [npo][nr]; Coulomb sums of the beta strings [n_b][npo]
   int n_a, n_b, lda, ldt, npo, nr, mt, nst, nrow;   // nrow: wavefronts per state, each with every nrow-th pair tile
   template <typename T>
@@ -426,6 +429,39 @@ struct FciArgs {
   template <typename T>
   __device__ const T *Gb() const { return static_cast<const T *>(gbs); }
 };
+
+// v(a, b) of state st, connected determinant by connected determinant.  The
+// products multiply an infinity or NaN of u by the zeros of elements that are
+// not there; a sum that came out not finite is formed again from those that are.
+template <typename T>
+__device__ __forceinline__ double fci_element(const FciArgs &A, int b, int a, int st, const T *__restrict__ u) {
+  auto at = [&](int bb, int aa) { return (double)u[((int64_t)bb * A.n_a + aa) * A.nst + st]; };
+  auto val = [](const void *x, int e) { return (double)static_cast<const T *>(x)[e]; };
+  const FciConn C = *A.conn;
+  const T *vo = A.Vo<T>(), *gb = A.Gb<T>() + (int64_t)b * A.npo;
+  double t = A.hdiag[(int64_t)b * A.n_a + a] * at(b, a);
+  for (int e = C.ad_ptr[a]; e < C.ad_ptr[a + 1]; ++e) t += val(C.ad_val, e) * at(b, C.ad_idx[e]);
+  for (int e = C.bd_ptr[b]; e < C.bd_ptr[b + 1]; ++e) t += val(C.bd_val, e) * at(C.bd_idx[e], a);
+  for (int e = C.as_ptr[a]; e < C.as_ptr[a + 1]; ++e) {
+    const uint32_t inf = C.as_info[e];
+    const double g = (double)gb[off_pair(inf & 0xff, (inf >> 8) & 0xff)];
+    t += (val(C.as_val, e) + ((inf >> 16) & 1 ? -g : g)) * at(b, C.as_idx[e]);
+  }
+  for (int f = A.bs_ptr[b]; f < A.bs_ptr[b + 1]; ++f) {
+    const uint32_t inf = A.bs_info[f];
+    const T *row = vo + (int64_t)off_pair(inf & 0xff, (inf >> 8) & 0xff) * A.nr;
+    const uint32_t neg = (inf >> 16) & 1;
+    double g = 0.0;
+    for (uint64_t y = A.astr[a]; y; y &= y - 1) g += (double)row[A.npo + __ffsll((unsigned long long)y) - 1];
+    t += (val(C.bs_val, f) + (neg ? -g : g)) * at(A.bs_idx[f], a);
+    for (int e = C.as_ptr[a]; e < C.as_ptr[a + 1]; ++e) {
+      const uint32_t ia = C.as_info[e];
+      const double h = (double)row[off_pair(ia & 0xff, (ia >> 8) & 0xff)];
+      t += (neg ^ ((ia >> 16) & 1) ? -h : h) * at(A.bs_idx[f], C.as_idx[e]);
+    }
+  }
+  return t;
+}
 
 // One workgroup per beta string b; wavefront w < nst nrow owns state w % nst
 // and the pair tiles w / nst, w / nst + nrow, ... and adds into a column of
@@ -700,7 +736,9 @@ __global__ __launch_bounds__(512, 2) void sigma_fci_ab_kernel(FciArgs A, const T
       if (st < A.nst) {
         double t = 0.0;
         for (int r = 0; r < A.nrow; ++r) t += col[(size_t)(r * A.nst + st) * ldc + a];
-        v[e * A.nst + st] = (T)(t + (double)yy[st] + (double)(hd * uu[st]));
+        t += (double)yy[st] + (double)(hd * uu[st]);
+        if (!isfinite(t)) t = fci_element<T>(A, b, a, st, u);
+        v[e * A.nst + st] = (T)t;
       }
   }
 }
@@ -823,13 +861,18 @@ void build_tables(qpx_ctx *c) {
     t.mem.lay(t.tgt, (size_t)mt * P.ldt * 4);
     t.mem.lay(t.gb, (size_t)npo * W.n_b);
     t.mem.lay(t.vo, (size_t)npo * nr);
+    t.mem.lay(t.conn, 1);
   });
   const SpinArgs a = spin_args(W.ca, W.n_a, P.a, 0, P.map_a), b = spin_args(W.cb, W.n_b, P.b, 0, P.map_b);
   hipLaunchKernelGGL(fci_coef_kernel<T>, dim3(P.a.ntile + P.b.ntile), dim3(256), 0, s, a,
                      CoefArgs<T>{Prec<T>::sval(W.ca), Prec<T>::dval(W.ca), t.coef_a.p}, b,
                      CoefArgs<T>{Prec<T>::sval(W.cb), Prec<T>::dval(W.cb), t.coef_b.p});
   const TableArgs<T> A{P.map_a.p, W.astr.p, W.bstr.p, Prec<T>::V(c->H), W.n_a, W.n_b, P.ldt, M, npo, nr, c->H.npair,
-                       (int64_t)mt * P.ldt * 4, (int64_t)npo * W.n_b, (int64_t)npo * nr, t.tgt.p, t.gb.p, t.vo.p};
+                       (int64_t)mt * P.ldt * 4, (int64_t)npo * W.n_b, (int64_t)npo * nr, t.tgt.p, t.gb.p, t.vo.p,
+                       FciConn{W.ca.s_ptr.p, W.ca.s_idx.p, W.ca.d_ptr.p, W.ca.d_idx.p, W.cb.d_ptr.p, W.cb.d_idx.p,
+                               W.ca.s_info.p, Prec<T>::sval(W.ca), Prec<T>::dval(W.ca), Prec<T>::sval(W.cb),
+                               Prec<T>::dval(W.cb)},
+                       t.conn.p};
   hipLaunchKernelGGL(fci_tables_kernel<T>, dim3((unsigned)std::min<int64_t>((A.n_tgt + A.n_gb + A.n_vo + 255) / 256, 4096)),
                      dim3(256), 0, s, A);
   QPX_HIP(hipGetLastError());
@@ -846,7 +889,7 @@ void launch_ab(qpx_ctx *c, const Shape &S, int nst, const T *pb, T *y, const T *
   // two of KS integrals leave of the 256 registers
   constexpr int NT = KS * (int)sizeof(T) <= (sizeof(T) == 8 ? 16 : 40) ? 4 : KS * (int)sizeof(T) <= 96 ? 2 : 1;
   FciArgs A{W.bstr.p, W.cb.s_ptr.p, W.cb.s_idx.p, W.cb.s_info.p, t.tgt.p, W.astr.p, P.map_a.p,
-            P.map_b.p, W.hdiag.p, W.sdiag.p, t.vo.p, t.gb.p, W.n_a, W.n_b, P.lda, P.ldt,
+            P.map_b.p, W.hdiag.p, W.sdiag.p, t.conn.p, t.vo.p, t.gb.p, W.n_a, W.n_b, P.lda, P.ldt,
             c->H.M * (c->H.M - 1) / 2, c->H.M * (c->H.M + 1) / 2, S.mt, nst, S.nrow};
   auto k = sigma_fci_ab_kernel<T, KS, NT>;
   QPX_HIP(hipFuncSetAttribute((const void *)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S.lds));

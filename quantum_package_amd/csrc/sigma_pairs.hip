@@ -707,6 +707,63 @@ __global__ __launch_bounds__(256) void pair_singles_kernel(SingleArgs A, int64_t
   for (int st = 0; st < NST; ++st) part[p * NST + st] = (T)flip(acc[st], own & kSign);
 }
 
+// what a sum that is not finite is formed again from
+template <typename T>
+struct EntryTable {
+  const uint2 *ent;
+  const uint32_t *off;
+  const int2 *wave;
+  const T *tab;
+  int64_t n_dbl;
+  int M, npo;
+  uint32_t tab2;
+};
+
+// Sum of the off-diagonal terms of a determinant's state, without the pairs that
+// are not connected: the doubles kernel multiplies an infinity or NaN of u by
+// their zeros.
+template <typename T, int NST>
+__device__ __forceinline__ double entry_sums(const EntryTable<T> &E, const int *sp, int S, const T *__restrict__ u,
+                                             const T *__restrict__ part, int st) {
+  auto split = [](uint32_t r, uint32_t *p, uint32_t *q) {   // pair r = (p < q)
+    uint32_t t = 1;
+    while ((t + 1) * t / 2 <= r) ++t;
+    *q = t;
+    *p = r - t * (t - 1) / 2;
+  };
+  double sum = 0.0;
+  for (int t = 0; t < S; ++t) {
+    const int at = sp[t];
+    if (at < 0) continue;
+    double x = (double)part[(int64_t)at * NST + st];
+    if (at < E.n_dbl && !isfinite(x)) {
+      const int2 d = E.wave[at >> 6];
+      const int first = d.y >= 64 ? d.x : at - (at & 63) % d.y;
+      const uint32_t own = E.ent[at].x, off = E.off[at], M = (uint32_t)E.M, M2 = M * M;
+      const bool ab = E.ent[at].y < E.tab2;
+      uint32_t i = off % M, j = off / M;
+      if (!ab) split(off, &i, &j);
+      x = 0.0;
+      for (int n = first; n < first + d.y; ++n) {
+        const uint2 e = E.ent[n];
+        uint32_t a, b;
+        if (ab) {
+          a = e.y / (M2 * M);
+          b = e.y / M2 % M;
+          if (a == i || b == j) continue;
+        } else {
+          split((e.y - E.tab2) / (uint32_t)E.npo, &a, &b);
+          if (a == i || a == j || b == i || b == j) continue;
+        }
+        x += (double)E.tab[e.y + off] * (double)flip(u[(int64_t)(e.x & ~kSign) * NST + st], e.x & kSign);
+      }
+      x = flip(x, own & kSign);
+    }
+    sum += x;
+  }
+  return sum;
+}
+
 // v and s of a determinant: 16 lanes add its entries' sums, slots l, l + 16,
 // ..., then a fixed tree.  In FP64 in both precisions: an FP32 call's error
 // would otherwise be that of hundreds of sums and of the list of spin exchanges
@@ -717,7 +774,7 @@ __global__ __launch_bounds__(256) void pair_collect_kernel(const int *__restrict
                                                            const uint32_t *__restrict__ xlist,
                                                            const double *__restrict__ hdiag,
                                                            const double *__restrict__ sdiag, const T *__restrict__ u,
-                                                           T *__restrict__ v, T *__restrict__ s) {
+                                                           EntryTable<T> E, T *__restrict__ v, T *__restrict__ s) {
   const int64_t k = blockIdx.x * (int64_t)16 + (threadIdx.x >> 4);
   const int l = threadIdx.x & 15;
   const bool on = k < n;
@@ -746,7 +803,11 @@ __global__ __launch_bounds__(256) void pair_collect_kernel(const int *__restrict
 #pragma unroll
   for (int st = 0; st < NST; ++st) {
     const double x = (double)u[k * NST + st];
-    if (l == st) v[k * NST + st] = (T)(acc[st] + hdiag[k] * x);
+    if (l == st) {
+      double t = acc[st];
+      if (!isfinite(t)) t = entry_sums<T, NST>(E, slotpos + k * S, S, u, part, st);
+      v[k * NST + st] = (T)(t + hdiag[k] * x);
+    }
     if (l == 8 + st) {
       double t = sdiag[k] * x;
       for (int q = xptr[k]; q < xptr[k + 1]; ++q) {
@@ -989,8 +1050,10 @@ void launch(qpx_ctx *c, char *ws, const T *tab, const double *fock, const T *u, 
     hipLaunchKernelGGL((pair_singles_kernel<T, NI, NST>), dim3((unsigned)(ns / 256)), dim3(256), 0, st, A, X.n_dbl,
                        X.ent.p, X.off.p, X.wave.p, fock, GS, GO, u, part);
   }
+  const int M = c->H.M;
+  const EntryTable<T> E{X.ent.p, X.off.p, X.wave.p, tab, X.n_dbl, M, M * (M - 1) / 2, (uint32_t)((int64_t)M * M * M * M)};
   hipLaunchKernelGGL((pair_collect_kernel<T, NST>), dim3((unsigned)((W.n_det + 15) / 16)), dim3(256), 0, st, X.slotpos.p,
-                     X.S, W.n_det, part, X.xptr.p, X.xlist.p, W.hdiag.p, W.sdiag.p, u, v, s);
+                     X.S, W.n_det, part, X.xptr.p, X.xlist.p, W.hdiag.p, W.sdiag.p, u, E, v, s);
   QPX_HIP(hipGetLastError());
 }
 

@@ -148,3 +148,27 @@ def test_product_spaces_in_turn(ctx):
             assert c._sigma_kernels() == STRINGS
         own.close()
         assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+@pytest.mark.parametrize("prec", [0, 1])
+@pytest.mark.parametrize("kind,arg", [("product", (8, 4, 4, 0.0)), ("product", (12, 3, 2, 0.4)), ("product", (14, 6, 1, 0.0)),
+                                      ("buckets", (20, 3, 2, 0.9)), ("buckets", (14, 3, 2, 0.7)), ("buckets", (70, 2, 1, 0.25))])
+def test_infinities_stay_where_they_are(ctx, kind, arg, prec, bad):
+    """An infinite or NaN entry of u reaches the determinants connected to its
+    own and no others, and one state only, as with the scanning kernel; the
+    other entries keep their values (FP64: 1e-11, FP32: 2e-5 of the largest)."""
+    M, na, nb, x = arg
+    dets = _product_space(M, na, nb, x, 7) if kind == "product" else _singles_space(M, na, nb, x, M + 1)
+    u = _set(ctx, M, na, nb, dets)
+    u[dets.shape[0] // 3, 0] = bad
+    _say(f"[sigma not finite] {kind} M={M} {na}a{nb}b prec={prec} {bad} n_det={dets.shape[0]}")
+    ctx._force_sigma_path(SCAN)
+    want = ctx.H_S2_u_0_nstates(u)
+    ctx._force_sigma_path(1 if kind == "product" else 3)
+    got = ctx.H_S2_u_0_nstates(u, prec=prec)
+    assert ctx._sigma_kernels() == (STRINGS if kind == "product" else BUCKET)
+    for x, r in zip(got, want):
+        ok = np.isfinite(r)
+        assert np.array_equal(np.isfinite(x), ok) and not ok.all()
+        assert np.max(np.abs(x[ok] - r[ok])) < (1e-11 if prec == 0 else 2e-5) * np.max(np.abs(r[ok]))
