@@ -70,8 +70,22 @@ int qpx_sigma(qpx_ctx *ctx, int prec, int n_st, int64_t sze, const double *u, do
  * memory: u_t, v_t, s_t are (n_st, n_det) state-fastest in the context's
  * bilinear (beta-column-major) order, of type double (QPX_FP64) or float
  * (QPX_FP32).  v_t and s_t are overwritten.  stream may be NULL (the
- * context's stream). */
+ * context's stream).
+ * The call may be captured into a graph, also as the first one of a
+ * wavefunction or precision; the graph is valid until the next
+ * qpx_set_hamiltonian or qpx_set_wavefunction.  Calls of one context on
+ * different streams share scratch memory and run one after another (contexts
+ * do not wait for each other).  A captured call has scratch of its own, so its
+ * replays may run beside other calls, but the executables made from one capture
+ * share it and must not run at once. */
 int qpx_sigma_device(qpx_ctx *ctx, int prec, int n_st, const void *u_t, void *v_t, void *s_t, void *stream);
+
+/* Gives back the scratch memory of the captured sigma calls of the context
+ * (up to about the size of a call's u, v and s each for full-CI spaces, several
+ * times that for selected ones); for programs that capture again and again
+ * between two wavefunctions.  Waits for the device.  The graphs captured before
+ * must not be replayed any more.  No counterpart in the reference. */
+int qpx_release_captured(qpx_ctx *ctx);
 
 /* Permutation of the context's bilinear order: perm[k] = psi_det index
  * (0-based) of bilinear position k (psi_bilinear_matrix_order - 1). */

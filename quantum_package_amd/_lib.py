@@ -29,6 +29,7 @@ SIGNATURES = [
     ("qpx_set_wavefunction", C.c_int, [c_vp, C.c_int, C.c_int64, c_u64p]),
     ("qpx_sigma", C.c_int, [c_vp, C.c_int, C.c_int, C.c_int64, c_dp, c_dp, c_dp]),
     ("qpx_sigma_device", C.c_int, [c_vp, C.c_int, C.c_int, c_vp, c_vp, c_vp, c_vp]),
+    ("qpx_release_captured", C.c_int, [c_vp]),
     ("qpx_get_bilinear_order", C.c_int, [c_vp, c_i64p]),
     ("qpx_diag_h", C.c_int, [c_vp, c_dp]),
     ("qpx_davidson", C.c_int, [c_vp, C.c_int, C.c_int, C.c_double, C.c_int, C.c_int, C.c_int, C.c_int,

@@ -101,6 +101,11 @@ class Context:
             return v[:, 0], s[:, 0]
         return v, s
 
+    def release_captured(self):
+        """Gives back the scratch of sigma calls captured into graphs, which must
+        not be replayed any more."""
+        self._check(self.L.qpx_release_captured(self.ptr))
+
     def u_0_H_u_0(self, u_0, prec: int = FP64):
         """e_0 = <u_0|H|u_0> per state (no division by the norm when it is
         nonzero, as the reference)."""

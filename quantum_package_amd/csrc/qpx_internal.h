@@ -350,8 +350,10 @@ struct StreamWorkspace {
     if (done) (void)hipEventDestroy(done);
   }
   // A captured graph owns its scratch (one buffer per capture and stream, till
-  // the wavefunction it was captured for goes): it may be replayed on any
-  // stream, beside other calls and after calls that need more.
+  // the wavefunction it was captured for goes or qpx_release_captured): it may be
+  // replayed on any stream, beside other calls and after calls that need more.
+  // The runtime tells nobody that a graph is gone: a user object retained by one
+  // is not released with its last executable.
   struct Captured {
     hipStream_t s;
     unsigned long long id;

@@ -823,6 +823,15 @@ extern "C" int qpx_sigma_device(qpx_ctx *c, int prec, int nst, const void *u_t, 
   });
 }
 
+extern "C" int qpx_release_captured(qpx_ctx *c) {
+  return qpx_guard(c, [&] {
+    QPX_HIP(hipSetDevice(c->device));
+    QPX_HIP(hipDeviceSynchronize());   // replays that still run
+    c->ws_fci.graphs.clear();
+    c->ws_pairs.graphs.clear();
+  });
+}
+
 // LDS read bandwidth of the device: every lane of 1024-thread workgroups
 // (two per CU, 64 KiB of LDS each) reads 16 bytes per iteration from LDS, in
 // the conflict-free pattern (consecutive lanes, consecutive 16-byte words),

@@ -294,3 +294,33 @@ def test_calls_on_per_thread_streams(ctx, hip, kind, path):
     for x, want in zip(xs, alone):
         assert _same(x.out(), want)
         x.free()
+
+
+@pytest.mark.parametrize("kind,path", [("product", 1), ("selected", 3)])
+def test_released_captures_give_their_memory_back(ctx, hip, kind, path):
+    """A program that captures again and again holds no more memory than one
+    capture needs; later captures replay as the first."""
+    n = _prepare(ctx, kind)
+    ctx._force_sigma_path(path)
+    st = hip.stream()
+    x = Vectors(hip, n, 4, 0, 1)
+    x.sigma(ctx, st)
+    hip.sync()
+    want = x.out()
+
+    def round_trip():
+        g = hip.capture(st, lambda: x.sigma(ctx, st))
+        x.clear()
+        hip.replay(g, st)
+        hip.sync()
+        assert _same(x.out(), want)
+        hip.drop(g)
+        ctx.release_captured()
+
+    round_trip()
+    free = hip.free_bytes()
+    _say(f"[sigma captures] {kind} n_det={n}")
+    for _ in range(100):   # 100 scratch buffers: 240 MB for the product space, tens of MB for the other
+        round_trip()
+    assert free - hip.free_bytes() < 8 << 20
+    x.free()
