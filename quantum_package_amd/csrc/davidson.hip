@@ -488,9 +488,10 @@ extern "C" int qpx_davidson(qpx_ctx *c, int N_st, int N_st_diag, double threshol
     S.alloc((size_t)n * nc);
     uin_d.alloc((size_t)n * N_st_diag);
     host_io.alloc((size_t)n * N_st_diag);
-    // the caller's N_st guess vectors and random ones behind them, normalised
-    QPX_HIP(hipMemcpy2DAsync(host_io.p, sizeof(double) * n, u_in, sizeof(double) * dim_in, sizeof(double) * n, N_st,
-                             hipMemcpyHostToDevice, st));
+    // the caller's N_st guess vectors and random ones behind them, normalised;
+    // copied column by column: a 2D copy's pitch ends at 2^31 - 1 bytes, 268M rows
+    for (int k = 0; k < N_st; ++k)
+      QPX_HIP(hipMemcpyAsync(host_io.p + n * k, u_in + dim_in * k, sizeof(double) * n, hipMemcpyHostToDevice, st));
     int gridp = (int)std::min<int64_t>((n * N_st_diag + 255) / 256, 65536);
     hipLaunchKernelGGL(guess_kernel, dim3(gridp), dim3(256), 0, st, host_io.p, n, N_st, seed, Wf.perm_d.p, n,
                        N_st_diag, uin_d.p);
@@ -672,8 +673,8 @@ extern "C" int qpx_davidson(qpx_ctx *c, int N_st, int N_st_diag, double threshol
     hipLaunchKernelGGL(permute_out_kernel, dim3(gridp), dim3(256), 0, st, uin_d.p, n, Wf.perm_d.p, n, N_st_diag,
                        host_io.p, n);
     QPX_HIP(hipGetLastError());
-    QPX_HIP(hipMemcpy2DAsync(u_in, sizeof(double) * dim_in, host_io.p, sizeof(double) * n, sizeof(double) * n, N_st_diag,
-                             hipMemcpyDeviceToHost, st));
+    for (int k = 0; k < N_st_diag; ++k)
+      QPX_HIP(hipMemcpyAsync(u_in + dim_in * k, host_io.p + n * k, sizeof(double) * n, hipMemcpyDeviceToHost, st));
     QPX_HIP(hipStreamSynchronize(st));
     for (int k = 0; k < N_st_diag; ++k) {
       energies[k] = lambda[k];
