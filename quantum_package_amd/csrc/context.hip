@@ -74,8 +74,8 @@ bool ensure_g4(qpx_ctx *c) {
   if (H.M > kG4MaxOrb) return false;
   if (H.G4.p) return true;
   const int64_t n4 = (int64_t)H.M * H.M * H.M * H.M;
-  H.G4.alloc(n4);
   H.G4f.alloc(n4);
+  H.G4.alloc(n4);   // the larger one last: where it fits, both are there
   hipLaunchKernelGGL(g4_fill_kernel, dim3((unsigned)std::min<int64_t>((n4 + 255) / 256, 1 << 16)), dim3(256), 0,
                      c->stream, H.V.p, H.M, H.npair, H.G4.p, H.G4f.p);
   QPX_HIP(hipGetLastError());
@@ -147,6 +147,7 @@ extern "C" int qpx_set_hamiltonian(qpx_ctx *c, int M, int na, int nb, const doub
     QPX_REQUIRE(n8 == npair * (npair + 1) / 2, "eri_packed length must be npair*(npair+1)/2");
     // sigma calls enqueued on a caller's stream may still read the integrals
     QPX_HIP(hipDeviceSynchronize());
+    c->ham_set = c->W.valid = false;   // until every array below is there
     Ham &H = c->H;
     H.M = M;
     H.na = na;
@@ -229,6 +230,5 @@ extern "C" int qpx_set_hamiltonian(qpx_ctx *c, int M, int na, int nb, const doub
     H.G4f.release();
     H.release_pair_tables();
     c->ham_set = true;
-    c->W.valid = false;
   });
 }

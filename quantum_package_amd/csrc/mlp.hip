@@ -730,6 +730,7 @@ constexpr int kChunks = 64;      // most row chunks of a column sum
 
 void ensure(qpx_mlp *m, int n) {
   if (n <= m->cap) return;
+  m->cap = 0;   // should one of the allocations fail
   m->desc.alloc((size_t)4 * n);
   m->fdesc.alloc((size_t)3 * n);
   m->tgt.alloc(n);
@@ -740,6 +741,7 @@ void ensure(qpx_mlp *m, int n) {
 void ensure_train(qpx_mlp *m, int n) {
   ensure(m, n);
   if (n <= m->tcap) return;
+  m->tcap = 0;
   const int Hd = m->hid;
   m->Xb.alloc((size_t)n * m->din);
   for (DBuf<uint16_t> *b : {&m->H1b, &m->H2b, &m->dZ1b, &m->dZ2b, &m->dZ3b}) b->alloc((size_t)n * Hd);
