@@ -7,6 +7,7 @@ import numpy as np
 import pytest
 
 from quantum_package_amd.hamiltonian import Hamiltonian, fci_space, hf_determinant, synthetic_hamiltonian
+from oracle import oracle as O
 from test_gpu_sigma import BUCKETS, PRODUCT, _product_space, _random_space, _say, _singles_space
 
 pytestmark = pytest.mark.gpu
@@ -172,3 +173,40 @@ def test_infinities_stay_where_they_are(ctx, kind, arg, prec, bad):
         ok = np.isfinite(r)
         assert np.array_equal(np.isfinite(x), ok) and not ok.all()
         assert np.max(np.abs(x[ok] - r[ok])) < (1e-11 if prec == 0 else 2e-5) * np.max(np.abs(r[ok]))
+
+
+def _against_oracle(ctx, M, na, nb, dets, nst, path, kernels):
+    """FP64 to 1e-11 of the largest entry, FP32 to 2e-5 of the norm"""
+    H = synthetic_hamiltonian(M, na, nb, seed=77)
+    ctx.set_hamiltonian(H)
+    ctx.set_wavefunction(dets)
+    u = np.random.default_rng(5).standard_normal((dets.shape[0], nst))
+    want = O.sigma(O.Ham(H), O.Bilinear(dets), u)
+    ctx._force_sigma_path(path)
+    for prec in (0, 1):
+        for x, r in zip(ctx.H_S2_u_0_nstates(u, prec=prec), want):
+            if prec == 0:
+                assert np.max(np.abs(x - r)) < 1e-11 * max(1.0, np.max(np.abs(r)))
+            else:
+                assert np.linalg.norm(x - r) < 2e-5 * max(1.0, np.linalg.norm(r))
+        assert ctx._sigma_kernels() == kernels
+
+
+# by the most alpha singles a string has: up to 48, 64 and 96, and sets that are
+# no product space, which the automatic path sends to the dense map
+@pytest.mark.parametrize("M,na,nb,n,nst,path", [
+    (8, 4, 4, None, 4, 4), (14, 3, 3, None, 4, 4), (24, 3, 1, None, 4, 4), (30, 3, 1, None, 1, 4),
+    (12, 4, 4, 3000, 3, 4), (12, 4, 4, 3000, 2, 0)])
+def test_dense_map_kernels(ctx, M, na, nb, n, nst, path):
+    dets = fci_space(M, na, nb) if n is None else _random_space(M, na, nb, n, 7)
+    _say(f"[dense map] M={M} {na}a{nb}b nst={nst} path={path} n_det={dets.shape[0]}")
+    _against_oracle(ctx, M, na, nb, dets, nst, path, DENSE)
+
+
+@pytest.mark.parametrize("M,ne,nst", [(17, 8, 1), (17, 8, 4), (19, 9, 2), (19, 9, 4)])
+def test_string_driven_kernels_of_many_singles(ctx, M, ne, nst):
+    """72 and 90 beta singles of a string (20 and 24 steps of four): the first
+    string and its single excitations, of both spins."""
+    dets = _singles_space(M, ne, ne, 2.0, 1)
+    _say(f"[sigma many singles] M={M} {ne}a{ne}b nst={nst} n_det={dets.shape[0]}")
+    _against_oracle(ctx, M, ne, ne, dets, nst, 1, STRINGS)
