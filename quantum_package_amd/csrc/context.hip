@@ -146,7 +146,7 @@ extern "C" int qpx_set_hamiltonian(qpx_ctx *c, int M, int na, int nb, const doub
     int64_t npair = (int64_t)M * (M + 1) / 2;
     QPX_REQUIRE(n8 == npair * (npair + 1) / 2, "eri_packed length must be npair*(npair+1)/2");
     // sigma calls enqueued on a caller's stream may still read the integrals
-    QPX_HIP(hipDeviceSynchronize());
+    wait_device();
     c->ham_set = c->W.valid = false;   // until every array below is there
     Ham &H = c->H;
     H.M = M;

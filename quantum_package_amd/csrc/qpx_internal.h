@@ -56,6 +56,15 @@ inline void device_alloc(void **p, size_t bytes) {
   QPX_HIP(e);
 }
 
+// Waits for the device.  hipDeviceSynchronize would fail while any thread of the
+// process captures a stream, and break its capture; hipFree, which waits too, is
+// refused only where an allocation is (a capture in the global mode).
+inline void wait_device() {
+  void *p = nullptr;
+  device_alloc(&p, 256);
+  QPX_HIP(hipFree(p));
+}
+
 // What a context keeps of one wavefunction's arrays and scratch for the next, of
 // the bucket kernels and of the string-driven ones; more costs less to allocate
 // again than the set-up it serves (some 10^8 entries to sort).

@@ -826,7 +826,7 @@ extern "C" int qpx_sigma_device(qpx_ctx *c, int prec, int nst, const void *u_t, 
 extern "C" int qpx_release_captured(qpx_ctx *c) {
   return qpx_guard(c, [&] {
     QPX_HIP(hipSetDevice(c->device));
-    QPX_HIP(hipDeviceSynchronize());   // replays that still run
+    wait_device();   // replays that still run
     c->ws_fci.graphs.clear();
     c->ws_pairs.graphs.clear();
   });

@@ -343,7 +343,7 @@ void build_wavefunction(qpx_ctx *c, int nint, int64_t n_det, const uint64_t *psi
   W.valid = false;
   // sigma calls enqueued on a caller's stream may still read the arrays below,
   // which are overwritten on the context's stream
-  QPX_HIP(hipDeviceSynchronize());
+  wait_device();
   W.sp.clear();
   W.fci.clear();
   W.pr.clear();

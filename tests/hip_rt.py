@@ -7,7 +7,7 @@ import ctypes as C
 import numpy as np
 
 NON_BLOCKING = 1
-CAPTURE_GLOBAL = 0
+CAPTURE_GLOBAL, CAPTURE_THREAD_LOCAL = 0, 1
 
 
 class Hip:
@@ -32,9 +32,9 @@ class Hip:
         self.call("hipStreamCreateWithFlags", C.byref(s), C.c_uint(NON_BLOCKING))
         return s
 
-    def capture(self, stream, enqueue):
+    def capture(self, stream, enqueue, mode=CAPTURE_GLOBAL):
         """The executable graph of what enqueue() puts on the stream."""
-        self.call("hipStreamBeginCapture", stream, C.c_int(CAPTURE_GLOBAL))
+        self.call("hipStreamBeginCapture", stream, C.c_int(mode))
         graph, ex = C.c_void_p(), C.c_void_p()
         try:
             enqueue()

@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from quantum_package_amd.hamiltonian import fci_space, synthetic_hamiltonian
-from hip_rt import Arr, Hip
+from hip_rt import CAPTURE_THREAD_LOCAL, Arr, Hip
 from test_gpu_sigma import _say, _singles_space
 from test_gpu_sigma_paths import failing_allocations
 
@@ -323,4 +323,43 @@ def test_released_captures_give_their_memory_back(ctx, hip, kind, path):
     for _ in range(100):   # 100 scratch buffers: 240 MB for the product space, tens of MB for the other
         round_trip()
     assert free - hip.free_bytes() < 8 << 20
+    x.free()
+
+
+def test_set_up_beside_a_capture(ctx, hip):
+    """Another thread sets up a context of its own, runs it and gives captures
+    back while this one captures in the thread-local mode: both work."""
+    from quantum_package_amd.api import Context
+    n = _prepare(ctx, "product")
+    x, st = Vectors(hip, n, 1, 0, 1), hip.stream()
+    x.sigma(ctx, st)
+    hip.sync()
+    want = x.out()
+    M, na, nb, dets = _space("selected")
+    u = np.random.default_rng(2).standard_normal(dets.shape[0])
+    got = []
+
+    def other():
+        c = Context(0)
+        for _ in range(2):
+            c.set_hamiltonian(synthetic_hamiltonian(M, na, nb, seed=4))
+            c.set_wavefunction(dets)
+            c._force_sigma_path(3)
+            got.append(c.H_S2_u_0_nstates(u))
+            c.release_captured()
+        c.close()
+
+    def enqueue():
+        x.sigma(ctx, st)
+        t = threading.Thread(target=other)
+        t.start()
+        t.join()
+
+    _say(f"[sigma beside a capture] n_det={n}")
+    g = hip.capture(st, enqueue, CAPTURE_THREAD_LOCAL)
+    x.clear()
+    hip.replay(g, st)
+    hip.sync()
+    assert _same(x.out(), want) and len(got) == 2 and _same(got[0], got[1])
+    hip.drop(g)
     x.free()
