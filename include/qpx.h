@@ -62,8 +62,9 @@ int qpx_set_wavefunction(qpx_ctx *ctx, int n_int, int64_t n_det, const uint64_t 
  * v = H u, s = S^2 u for n_st vectors.  u, v, s are (sze, n_st)
  * column-major in psi_det order, sze >= n_det.  u is not modified (the
  * reference permutes it in place and restores it).  prec = QPX_FP64 or
- * QPX_FP32 (FP32 u, integrals and accumulation; results returned as
- * double). */
+ * QPX_FP32 (FP32 u and integrals, sums in FP32 or FP64 by path; results
+ * returned as double).  Non-finite entries of u reach the determinants
+ * connected to theirs and no others. */
 int qpx_sigma(qpx_ctx *ctx, int prec, int n_st, int64_t sze, const double *u, double *v, double *s);
 
 /* H_S2_u_0_nstates_openmp_work (src/Davidson/u0Hu0.irp.f:69-96) on device

@@ -38,15 +38,15 @@ int qpx_debug_fail_alloc(int64_t above, int hip_error);
 /* One qpx_sigma_device call per repetition on `stream`; ms (2) receives the
  * average duration of its two kernel phases (string-driven path: same-spin
  * kernels, alpha/beta kernel; dense path: column kernel, row kernel; sparse
- * path: the bucket kernel, 0), measured with HIP events on
+ * paths and scan: the whole call, 0), measured with HIP events on
  * that stream. */
 int qpx_debug_sigma_kernel_times(qpx_ctx *ctx, int prec, int n_st, const void *u_t, void *v_t, void *s_t,
                                  void *stream, float *ms, int reps);
 
 /* LDS read bandwidth of the context's device (bytes/s): two 1024-thread
  * workgroups per CU read 16 bytes per lane per iteration from LDS in the
- * conflict-free pattern, timed with HIP events (the peak the dense-map
- * sigma kernel's LDS roofline is quoted against). */
+ * conflict-free pattern, timed with HIP events (the bound of the dense-map
+ * sigma kernels). */
 int qpx_debug_lds_bandwidth(qpx_ctx *ctx, double *bytes_per_s);
 
 /* Entries the sparse sigma walk visits per call in each bucket class (sum
@@ -59,8 +59,8 @@ int qpx_debug_sparse_stats(qpx_ctx *ctx, int64_t *visited);
  * must equal that call's block count. */
 int qpx_debug_select_block_ticks(qpx_ctx *ctx, int64_t *ticks, int64_t n);
 
-/* C (M x N) = bf16(A) bf16(B) through the network's GEMM kernel with A
- * stored transposed (ta = 1, K x M row-major) and/or B transposed (tb = 1,
+/* C (M x N) = bf16(A) bf16(B) through the tile of the network's weight
+ * gradients with A stored transposed (ta = 1, K x M row-major) and/or B transposed (tb = 1,
  * N x K) and the split-K path forced (split = 1). */
 int qpx_debug_mlp_gemm(qpx_mlp *mlp, int M, int N, int K, const float *A, const float *B, int ta, int tb, int split,
                        float *C);

@@ -21,7 +21,9 @@
 // their slices and makes the Adam step.  It was 28 launches, with every activation and its
 // gradient written and read in FP32 and bf16: 235 us a step at batch 4096.
 //
-// GEMM: C(MxN) = A(MxK) B(KxN), A and B bf16 with arbitrary row/column
+// The weight gradients' product (gemm_tile, launched by grad_kernel; the plain
+// GEMM around it serves the checks of the tile's lane layout):
+// C(MxN) = A(MxK) B(KxN), A and B bf16 with arbitrary row/column
 // strides (so A^T, B^T need no copies), C fp32; workgroup tile 64x64, four
 // wavefronts each owning 32x32 = 2x2 tiles of v_mfma_f32_16x16x32_bf16
 // (CDNA4's bf16 MFMA with K = 32, one per tile and K-tile of 32).
@@ -688,9 +690,12 @@ struct qpx_mlp {
 
 namespace {
 
-// C = A B.  With a workspace, a product whose tile grid
-// leaves most CUs idle and whose K is long (the weight gradients, K = batch)
-// is cut along K across workgroups and reduced in slice order.
+// C = A B by the weight gradients' tile, in every operand layout the tile can
+// stage; the network itself launches the tile from grad_kernel, with runs along
+// i and j and slices that adam_kernel sums.  Called by the checks alone
+// (qpx_mlp_gemm_check, qpx_debug_mlp_gemm).  With a workspace, a product whose
+// tile grid leaves most CUs idle and whose K is long is cut along K across
+// workgroups and reduced in slice order.
 void gemm(hipStream_t st, const uint16_t *A, int64_t ars, int64_t acs, const uint16_t *B, int64_t brs, int64_t bcs,
           float *C, int64_t crs, int M, int N, int K, DBuf<float> *ws = nullptr) {
   // 16-byte runs need a 16-byte-aligned base and a multiple-of-8 stride
@@ -1064,9 +1069,9 @@ extern "C" int qpx_mlp_predict(qpx_mlp *m, int n, const int *desc, const float *
   });
 }
 
-// Prediction without any allocation: the descriptors are staged, and the
-// activations kept, in this device's file-scope scratch (kStaticRows rows at
-// most).  Every call on a GPU shares that scratch: calls that overlap on one
+// Prediction without any allocation: the descriptors and the predictions are
+// staged in this device's file-scope scratch (kStaticRows rows at most; the
+// activations live in LDS).  Every call on a GPU shares that scratch: calls that overlap on one
 // GPU (from several threads or networks) race.
 extern "C" int qpx_mlp_predict_static(qpx_mlp *m, int n, const int *desc, const float *fdesc, float *out) {
   return mguard(m, [&] {
@@ -1124,13 +1129,11 @@ extern "C" int qpx_mlp_param(qpx_mlp *m, int which, int grad, int set, float *da
   });
 }
 
-// Plain bf16 GEMM C = A B (row-major A n x k, B k x m, fp32 inputs rounded
-// to bf16), for the lane-layout and accuracy checks of the MFMA tiles.
-// Test entry: C = A B through the network's GEMM in every operand layout it
-// is called with.  ta = 0: A given (M x K) row-major; ta = 1: A given as its
+// Test entry: C = A B through the weight gradients' tile in every operand layout
+// it can stage.  ta = 0: A given (M x K) row-major; ta = 1: A given as its
 // transpose, (K x M) row-major.  tb = 0: B (K x N) row-major; tb = 1: (N x K).
-// split = 1 passes a workspace, so the K split runs where it would for a
-// weight gradient.
+// split = 1 passes a workspace, so K is cut across workgroups where the tile
+// grid is small.
 extern "C" int qpx_debug_mlp_gemm(qpx_mlp *m, int M, int N, int K, const float *A, const float *B, int ta, int tb,
                                   int split, float *C) {
   if (M < 1 || N < 1 || K < 1 || !A || !B || !C) return 1;
@@ -1154,6 +1157,8 @@ extern "C" int qpx_debug_mlp_gemm(qpx_mlp *m, int M, int N, int K, const float *
   });
 }
 
+// Plain bf16 GEMM C = A B (row-major A n x k, B k x m, fp32 inputs rounded
+// to bf16), for the lane-layout and accuracy checks of the MFMA tiles.
 extern "C" int qpx_mlp_gemm_check(qpx_mlp *m, int M, int N, int K, const float *A, const float *B, float *C) {
   return mguard(m, [&] {
     QPX_HIP(hipSetDevice(m->device));

@@ -33,9 +33,10 @@
 // 262,144 determinants, 96 orbitals, 10 + 10 electrons, FP64, 4 states: 7.6 ms
 // by determinant, here 2.3 (doubles 1.59, singles 0.21, collection 0.46);
 // 40,003, 50 orbitals, FP32, 2 states: 459 and 125 us.  The doubles read 7.5 GB
-// from HBM at 4.6 TB/s (an integral table of 0.85 GB in an order with little
-// reuse), the collection 3.2 GB at 7 TB/s: both at what the card gives, so half
-// the occupancy or twice the loads in flight changes nothing.  The table
+// from HBM, at 4.7 TB/s (an integral table of 0.85 GB in an order with little
+// reuse: half the occupancy or twice the loads in flight changes nothing; at 2.1M
+// determinants, with longer buckets, they reach 7.6 TB/s), the collection 3.2 GB
+// at 7 TB/s.  The table
 // packed by pair symmetry (0.34 GB) was slower, 1.82 ms: neighbouring lanes
 // no longer read neighbouring words.
 #include <algorithm>
