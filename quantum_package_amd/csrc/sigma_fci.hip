@@ -1013,18 +1013,16 @@ bool fci_pays(qpx_ctx *c, int nst, size_t ts) {
 }
 
 // False when the tables or the scratch do not fit the device's memory: the
-// caller then takes a path that needs none.  What the call began goes again;
-// what was there before it stays, for the calls and captured graphs that use it.
+// caller then takes a path that needs none.  What the call began and could not
+// finish goes again; what is complete stays, for the calls and captured graphs
+// that use it.
 bool sigma_fci(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, hipStream_t st) {
   ensure_conn(c);
   FciPlan &P = c->W.fci;
-  const bool had_plan = P.valid, had_tables = prec == QPX_FP64 ? P.t64.valid : P.t32.valid;
   auto drop = [&] {
-    if (!had_tables) {
-      if (prec == QPX_FP64) P.t64.release();
-      else P.t32.release();
-    }
-    if (!had_plan) P.release();
+    if (prec == QPX_FP64 && !P.t64.valid) P.t64.release();
+    if (prec != QPX_FP64 && !P.t32.valid) P.t32.release();
+    if (!P.valid) P.release();
   };
   char *ws = nullptr;
   try {

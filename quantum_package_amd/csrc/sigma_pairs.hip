@@ -1087,10 +1087,11 @@ namespace qpx {
 
 // False when the entries, their sums or the integral table do not fit: the
 // caller then walks the buckets determinant by determinant (sigma_sparse.hip).
-// What the call began goes again; what was there before it stays, for the calls
-// and captured graphs that use it.  Entries that do not fit are not tried again
-// for this wavefunction; a table or sums (of a precision, of a number of
-// states) are, which costs an allocation.
+// What the call began and could not finish goes again; what is complete stays,
+// for the calls and captured graphs that use it (the walk's set-up gives it up
+// if it needs the room).  Entries that do not fit are not tried again for this
+// wavefunction; a table or sums (of a precision, of a number of states) are,
+// which costs an allocation.
 bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s, hipStream_t st) {
   Wfn &W = c->W;
   Ham &H = c->H;
@@ -1101,21 +1102,23 @@ bool sigma_pairs(qpx_ctx *c, int prec, int nst, const void *u, void *v, void *s,
   if (H.M > kG4MaxOrb || nst > kMaxState || H.na > kMaxElec || H.nb > kMaxElec || H.na < 1 || H.nb < 1) return false;
   if (W.pr.failed) return false;
   const bool f64 = prec == QPX_FP64;
-  const bool had_entries = W.pr.valid, had_table = f64 ? H.Pt.p != nullptr : H.Ptf.p != nullptr;
+  const bool had_entries = W.pr.valid;
+  bool table = f64 ? H.Pt.p != nullptr : H.Ptf.p != nullptr, entries = had_entries;
   auto drop = [&] {
-    if (!had_entries) {
+    if (!entries) {
       W.pr.release();
       c->ws_pairs.release();
     }
-    if (had_table) return;
+    if (table) return;
     if (f64) H.Pt.release();
     else H.Ptf.release();
   };
   char *ws = nullptr;
-  bool ok = false, entries = had_entries, failed = false;   // failed: the entries do not fit
+  bool ok = false, failed = false;   // failed: the entries do not fit
   try {
     if (f64) build_table<double>(c, H.Pt);
     else build_table<float>(c, H.Ptf);
+    table = true;
     if (!entries) {
       failed = true;
       switch (W.nint) {
